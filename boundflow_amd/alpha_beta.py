@@ -42,6 +42,8 @@ from .crown import (
     forward_ibp_trace,
     NotAChain,
     parse_chain,
+    takes_parts,
+    weight_parts,
 )
 from .profiling import launch as _timed
 from .spec import InputSpec, IntervalState, normalize_input_spec
@@ -213,12 +215,16 @@ def _grad_pass(spec: InputSpec, chain: Chain, trace: ForwardTrace, saved: dict, 
             vec_ld = 0
         gt = torch.empty(M, n_out, device=dev)
         if layer.kind == "linear":
-            wsz = int(_lib.load().bf_gemm_rank1_workspace(M, n_out, n_in))
-            ws = torch.empty(wsz, device=dev) if wsz else None
+            rank1 = (_lib.ptr(G if vec is not None else None), _lib.ptr(vec), vec_ld)
             with _timed("grad_gemm", 2.0 * M * n_in * n_out, 4.0 * (M * n_in + M * n_out + n_in * n_out)):
-                _lib.call("bf_gemm_rank1", _lib.ptr(g), n_in, _lib.ptr(layer.weight.contiguous()), n_in, 1,
-                          _lib.ptr(gt), n_out, M, n_out, n_in, S, _lib.ptr(G if vec is not None else None),
-                          _lib.ptr(vec), vec_ld, _lib.ptr(ws), wsz, stream)
+                if takes_parts(M, n_out, n_in, S, g):
+                    _lib.call("bf_gemm_rank1_parts", _lib.ptr(g), n_in, _lib.ptr(weight_parts(layer.weight, True)),
+                              _lib.ptr(gt), n_out, M, n_out, n_in, S, *rank1, stream)
+                else:
+                    wsz = int(_lib.load().bf_gemm_rank1_workspace(M, n_out, n_in))
+                    ws = torch.empty(wsz, device=dev) if wsz else None
+                    _lib.call("bf_gemm_rank1", _lib.ptr(g), n_in, _lib.ptr(layer.weight.contiguous()), n_in, 1,
+                              _lib.ptr(gt), n_out, M, n_out, n_in, S, *rank1, _lib.ptr(ws), wsz, stream)
         else:
             Ci, Hi, Wi = layer.in_shape
             Co, Ho, Wo = layer.out_shape

@@ -48,7 +48,7 @@ from .spec import BoxPerturbation, InputSpec, IntervalState, LpBallPerturbation,
 # Derived operands kept across queries
 
 _DERIVED: "OrderedDict[tuple, tuple]" = OrderedDict()
-_DERIVED_MAX = 64
+_DERIVED_MAX = 192   # a layer keeps up to three: its transpose and its packed parts either way
 _SCOPE = threading.local()
 
 
@@ -59,7 +59,7 @@ def derived(tag: str, sources: Tuple[torch.Tensor, ...], make: Callable[[], torc
     queries skip the copy.  Operands that depend on a query's inputs are never kept here.
 
     * The entry keeps its sources alive, so their storage cannot be reused under the same
-      key; at most 64 entries are kept.  A change written through ``tensor.data`` does not
+      key; at most ``_DERIVED_MAX`` entries are kept.  A change written through ``tensor.data`` does not
       bump the version and is not seen: change parameters through the tensor itself.
     * A hit on another stream than the one that made the entry waits for the producer
       (an event recorded after ``make()``), so the consumer never reads it half-written.
@@ -67,29 +67,50 @@ def derived(tag: str, sources: Tuple[torch.Tensor, ...], make: Callable[[], torc
       which the captured query keeps: a replay never reads an entry the process-wide
       cache has since evicted, and ``refresh_scope`` remakes (in place, before a replay)
       every entry whose source changed in place since it was made."""
+    out = _kept(tag, sources)
+    if out is None:
+        out = make()
+        _keep(tag, sources, out, make)
+    return out
+
+
+def _kept(tag: str, sources: Tuple[torch.Tensor, ...]) -> Optional[torch.Tensor]:
     scope = getattr(_SCOPE, "memo", None)
     table = _DERIVED if scope is None else scope
     key = (tag,) + tuple(id(t) for t in sources)
     hit = table.get(key)
+    if hit is None or hit[1] != tuple(t._version for t in sources) or not all(a is b for a, b in zip(hit[0], sources)):
+        return None
+    if scope is None:
+        _DERIVED.move_to_end(key)
+        out, stream, event = hit[2]
+        if event is not None and torch.cuda.current_stream(out.device) != stream:
+            torch.cuda.current_stream(out.device).wait_event(event)
+        return out
+    return hit[2][0]
+
+
+def _keep(tag: str, sources: Tuple[torch.Tensor, ...], out: torch.Tensor, make: Callable[[], torch.Tensor],
+          made=None) -> None:
+    """Enter ``out``; ``made``: the (stream, event) of a launch that made several entries."""
+    scope = getattr(_SCOPE, "memo", None)
+    table = _DERIVED if scope is None else scope
+    stream, event = made or (_made_here(out) if scope is None else (None, None))
+    key = (tag,) + tuple(id(t) for t in sources)
     versions = tuple(t._version for t in sources)
-    if hit is not None and all(a is b for a, b in zip(hit[0], sources)) and hit[1] == versions:
-        if scope is None:
-            _DERIVED.move_to_end(key)
-            out, stream, event = hit[2]
-            if event is not None and torch.cuda.current_stream(out.device) != stream:
-                torch.cuda.current_stream(out.device).wait_event(event)
-            return out
-        return hit[2][0]
-    out = make()
-    stream = event = None
-    if scope is None and out.is_cuda:
-        stream = torch.cuda.current_stream(out.device)
-        event = torch.cuda.Event()
-        event.record(stream)
     table[key] = (tuple(sources), versions, (out, stream, event), make if scope is not None else None)
     if scope is None and len(_DERIVED) > _DERIVED_MAX:
         _DERIVED.popitem(last=False)
-    return out
+
+
+def _made_here(out: torch.Tensor):
+    """The current stream and an event on it, after which ``out`` is whole."""
+    if not out.is_cuda:
+        return None, None
+    stream = torch.cuda.current_stream(out.device)
+    event = torch.cuda.Event()
+    event.record(stream)
+    return stream, event
 
 
 @contextlib.contextmanager
@@ -139,6 +160,70 @@ def call_memo(save: Optional[dict], key: str, make: Callable[[], torch.Tensor]) 
 def transposed(W: torch.Tensor) -> torch.Tensor:
     """W^T, contiguous (the contraction's faster operand layout), kept across queries."""
     return derived("wt", (W,), lambda: W.t().contiguous())
+
+
+def weight_parts(W: torch.Tensor, trans_b: bool, also=()) -> torch.Tensor:
+    """A weight [N, P] packed for the contractions on the bf16 matrix cores (bf_gemm_pack_parts),
+    kept across queries: for rows of N coefficients (the backward's A W) or, with ``trans_b``,
+    for rows of P (the reverse pass's g W^T).  ``also``: the (weight, trans_b) pairs whose
+    packing the caller will ask for next; what of them is missing is packed in the same launch."""
+    out = _kept(_PARTS[trans_b], (W,))
+    if out is not None:
+        return out
+    todo = [(W, trans_b)] + [(w, t) for w, t in also if not (w is W and t == trans_b)
+                             and _kept(_PARTS[t], (w,)) is None]
+    outs = _pack(todo)
+    scope = getattr(_SCOPE, "memo", None)
+    made = _made_here(outs[0]) if scope is None else None
+    for (w, t), o in zip(todo, outs):
+        _keep(_PARTS[t], (w,), o, lambda w=w, t=t: _pack([(w, t)])[0], made)
+    return outs[0]
+
+
+_PARTS = {False: "parts", True: "parts_t"}
+
+
+def _pack(todo) -> List[torch.Tensor]:
+    src = [w.contiguous() for w, _t in todo]
+    sizes = [(int(w.shape[0]), int(w.shape[1])) for w in src]
+    N = [n if t else p for (n, p), (_w, t) in zip(sizes, todo)]
+    K = [p if t else n for (n, p), (_w, t) in zip(sizes, todo)]
+    outs = [torch.empty(int(_lib.load().bf_gemm_parts_floats(n, k)), device=w.device, dtype=torch.float32)
+            for n, k, w in zip(N, K, src)]
+    _lib.call("bf_gemm_pack_parts", len(todo), _lib.ptr_array(src), _lib.i64_array([p for _n, p in sizes]),
+              _lib.i32_array([int(t) for _w, t in todo]), _lib.i64_array(N), _lib.i64_array(K), _lib.ptr_array(outs),
+              _lib.stream_handle())
+    return outs
+
+
+def chain_parts(layers: List[AffineLayer], layer: AffineLayer, M: int, S: int, nz: int, save: Optional[dict],
+                trans_b: bool = False) -> torch.Tensor:
+    """``weight_parts`` of a chain's linear layer; when it is not kept yet, with those of the
+    other layers the query will read: the backward's, and with a gradient to follow the reverse
+    pass's."""
+    def also():
+        take = _lib.load().bf_gemm_parts_config
+        for other in layers:
+            if other.kind != "linear":
+                continue
+            n, p = _numel(other.out_shape), _numel(other.in_shape)
+            if take(M, p, n, S, nz):
+                yield other.weight, False
+            if save is not None and save.get("grad_rows") is not None and take(M, n, p, S, 1):
+                yield other.weight, True
+    return weight_parts(layer.weight, trans_b, also())
+
+
+def takes_parts(M: int, N: int, K: int, S: int, *coeffs: Optional[torch.Tensor], nz: int = 0) -> bool:
+    """Whether the contraction of M coefficient rows (S per domain) of K values into N runs on
+    packed weight parts: the library's rule on the shape, and 16-byte aligned rows (``nz`` in
+    place of ``coeffs``: that many bounds, whose rows are still to be made)."""
+    nz = nz or sum(t is not None for t in coeffs)
+    # (most small queries end here, without a call into the library)
+    if K < 64 or K % 4 or -(-M // 128) * -(-N // 128) * nz < 128:
+        return False
+    return (all(t is None or t.data_ptr() % 16 == 0 for t in coeffs)
+            and _lib.load().bf_gemm_parts_config(M, N, K, S, nz) != 0)
 
 
 # ---------------------------------------------------------------------------
@@ -565,8 +650,6 @@ def crown_backward(
                 return done
             continue
         W = layer.weight.contiguous()
-        # the contraction reads W^T [P, N] row-major: 128-bit operand loads along N
-        Wt = transposed(W)
         bias = None if layer.bias is None or pre_relaxed else layer.bias.contiguous()
         P = _numel(layer.in_shape)
         if k > 0 and linear_spec_C is None and k == len(layers) - 1:
@@ -581,7 +664,9 @@ def crown_backward(
         shared_first = (stride == 0 and S >= EPILOGUE_MIN_ROWS and M >= EPILOGUE_MIN_M
                         and (k == 0 or layers[k - 1].kind == "linear"))
         small_grid = M < EPILOGUE_MIN_M and N >= RELAX_PASS_MIN_K
-        if relaxes and (shared_first or small_grid or relax_pass_next):
+        # (few rows per domain: no epilogue relaxed them, and the packed weight takes no prologue)
+        packed = relaxes and takes_parts(M, P, N, S, nz=int(A_u is not None) + int(A_l is not None))
+        if relaxes and (shared_first or small_grid or relax_pass_next or packed):
             # A coefficient shared by every domain (the first region of a C = I query):
             # its relaxation differs per domain, so one bandwidth-bound pass writes it
             # per domain (with the bias terms and, at the input layer, the center sums)
@@ -628,12 +713,14 @@ def crown_backward(
                 save["h"] = h_out
                 save["cvec"] = trace.input_center_proj.get(layer.out_name)
             nz = int(A_u is not None) + int(A_l is not None)
+            in_parts = takes_parts(M, P, N, S, A_u, A_l)
             # bytes: the coefficient rows and the weight read, the row partial norms written, the
             # gradient seed [M, P] written when asked
             with _timed("crown_linear_concretize", 2.0 * nz * M * N * P,
                         4.0 * nz * (M * N + N * P + M * -(-P // 128)) + (4.0 * M * P if h_out is not None else 0.0)):
-                _lib.call("bf_crown_linear_concretize", _lib.ptr(A_u), _lib.ptr(A_l), stride, B, S, N, _lib.ptr(Wt),
-                          P, _lib.ptr(rad), eps, input_norm_p(pert), _lib.ptr(c_u), _lib.ptr(c_l), _lib.ptr(b_u),
+                _lib.call("bf_crown_linear_concretize_parts" if in_parts else "bf_crown_linear_concretize",
+                          _lib.ptr(A_u), _lib.ptr(A_l), stride, B, S, N,
+                          _lib.ptr(chain_parts(layers, layer, M, S, nz, save) if in_parts else transposed(W)), P, _lib.ptr(rad), eps, input_norm_p(pert), _lib.ptr(c_u), _lib.ptr(c_l), _lib.ptr(b_u),
                           _lib.ptr(b_l),
                           _lib.ptr(h_scale), _lib.ptr(h_out), _lib.ptr(ws), _lib.ptr(lb), _lib.ptr(ub), stream)
             if save is not None:
@@ -667,7 +754,7 @@ def crown_backward(
             with _timed("crown_relu_linear_concretize", 2.0 * nz * M * N * P,
                         4.0 * nz * (M * N + N * P) + 16.0 * B * N + (4.0 * M * P if h_out is not None else 0.0)):
                 _lib.call("bf_crown_relu_linear_concretize", _lib.ptr(A_u), _lib.ptr(A_l), stride, B, S, N,
-                          _lib.ptr(relax), _lib.ptr(add), add_ld, _lib.ptr(Wt), P, 1, _lib.ptr(bias), _lib.ptr(cvec),
+                          _lib.ptr(relax), _lib.ptr(add), add_ld, _lib.ptr(transposed(W)), P, 1, _lib.ptr(bias), _lib.ptr(cvec),
                           _lib.ptr(rad), eps, input_norm_p(pert), _lib.ptr(b_u),
                           _lib.ptr(b_l), _lib.ptr(h_scale), _lib.ptr(h_out), _lib.ptr(ws), _lib.ptr(lb),
                           _lib.ptr(ub), stream)
@@ -679,6 +766,7 @@ def crown_backward(
         nb_u = torch.empty(M, device=dev, dtype=torch.float32) if A_u is not None else None
         nb_l = torch.empty(M, device=dev, dtype=torch.float32) if A_l is not None else None
         nz = int(A_u is not None) + int(A_l is not None)
+        plain = relax is None and add is None and bias is None   # nothing to relax, no bias rows to make
         a_rows = M if stride != 0 else S
         flops, nbytes = 2.0 * nz * M * N * P, 4.0 * nz * (a_rows * N + N * P + M * P)
         # The head region (the spec C through the last layer, nothing to relax) depends on C
@@ -714,11 +802,16 @@ def crown_backward(
                        + 4.0 * nz * M * -(-P // 128) * (2 if cvec is not None else 1))
             with _timed("crown_relu_linear_relu_fwd", flops,
                         nbytes + e_bytes + (4.0 * M * P if pre_l is not None else 0.0)):
-                _lib.call("bf_crown_relu_linear_relu_fwd", _lib.ptr(A_u), _lib.ptr(A_l), stride, B, S, N,
-                          _lib.ptr(relax), _lib.ptr(add), add_ld, _lib.ptr(Wt), P, _lib.ptr(bias), _lib.ptr(b_u),
-                          _lib.ptr(b_l), _lib.ptr(n_table), _lib.ptr(n_add), n_add_ld, _lib.ptr(n_bias),
-                          _lib.ptr(cvec), P, _lib.ptr(ws), _lib.ptr(nA_u), _lib.ptr(nA_l), None, _lib.ptr(pre_l),
-                          _lib.ptr(nb_u), _lib.ptr(nb_l), _lib.ptr(nc_u), _lib.ptr(nc_l), stream)
+                after = (_lib.ptr(b_u), _lib.ptr(b_l), _lib.ptr(n_table), _lib.ptr(n_add), n_add_ld, _lib.ptr(n_bias),
+                         _lib.ptr(cvec), P, _lib.ptr(ws), _lib.ptr(nA_u), _lib.ptr(nA_l), None, _lib.ptr(pre_l),
+                         _lib.ptr(nb_u), _lib.ptr(nb_l), _lib.ptr(nc_u), _lib.ptr(nc_l), stream)
+                if plain and takes_parts(M, P, N, S, A_u, A_l):
+                    _lib.call("bf_crown_linear_relu_fwd_parts", _lib.ptr(A_u), _lib.ptr(A_l), stride, B, S, N,
+                              _lib.ptr(chain_parts(layers, layer, M, S, nz, save)), P, *after)
+                else:
+                    _lib.call("bf_crown_relu_linear_relu_fwd", _lib.ptr(A_u), _lib.ptr(A_l), stride, B, S, N,
+                              _lib.ptr(relax), _lib.ptr(add), add_ld, _lib.ptr(transposed(W)), P, _lib.ptr(bias),
+                              *after)
             if pre_l is not None:
                 save.setdefault("A_in", {})[k - 1] = (pre_l, S * P)
                 save.setdefault("b_in", {})[k - 1] = nb_l
@@ -740,12 +833,16 @@ def crown_backward(
             if hit is not None:
                 nA_u, nA_l, nb_u, nb_l = hit
             else:
+                rows = (_lib.ptr(bias), None if keep_b else _lib.ptr(b_u), None if keep_b else _lib.ptr(b_l),
+                        _lib.ptr(nA_u), _lib.ptr(nA_l), None if keep_b else _lib.ptr(nb_u),
+                        None if keep_b else _lib.ptr(nb_l), stream)
                 with _timed("crown_relu_linear_fwd", flops, nbytes):
-                    _lib.call("bf_crown_relu_linear_fwd", _lib.ptr(A_u), _lib.ptr(A_l), stride, B, S, N,
-                              _lib.ptr(relax), _lib.ptr(add), add_ld, _lib.ptr(Wt), P, 1, _lib.ptr(bias),
-                              None if keep_b else _lib.ptr(b_u), None if keep_b else _lib.ptr(b_l), _lib.ptr(nA_u),
-                              _lib.ptr(nA_l), None if keep_b else _lib.ptr(nb_u), None if keep_b else _lib.ptr(nb_l),
-                              stream)
+                    if plain and takes_parts(M, P, N, S, A_u, A_l):
+                        _lib.call("bf_crown_linear_parts", _lib.ptr(A_u), _lib.ptr(A_l), stride, B, S, N,
+                                  _lib.ptr(chain_parts(layers, layer, M, S, nz, save)), P, *rows)
+                    else:
+                        _lib.call("bf_crown_relu_linear_fwd", _lib.ptr(A_u), _lib.ptr(A_l), stride, B, S, N,
+                                  _lib.ptr(relax), _lib.ptr(add), add_ld, _lib.ptr(transposed(W)), P, 1, *rows)
                 if head_key is not None:
                     save["memo"][head_key] = (nA_u, nA_l, nb_u, nb_l)
             pre_relaxed = False

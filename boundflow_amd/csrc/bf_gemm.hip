@@ -85,7 +85,7 @@ __global__ void relax_table_multi_kernel(TableSegs t, int64_t D) {
                    ((int64_t)blockIdx.x - t.bstart[s]) * blockDim.x + threadIdx.x);
 }
 
-// BOUNDFLOW_GEMM_TILE=G, =H, =Q or =S forces one configuration (for measurement);
+// BOUNDFLOW_GEMM_TILE=G, =H, =Q or =S forces one fp32 configuration (for measurement);
 // read once when the library is loaded, constant afterwards.
 static int forced_tile_from_env() {
   const char* v = std::getenv("BOUNDFLOW_GEMM_TILE");
@@ -130,11 +130,34 @@ int gemm_tile_choice(int64_t M, int64_t N, int nz, int64_t ks, int pro, bool dl)
 }
 
 int gemm_norm_cols(int64_t M, int64_t N, int pro);
+int launch_parts(const GemmArgs& a, int epi, int nz, hipStream_t stream);
+
+// Whether the three-part kernels take a plain contraction of this shape (packed weight, domains of
+// S rows): K whole float4s and at least four stages deep, rows within the 32-bit byte offsets of a
+// tile, and at least 128 tiles of 128 x 128.  A tile's stage takes about 0.64 us with one wave per
+// SIMD, so fewer tiles are bound by that latency and the fp32 tiles, which deal a short grid as 64 x
+// 64 over four times as many CUs, are level or faster (us on one MI355X, fp32 / parts): 72 tiles at
+// K = 512 26.2 / 27.3, at K = 256 16.6 / 16.8; 144 tiles 35.9 / 28.2 and 21.9 / 17.5, at K = 64
+// 10.6 / 9.3; 288 tiles 57.9 / 32.9; 1008 tiles 184.0 / 85.6.
+int gemm_parts_choice(int64_t M, int64_t N, int64_t K, int64_t S, int nz) {
+  if (kForcedTile || M <= 0 || N <= 0 || K < 64 || K % 4 != 0 || S <= 0 || N >= (1LL << 31) || K >= (1LL << 31))
+    return 0;
+  if (S >= (1LL << 29) / 4 || (512 + 4 * S) >= (1LL << 29) / K) return 0;
+  return ceil_div(M, (int64_t)128) * ceil_div(N, (int64_t)128) * nz >= 128 ? 1 : 0;
+}
 
 int gemm_dispatch(const GemmArgs& a, int pro, int epi, int nz, hipStream_t stream) {
   if ((pro != PRO_PLAIN && pro != PRO_RELAX) || (epi != EPI_STORE && epi != EPI_ABSSUM && epi != EPI_RELAX)) {
     set_error("gemm_dispatch: bad mode pro=%d epi=%d", pro, epi);
     return BF_EINVAL;
+  }
+  if (a.b_parts) {
+    bool rows = a.lda == a.K && a.lda_d >= 0 && a.lda_d % 4 == 0 && a.lda_d <= 2 * a.S * a.K;
+    for (int z = 0; z < nz; ++z) rows = rows && ((uintptr_t)a.A[z] & 15) == 0;
+    BF_REQUIRE(gemm_parts_choice(a.M, a.N, a.K, a.S, nz) && rows && pro == PRO_PLAIN && a.ksplit <= 1,
+               "gemm: a packed weight does not serve M=%lld N=%lld K=%lld with these rows (bf_gemm_parts_config)",
+               (long long)a.M, (long long)a.N, (long long)a.K);
+    return launch_parts(a, epi, nz, stream);
   }
   const int64_t ks = (pro == PRO_PLAIN && epi == EPI_STORE && a.ksplit > 1) ? a.ksplit : 1;
   const bool dl = gemm_dl_operands(a, nz);

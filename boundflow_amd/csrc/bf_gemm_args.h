@@ -18,6 +18,7 @@ struct GemmArgs {
   const float* B;   // [K, N] row-major (ldb) or, with trans_b, [N, K] row-major (ldb)
   int64_t ldb;
   int trans_b;
+  int b_parts;      // B is a packed weight (pack_parts): the three-part kernels take it, ldb and trans_b unread
   int abs_b;        // bit z set: product z uses |B| (interval radius products)
   // Interval operand of the IBP products (plain prologue, register-staged loop): A[0] = A[1]
   // hold the lower bounds and ivl_hi the upper ones (same layout); product z = 0 reads the

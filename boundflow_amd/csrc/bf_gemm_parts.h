@@ -1,0 +1,273 @@
+// fp32 contraction on the bf16 matrix cores (gfx950), for grids large enough to be
+// bound by the fp32 MFMA rate.
+//
+//   C[M, N] = A[M, K] x B[N, K]^T
+//
+// Every operand value is split into three bf16 parts, each the nearest bf16 of what the
+// parts before it leave: x = x0 + x1 + x2 exactly (8 + 8 + 8 significant bits against 24;
+// the exponent range of bf16 is fp32's).  A product is the sum of the six part products
+// above 2^-24 of it,
+//   x0 y0 + (x0 y1 + x1 y0) + (x1 y1 + x0 y2 + x2 y0),
+// each exact, summed in fp32 by v_mfma_f32_32x32x16_bf16: six of these take 192 cycles for
+// the 16 k steps that eight v_mfma_f32_32x32x2f32 take 512 for.  What is left out is below
+// 2^-24 of a product, the rounding of one fp32 addition, and the 6 roundings of a sum per
+// 16 k stand against 8.
+//
+// B (a layer's weight) comes packed: its parts made once per weight (pack_parts_kernel), in
+// the MFMA operand order, so that a stage's parts go straight from global memory to LDS.  A
+// wave owns WTM rows and all BN columns of the tile.  Its A rows pass through LDS as they
+// are (global_load_lds_dwordx4, private to the wave, so no barrier guards them) and it splits
+// them once, in registers.  Stages are 16 k deep, three of A and two of B; one barrier each.
+//
+// A tile with a sum that is not finite (an operand that is not, or a coefficient above the
+// largest bf16, whose parts are then not defined) is computed again by v_mfma_f32_32x32x2f32
+// from the fp32 values, so such operands give what they give on the fp32 tiles.
+#pragma once
+
+#include "bf_gemm_parts_epilogue.h"
+
+namespace bf {
+
+typedef float floatx2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef uint32_t uint32x4 __attribute__((ext_vector_type(4)));
+
+// Packed parts of B: per 32-column block and 16-k stage 3 KB, part by part, lane l's eight
+// values (column l % 32, k 8 (l / 32) .. + 7) at 16 l; columns and k past the end are zero.
+constexpr int PARTS_BLOCK = 3 * 64 * 4;   // floats of one block and stage
+
+template <int FM_, int NWM_, int OCC_>
+struct TileParts {
+  static constexpr int FM = FM_, FN = 4, NWM = NWM_, NWN = 1, OCC = OCC_;
+  static constexpr int WTM = 32 * FM, WTN = 32 * FN;   // wave tile
+  static constexpr int BM = WTM * NWM, BN = WTN, BK = 16, NT = 64 * NWM;
+  static constexpr int A_STAGE = BM * BK;              // floats of a stage of A rows
+  static constexpr int B_STAGE = FN * PARTS_BLOCK;     // floats of a stage of B parts
+  static constexpr int B_COPIES = 3 * FN / NWM;        // 1 KB copies of a B stage per wave
+  static_assert(B_COPIES * NWM == 3 * FN, "whole copies per wave");
+};
+
+// lds_copy16 from a scalar base and a byte offset per lane.
+__device__ __forceinline__ void lds_copy16_at(const float* base, uint32_t byte_off, float* lds_dst) {
+  const uint32_t off = (uint32_t)(uintptr_t)((lds_float*)lds_dst);
+  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(byte_off), "s"(base), "s"(off) : "memory");
+}
+
+// (x, y) -> the packed bf16 pair nearest to it, and what the pair leaves of both.
+__device__ __forceinline__ uint32_t take_part(float& x, float& y) {
+  const floatx2 xy = {x, y};
+  const uint32_t pk = __builtin_bit_cast(uint32_t, __builtin_convertvector(xy, bf16x2));   // v_cvt_pk_bf16_f32
+  x -= __uint_as_float(pk << 16);
+  y -= __uint_as_float(pk & 0xffff0000u);
+  return pk;
+}
+
+// Eight values -> their three parts as MFMA operands.
+__device__ __forceinline__ void split_parts(float (&v)[8], uint32x4 (&part)[3]) {
+#pragma unroll
+  for (int q = 0; q < 3; ++q)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) part[q][e] = take_part(v[2 * e], v[2 * e + 1]);
+}
+
+template <int EPI, class T>
+__global__ void __launch_bounds__(T::NT, T::OCC * T::NWM / 4) gemm_parts_kernel(GemmArgs p) {
+  constexpr int FM = T::FM, FN = T::FN, GBM = T::BM, GBN = T::BN, GBK = T::BK;
+  // three stages of A rows, two of B parts; the relaxation epilogue stages its operands over all of it
+  constexpr int SMEM = 3 * T::A_STAGE + 2 * T::B_STAGE;
+  __shared__ __attribute__((aligned(16))) float smem_ab[SMEM];
+  __shared__ float red[T::NWN][GBM];
+  float* const bs = smem_ab + 3 * T::A_STAGE;
+
+  const int t = threadIdx.x;
+  const int lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int lrow = lane & 31;
+  const int h = lane >> 5;   // lane half -> k 8 h .. 8 h + 7 of a stage, in A and B alike
+  const int z = (int)blockIdx.y;
+  const bool lower = p.z_lower_first ? (z == 0) : (z == 1);
+  const int64_t M = p.M, N = p.N, K = p.K;
+  const bool fits32 = M < (1LL << 31);
+  // XCD-aware tile order, as in gemm_kernel
+  const int64_t ntn = ceil_div(N, GBN);
+  const int64_t ntiles = ceil_div(M, GBM) * ntn;
+  const int64_t per_xcd = ceil_div(ntiles, 8);
+  const int64_t tile = (int64_t)(blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+  if (tile >= ntiles) return;
+  const int64_t tile_n = tile % ntn;
+  const int64_t m0 = (tile / ntn) * GBM;
+  const int64_t n0 = tile_n * GBN;
+  const int64_t cols = N - n0;
+  const int fn_act = cols >= GBN ? FN : (int)ceil_div(cols, 32);   // 32-column blocks inside N
+  const int nk = (int)ceil_div(K, (int64_t)GBK);
+
+  // copy slots of this wave's A rows: chunk j holds its rows 16 j .. 16 j + 15, float4 kq of row r
+  // at position 4 r + (kq ^ (r / 2 % 4)) of the chunk, as in gemm_kernel's direct-to-LDS loop.
+  // Byte offsets from the tile's first domain (below 2^32, checked at launch): a stage advances
+  // the scalar base alone.
+  constexpr int CHUNKS = T::WTM / 16;
+  const int64_t d0 = div_rows(m0, p.S, fits32);
+  const float* __restrict__ a_base = p.A[z] + d0 * p.lda_d;
+  uint32_t a_off[CHUNKS];
+  const int a_kq = (lane & 3) ^ ((lane >> 3) & 3);
+#pragma unroll
+  for (int j = 0; j < CHUNKS; ++j) {
+    const int64_t mr = m0 + wave * T::WTM + 16 * j + (lane >> 2);
+    const int64_t m = mr < M ? mr : M - 1;
+    const int64_t d = div_rows(m, p.S, fits32);
+    a_off[j] = (uint32_t)(4 * ((d - d0) * p.lda_d + (m - d * p.S) * p.lda + 4 * a_kq));
+  }
+  float* const a_wave = smem_ab + wave * T::WTM * GBK;
+  auto copy_a = [&](int slot, int kt) {
+    float* dst = a_wave + slot * T::A_STAGE;
+    const float* src = a_base + (int64_t)kt * GBK;
+    if (kt * GBK + GBK <= K) {
+#pragma unroll
+      for (int j = 0; j < CHUNKS; ++j) lds_copy16_at(src, a_off[j], dst + 256 * j);
+    } else {
+      // quads past K read the row start: they meet the zeros that B's parts hold there
+      const int back = kt * GBK + 4 * a_kq < K ? 0 : kt * GBK + 4 * a_kq;
+#pragma unroll
+      for (int j = 0; j < CHUNKS; ++j) lds_copy16(src + (int64_t)(a_off[j] / 4) - back, dst + 256 * j);
+    }
+  };
+  // this wave's copies of a B stage: block * 3 + part = B_COPIES wave .. ; blocks past N copy the
+  // last one inside
+  const float* __restrict__ b_base = p.B + (n0 / 32) * nk * PARTS_BLOCK;
+  int64_t b_src[T::B_COPIES];
+#pragma unroll
+  for (int c = 0; c < T::B_COPIES; ++c) {
+    const int u = T::B_COPIES * wave + c, blk = u / 3 < fn_act ? u / 3 : fn_act - 1;
+    b_src[c] = (int64_t)blk * nk * PARTS_BLOCK + (u % 3) * 256;
+  }
+  const uint32_t b_lane = 16 * lane;
+  auto copy_b = [&](int slot, int kt) {
+    const float* src = b_base + (int64_t)kt * PARTS_BLOCK;
+    float* dst = bs + slot * T::B_STAGE + T::B_COPIES * wave * 256;
+#pragma unroll
+    for (int c = 0; c < T::B_COPIES; ++c) lds_copy16_at(src + b_src[c], b_lane, dst + 256 * c);
+  };
+
+  floatx16 acc[FM][FN];
+  auto clear = [&]() {
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < FN; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+  };
+  clear();
+
+  // operand positions of this lane in its wave's A stage: row 32 i + lrow, k quads 2 h and 2 h + 1
+  const int swz = (lrow >> 1) & 3;
+  int a_pos[2];
+#pragma unroll
+  for (int jq = 0; jq < 2; ++jq) a_pos[jq] = 4 * (4 * lrow + ((2 * h + jq) ^ swz));
+
+  auto main_loop = [&](auto full_c) {
+    constexpr bool FULL = decltype(full_c)::value;
+    copy_a(0, 0);
+    copy_b(0, 0);
+    if (nk > 1) copy_a(1, 1);
+    int sa = 0;   // A slot of stage kt
+    for (int kt = 0; kt < nk; ++kt) {
+      const int sb = kt & 1;
+      // this stage's copies have landed; the next stage's A rows may still be in flight
+      if (kt + 1 < nk) wait_vmem<CHUNKS>(); else wait_vmem<0>();
+      lds_barrier();   // every wave's B parts are there; no wave reads the slots refilled next
+      if (kt + 1 < nk) copy_b(sb ^ 1, kt + 1);
+      if (kt + 2 < nk) copy_a(sa == 0 ? 2 : sa - 1, kt + 2);
+      const float* __restrict__ bst = bs + sb * T::B_STAGE + 4 * lane;
+      uint32x4 ap[FM][3], bp[2][3];
+      auto read_b = [&](int j) {
+#pragma unroll
+        for (int s = 0; s < 3; ++s)
+          bp[j & 1][s] = *reinterpret_cast<const uint32x4*>(bst + j * PARTS_BLOCK + 256 * s);
+      };
+#pragma unroll
+      for (int i = 0; i < FM; ++i) {
+        const float* src = a_wave + sa * T::A_STAGE + 512 * i;
+        const float4 lo = *reinterpret_cast<const float4*>(src + a_pos[0]);
+        const float4 hi = *reinterpret_cast<const float4*>(src + a_pos[1]);
+        if (i == FM - 1) read_b(0);
+        float v[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+        split_parts(v, ap[i]);
+      }
+      // the B parts of a column block are read one block ahead of their MFMAs (the fences keep
+      // the compiler from moving the reads to where they are used)
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int j = 0; j < FN; ++j) {
+        if (!FULL && j >= fn_act) continue;
+        if (j + 1 < FN && (FULL || j + 1 < fn_act)) read_b(j + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        // the smallest products first
+        constexpr int PA[6] = {2, 0, 1, 1, 0, 0}, PB[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+        for (int q = 0; q < 6; ++q)
+#pragma unroll
+          for (int i = 0; i < FM; ++i)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, ap[i][PA[q]]),
+                                                                __builtin_bit_cast(bf16x8, bp[j & 1][PB[q]]),
+                                                                acc[i][j], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      sa = sa == 2 ? 0 : sa + 1;
+    }
+  };
+  if (fn_act == FN) main_loop(std::true_type{});
+  else main_loop(std::false_type{});
+
+  // a sum that is not finite leaves a NaN here
+  float probe = 0.f;
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) probe = __builtin_fmaf(acc[i][j][r], 0.f, probe);
+  if (__any(probe != 0.f)) {
+    clear();
+    const float* arow[FM];
+#pragma unroll
+    for (int i = 0; i < FM; ++i) {
+      const int64_t mr = m0 + wave * T::WTM + 32 * i + lrow;
+      const int64_t m = mr < M ? mr : M - 1;
+      const int64_t d = div_rows(m, p.S, fits32);
+      arow[i] = p.A[z] + d * p.lda_d + (m - d * p.S) * p.lda;
+    }
+    for (int kt = 0; kt < nk; ++kt)
+      for (int e = 0; e < 8; ++e) {
+        const int64_t k = (int64_t)kt * GBK + 8 * h + e;
+        float av[FM], bv[FN];
+#pragma unroll
+        for (int i = 0; i < FM; ++i) av[i] = k < K ? arow[i][k] : 0.f;
+#pragma unroll
+        for (int j = 0; j < FN; ++j) {
+          // the fp32 value again: the sum of its parts, which is exact
+          const int blk = j < fn_act ? j : fn_act - 1;
+          const uint16_t* src = reinterpret_cast<const uint16_t*>(b_base + ((int64_t)blk * nk + kt) * PARTS_BLOCK) +
+                                8 * lane + e;
+          const float x0 = __uint_as_float((uint32_t)src[0] << 16), x1 = __uint_as_float((uint32_t)src[512] << 16),
+                      x2 = __uint_as_float((uint32_t)src[1024] << 16);
+          bv[j] = (x0 + x1) + x2;
+        }
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+          for (int j = 0; j < FN; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[i], bv[j], acc[i][j], 0, 0, 0);
+      }
+  }
+  __syncthreads();   // every wave is done with the stages before an epilogue reuses them
+  parts_epilogue<EPI, T, SMEM>(p, acc, smem_ab, red, m0, n0, tile_n, wave, 0, lane, z, lower);
+}
+
+// 128 x 128, 4 waves of 32 x 128, 3 workgroups per CU
+using TileP = TileParts<1, 4, 3>;
+
+int launch_parts(const GemmArgs& a, int epi, int nz, hipStream_t stream);
+
+}  // namespace bf

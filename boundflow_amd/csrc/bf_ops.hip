@@ -34,6 +34,10 @@ int concretize_finalize(const float* pu, const float* pl, int nparts, int64_t M,
                         hipStream_t stream);
 int gemm_partial_count(int64_t N);
 int gemm_norm_partial_count(int64_t M, int64_t N, int pro);
+int gemm_parts_choice(int64_t M, int64_t N, int64_t K, int64_t S, int nz);
+int64_t parts_floats(int64_t N, int64_t K);
+int pack_parts(int count, const float* const* B, const int64_t* ldb, const int* trans_b, const int64_t* N,
+               const int64_t* K, float* const* out, hipStream_t stream);
 int rows_finalize(const float* b_src, const float* pb, const float* pc, int nparts, int64_t M, float* b_out,
                   float* c_out, hipStream_t stream);
 int gemm_ksplit(int64_t M, int64_t N, int64_t K, int64_t* kchunk);
@@ -1363,6 +1367,49 @@ int bf_gemm_rank1(const float* A, int64_t lda, const float* B, int64_t ldb, int 
   return splitk_reduce(workspace, ks, M, N, C, ldc, r_row, v_col, v_ld, S, stream);
 }
 
+int bf_gemm_parts_config(int64_t M, int64_t N, int64_t K, int64_t S, int nz) {
+  return nz < 1 || nz > 2 ? 0 : gemm_parts_choice(M, N, K, S, nz);
+}
+
+int64_t bf_gemm_parts_floats(int64_t N, int64_t K) { return N <= 0 || K <= 0 ? 0 : parts_floats(N, K); }
+
+int bf_gemm_pack_parts(int count, const float* const* B, const int64_t* ldb, const int* trans_b, const int64_t* N,
+                       const int64_t* K, float* const* parts, hipStream_t stream) {
+  BF_REQUIRE(count >= 0, "bf_gemm_pack_parts: bad count");
+  if (count == 0) return BF_OK;
+  BF_REQUIRE(B && ldb && trans_b && N && K && parts, "bf_gemm_pack_parts: null array");
+  for (int j = 0; j < count; ++j) {
+    BF_REQUIRE(N[j] > 0 && K[j] > 0 && B[j] && parts[j], "bf_gemm_pack_parts: size or null pointer of weight %d", j);
+    BF_REQUIRE(((uintptr_t)parts[j] & 15) == 0, "bf_gemm_pack_parts: parts %d must be 16-byte aligned", j);
+  }
+  return pack_parts(count, B, ldb, trans_b, N, K, parts, stream);
+}
+
+int bf_gemm_rank1_parts(const float* A, int64_t lda, const float* parts, float* C, int64_t ldc, int64_t M, int64_t N,
+                        int64_t K, int64_t S, const float* r_row, const float* v_col, int64_t v_ld,
+                        hipStream_t stream) {
+  BF_REQUIRE(M >= 0 && N >= 0 && K >= 0 && S > 0, "bf_gemm_rank1_parts: bad sizes");
+  if (M == 0 || N == 0) return BF_OK;
+  BF_REQUIRE(A && parts && C && ((r_row == nullptr) == (v_col == nullptr)), "bf_gemm_rank1_parts: null pointer");
+  GemmArgs a;
+  memset(&a, 0, sizeof(a));
+  a.A[0] = A;
+  a.C[0] = C;
+  a.lda = lda;
+  a.lda_d = lda * S;
+  a.ldc = ldc;
+  a.B = parts;
+  a.b_parts = 1;
+  a.M = M;
+  a.N = N;
+  a.K = K;
+  a.S = S;
+  a.r1_row = r_row;
+  a.r1_col = v_col;
+  a.r1_ld = v_ld;
+  return gemm_dispatch(a, PRO_PLAIN, EPI_STORE, 1, stream);
+}
+
 int bf_concretize_finalize(const float* partial_u, const float* partial_l, int nparts, int64_t M,
                            const float* cen_u, const float* cen_l, const float* b_u, const float* b_l, float eps,
                            int norm_p, float* lb, float* ub, hipStream_t stream) {
@@ -1570,7 +1617,7 @@ int bf_crown_relu_linear_concretize_noalloc(const float* A_u, const float* A_l, 
                                          cvec, rad, eps, norm_p, b_u_in, b_l_in, h_scale, h_out, ws, lb, ub, stream);
 }
 
-int bf_crown_relu_linear_relu_fwd(const float* A_u, const float* A_l, int64_t a_dstride, int64_t D, int64_t S,
+static int relu_linear_relu_fwd(int b_parts, const float* A_u, const float* A_l, int64_t a_dstride, int64_t D, int64_t S,
                                   int64_t N, const float* relax, const float* add_l, int64_t add_ld,
                                   const float* W_t, int64_t P, const float* bias, const float* b_u_in,
                                   const float* b_l_in, const float* relax_next, const float* add_next,
@@ -1654,6 +1701,7 @@ int bf_crown_relu_linear_relu_fwd(const float* A_u, const float* A_l, int64_t a_
   a.lda_d = a_dstride;
   a.ldc = P;
   a.B = W_t;
+  a.b_parts = b_parts;
   a.trans_b = 1;
   a.ldb = N;
   a.M = M;
@@ -1679,11 +1727,75 @@ int bf_crown_relu_linear_relu_fwd(const float* A_u, const float* A_l, int64_t a_
   return BF_OK;
 }
 
+int bf_crown_relu_linear_relu_fwd(const float* A_u, const float* A_l, int64_t a_dstride, int64_t D, int64_t S,
+                                  int64_t N, const float* relax, const float* add_l, int64_t add_ld,
+                                  const float* W_t, int64_t P, const float* bias, const float* b_u_in,
+                                  const float* b_l_in, const float* relax_next, const float* add_next,
+                                  int64_t add_next_ld, const float* bias_next, const float* cvec_next,
+                                  int64_t cvec_next_ld, float* workspace, float* A_next_u, float* A_next_l,
+                                  float* A_pre_u, float* A_pre_l, float* b_u_out, float* b_l_out, float* c_u_out,
+                                  float* c_l_out, hipStream_t stream) {
+  return relu_linear_relu_fwd(0, A_u, A_l, a_dstride, D, S, N, relax, add_l, add_ld, W_t, P, bias, b_u_in, b_l_in, relax_next, add_next, add_next_ld, bias_next, cvec_next, cvec_next_ld, workspace, A_next_u, A_next_l, A_pre_u, A_pre_l, b_u_out, b_l_out, c_u_out, c_l_out, stream);
+}
+
+// The two-region step of an already relaxed coefficient against a packed weight.
+int bf_crown_linear_relu_fwd_parts(const float* A_u, const float* A_l, int64_t a_dstride, int64_t D, int64_t S,
+                                   int64_t N, const float* parts, int64_t P, const float* b_u_in, const float* b_l_in,
+                                   const float* relax_next, const float* add_next, int64_t add_next_ld,
+                                   const float* bias_next, const float* cvec_next, int64_t cvec_next_ld,
+                                   float* workspace, float* A_next_u, float* A_next_l, float* A_pre_u, float* A_pre_l,
+                                   float* b_u_out, float* b_l_out, float* c_u_out, float* c_l_out,
+                                   hipStream_t stream) {
+  return relu_linear_relu_fwd(1, A_u, A_l, a_dstride, D, S, N, nullptr, nullptr, 0, parts, P, nullptr, b_u_in, b_l_in,
+                              relax_next, add_next, add_next_ld, bias_next, cvec_next, cvec_next_ld, workspace,
+                              A_next_u, A_next_l, A_pre_u, A_pre_l, b_u_out, b_l_out, c_u_out, c_l_out, stream);
+}
+
+int bf_crown_linear_parts(const float* A_u, const float* A_l, int64_t a_dstride, int64_t D, int64_t S, int64_t N,
+                          const float* parts, int64_t P, const float* bias, const float* b_u_in, const float* b_l_in,
+                          float* A_prev_u, float* A_prev_l, float* b_u_out, float* b_l_out, hipStream_t stream) {
+  BF_REQUIRE(D >= 0 && S >= 0 && N > 0 && P > 0, "bf_crown_linear_parts: bad sizes");
+  const int64_t M = D * S;
+  if (M == 0) return BF_OK;
+  BF_REQUIRE(parts != nullptr && (A_u || A_l), "bf_crown_linear_parts: null weight or no coefficient");
+  BF_REQUIRE((A_u != nullptr) == (A_prev_u != nullptr) && (A_l != nullptr) == (A_prev_l != nullptr),
+             "bf_crown_linear_parts: input/output pointer mismatch");
+  GemmArgs a;
+  memset(&a, 0, sizeof(a));
+  int nz = 0;
+  if (A_u) { a.A[nz] = A_u; a.C[nz++] = A_prev_u; }
+  if (A_l) { a.A[nz] = A_l; a.C[nz++] = A_prev_l; }
+  a.lda = N;
+  a.lda_d = a_dstride;
+  a.ldc = P;
+  a.B = parts;
+  a.b_parts = 1;
+  a.M = M;
+  a.N = P;
+  a.K = N;
+  a.S = S;
+  const int rc = gemm_dispatch(a, PRO_PLAIN, EPI_STORE, nz, stream);
+  if (rc || !(b_u_out || b_l_out)) return rc;
+  // the bias rows in a pass of their own (A read once, no coefficient written); b_out = b_in without a bias
+  if (bias) {
+    const RelaxSrc none{nullptr, nullptr, nullptr, nullptr, 0};
+    return relax_pass(A_u, A_l, a_dstride, D, S, N, none, nullptr, 0, bias, nullptr, b_u_in, b_l_in, nullptr, nullptr,
+                      b_u_out, b_l_out, nullptr, nullptr, stream, true);
+  }
+  for (int side = 0; side < 2; ++side) {
+    float* out = side == 0 ? b_u_out : b_l_out;
+    if (!out) continue;
+    const int r2 = rows_finalize(side == 0 ? b_u_in : b_l_in, nullptr, nullptr, 0, M, out, nullptr, stream);
+    if (r2) return r2;
+  }
+  return BF_OK;
+}
+
 int64_t bf_crown_relu_linear_relu_fwd_workspace(int64_t D, int64_t S, int64_t P) {
   return 4 * (int64_t)gemm_partial_count(P) * D * S;
 }
 
-int bf_crown_linear_concretize(const float* A_u, const float* A_l, int64_t a_dstride, int64_t D, int64_t S,
+static int linear_concretize(int b_parts, const float* A_u, const float* A_l, int64_t a_dstride, int64_t D, int64_t S,
                                int64_t N, const float* W_t, int64_t I, const float* rad, float eps, int norm_p,
                                const float* cen_u, const float* cen_l, const float* b_u, const float* b_l,
                                const float* h_scale, float* h_out, float* workspace, float* lb, float* ub,
@@ -1713,6 +1825,7 @@ int bf_crown_linear_concretize(const float* A_u, const float* A_l, int64_t a_dst
   a.lda = N;
   a.lda_d = a_dstride;
   a.B = W_t;
+  a.b_parts = b_parts;
   a.trans_b = 1;
   a.ldb = N;
   a.M = M;
@@ -1734,6 +1847,24 @@ int bf_crown_linear_concretize(const float* A_u, const float* A_l, int64_t a_dst
   }
   return concretize_finalize(A_u ? pu : nullptr, A_l ? pl : nullptr, nparts, M, cen_u, cen_l, b_u, b_l,
                              rad ? 1.0f : eps, norm_p, A_l ? lb : nullptr, A_u ? ub : nullptr, stream);
+}
+
+int bf_crown_linear_concretize(const float* A_u, const float* A_l, int64_t a_dstride, int64_t D, int64_t S,
+                               int64_t N, const float* W_t, int64_t I, const float* rad, float eps, int norm_p,
+                               const float* cen_u, const float* cen_l, const float* b_u, const float* b_l,
+                               const float* h_scale, float* h_out, float* workspace, float* lb, float* ub,
+                               hipStream_t stream) {
+  return linear_concretize(0, A_u, A_l, a_dstride, D, S, N, W_t, I, rad, eps, norm_p, cen_u, cen_l, b_u, b_l, h_scale, h_out,
+                           workspace, lb, ub, stream);
+}
+
+int bf_crown_linear_concretize_parts(const float* A_u, const float* A_l, int64_t a_dstride, int64_t D, int64_t S,
+                               int64_t N, const float* parts, int64_t I, const float* rad, float eps, int norm_p,
+                               const float* cen_u, const float* cen_l, const float* b_u, const float* b_l,
+                               const float* h_scale, float* h_out, float* workspace, float* lb, float* ub,
+                               hipStream_t stream) {
+  return linear_concretize(1, A_u, A_l, a_dstride, D, S, N, parts, I, rad, eps, norm_p, cen_u, cen_l, b_u, b_l, h_scale, h_out,
+                           workspace, lb, ub, stream);
 }
 
 int64_t bf_crown_linear_concretize_workspace(int64_t D, int64_t S, int64_t I) {

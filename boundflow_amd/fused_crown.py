@@ -37,7 +37,7 @@ import torch
 
 from . import _lib
 from .conv import packed_conv_transpose_weights
-from .crown import EPILOGUE_MIN_M, RELAX_PASS_MIN_K, derived, transposed
+from .crown import EPILOGUE_MIN_M, RELAX_PASS_MIN_K, derived, takes_parts, transposed, weight_parts
 from .profiling import launch as _timed
 
 
@@ -279,15 +279,16 @@ class HipFusedCrownExecutor:
         dl = torch.empty(D, S, device=dev, dtype=torch.float32)
         if request.kind == "linear":
             P = int(request.weight.shape[1])
-            Wt = transposed(request.weight)   # [P, N]: the kernel's faster operand layout, kept across calls
             pu = torch.empty(D, S, P, device=dev, dtype=torch.float32)
             pl = torch.empty(D, S, P, device=dev, dtype=torch.float32)
             table = torch.empty(D * N * 4, device=dev, dtype=torch.float32)
             with _timed("executor_relax_table", 0.0, 4.0 * 8 * D * N):
                 _lib.call("bf_relu_relax_table_from_planes", *[_lib.ptr(t) for t in planes], D * N, _lib.ptr(table), st)
-            if M < EPILOGUE_MIN_M and N >= RELAX_PASS_MIN_K:
-                # a region of few rows: the relaxation pass, then the plain-prologue contraction,
-                # whose 64 x 64 tiles spread the short grid over more CUs (as crown_backward does)
+            packed = takes_parts(M, P, N, S, nz=2)
+            if packed or (M < EPILOGUE_MIN_M and N >= RELAX_PASS_MIN_K):
+                # the relaxation pass, then the plain contraction: on the packed weight, or, for a
+                # region of few rows, as 64 x 64 tiles that spread the short grid over more CUs (as
+                # crown_backward does)
                 ru = torch.empty(M, N, device=dev, dtype=torch.float32)
                 rl = torch.empty(M, N, device=dev, dtype=torch.float32)
                 with _timed("executor_relu_relax", 0.0, 4.0 * (4 * M * N + 4 * D * N)):
@@ -295,13 +296,19 @@ class HipFusedCrownExecutor:
                               _lib.ptr(table), None, 0, _lib.ptr(bias), None, None, None, _lib.ptr(ru), _lib.ptr(rl),
                               _lib.ptr(du), _lib.ptr(dl), None, None, st)
                 with _timed("executor_linear", 4.0 * M * N * P, 4.0 * (2 * M * N + N * P + 2 * M * P)):
-                    _lib.call("bf_crown_relu_linear_fwd", _lib.ptr(ru), _lib.ptr(rl), S * N, D, S, N, None, None, 0,
-                              _lib.ptr(Wt), P, 1, None, None, None, _lib.ptr(pu), _lib.ptr(pl), None, None, st)
+                    rows = (None, None, None, _lib.ptr(pu), _lib.ptr(pl), None, None, st)
+                    if packed:
+                        _lib.call("bf_crown_linear_parts", _lib.ptr(ru), _lib.ptr(rl), S * N, D, S, N,
+                                  _lib.ptr(weight_parts(request.weight, False)), P, *rows)
+                    else:
+                        # W^T [P, N]: the kernel's faster operand layout, kept across calls
+                        _lib.call("bf_crown_relu_linear_fwd", _lib.ptr(ru), _lib.ptr(rl), S * N, D, S, N, None, None,
+                                  0, _lib.ptr(transposed(request.weight)), P, 1, *rows)
                 return FusedReluAffineResult(pu, pl, du, dl)
             with _timed("executor_relu_linear", 4.0 * M * N * P, 4.0 * (2 * M * N + 4 * D * N + N * P + 2 * M * P)):
                 _lib.call("bf_crown_relu_linear_fwd", _lib.ptr(request.A_u), _lib.ptr(request.A_l), S * N, D, S, N,
-                          _lib.ptr(table), None, 0, _lib.ptr(Wt), P, 1, _lib.ptr(bias), None, None, _lib.ptr(pu),
-                          _lib.ptr(pl), _lib.ptr(du), _lib.ptr(dl), st)
+                          _lib.ptr(table), None, 0, _lib.ptr(transposed(request.weight)), P, 1, _lib.ptr(bias), None, None,
+                          _lib.ptr(pu), _lib.ptr(pl), _lib.ptr(du), _lib.ptr(dl), st)
             return FusedReluAffineResult(pu, pl, du, dl)
         Co, Ho, Wo = (int(d) for d in request.output_shape)
         Ci, Hi, Wi = (int(d) for d in request.input_shape)

@@ -51,6 +51,48 @@ const char* bf_last_error(void);
  * No counterpart in the reference: introspection of this build's dispatch. */
 int bf_gemm_tile_config(int64_t M, int64_t N, int nz, int ksplit, int relax_prologue, int dl_operands);
 
+/* Contractions on the bf16 matrix cores.  A weight packed by bf_gemm_pack_parts (every
+ * value as three bf16 parts whose sum is the value, in the matrix operand order) serves
+ * contractions at fp32 accuracy at more than the fp32 MFMA rate: the *_parts entry points
+ * below, each the arithmetic of its namesake with the products of the parts down to
+ * 2^-24 of a product, summed in fp32.
+ * bf_gemm_parts_config: 1 when they take M rows (domains of S rows) x N outputs over K
+ * with nz bounds, else 0 (too few tiles, K below 64 or no multiple of 4, or rows past
+ * 32-bit offsets): the caller then takes the namesake.  Coefficient rows must be 16-byte
+ * aligned and dense.
+ * bf_gemm_pack_parts: count weights in one launch, B[j] as [N, K] (trans_b) or [K, N]
+ * row-major with row stride ldb -> parts[j], bf_gemm_parts_floats(N, K) floats, 16-byte
+ * aligned (host arrays of device pointers).
+ * No counterpart in the reference (its contractions are torch matmuls,
+ * runtime/crown_ibp.py:1371-1700). */
+int bf_gemm_parts_config(int64_t M, int64_t N, int64_t K, int64_t S, int nz);
+int64_t bf_gemm_parts_floats(int64_t N, int64_t K);
+int bf_gemm_pack_parts(int count, const float* const* B, const int64_t* ldb, const int* trans_b, const int64_t* N,
+                       const int64_t* K, float* const* parts, hipStream_t stream);
+
+/* bf_gemm_rank1 (unsplit), its B packed. */
+int bf_gemm_rank1_parts(const float* A, int64_t lda, const float* parts, float* C, int64_t ldc, int64_t M, int64_t N,
+                        int64_t K, int64_t S, const float* r_row, const float* v_col, int64_t v_ld,
+                        hipStream_t stream);
+/* bf_crown_relu_linear_fwd with nothing to relax, the weight [N, P] packed. */
+int bf_crown_linear_parts(const float* A_u, const float* A_l, int64_t a_dstride, int64_t D, int64_t S, int64_t N,
+                          const float* parts, int64_t P, const float* bias, const float* b_u_in, const float* b_l_in,
+                          float* A_prev_u, float* A_prev_l, float* b_u_out, float* b_l_out, hipStream_t stream);
+/* bf_crown_relu_linear_relu_fwd of an already relaxed coefficient, the weight packed. */
+int bf_crown_linear_relu_fwd_parts(const float* A_u, const float* A_l, int64_t a_dstride, int64_t D, int64_t S,
+                                   int64_t N, const float* parts, int64_t P, const float* b_u_in, const float* b_l_in,
+                                   const float* relax_next, const float* add_next, int64_t add_next_ld,
+                                   const float* bias_next, const float* cvec_next, int64_t cvec_next_ld,
+                                   float* workspace, float* A_next_u, float* A_next_l, float* A_pre_u, float* A_pre_l,
+                                   float* b_u_out, float* b_l_out, float* c_u_out, float* c_l_out,
+                                   hipStream_t stream);
+/* bf_crown_linear_concretize, the weight packed. */
+int bf_crown_linear_concretize_parts(const float* A_u, const float* A_l, int64_t a_dstride, int64_t D, int64_t S,
+                                     int64_t N, const float* parts, int64_t I, const float* rad, float eps, int norm_p,
+                                     const float* cen_u, const float* cen_l, const float* b_u, const float* b_l,
+                                     const float* h_scale, float* h_out, float* workspace, float* lb, float* ub,
+                                     hipStream_t stream);
+
 /* ---- kernel #1: IBP ---------------------------------------------------- */
 
 /* Interval linear layer in center/radius form, with the consumer ReLU's split
