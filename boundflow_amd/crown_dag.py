@@ -352,7 +352,7 @@ def crown_backward_dag(
     kept for ``lower_grad_pass``.  With ``relu_influence`` each ReLU input x reached by the
     backward gets max over specs of max(|A_u|, |A_l|) of the coefficient of the ReLU's
     output, [B, *shape of x] (crown_ibp.py:1810-1833)."""
-    from .crown import _flat_param, _init_spec, takes_parts, transposed, weight_parts
+    from .crown import STORE, _flat_param, _init_spec, takes_parts, transposed, weight_parts
 
     task = _module_task(module)
     params = module.params
@@ -471,7 +471,7 @@ def crown_backward_dag(
             with _timed("crown_linear", 2.0 * nz * M * N * P, 4.0 * nz * (M * N + N * P + M * P)):
                 rows = (_lib.ptr(bias), _lib.ptr(st.b_u), _lib.ptr(None if one else st.b_l), _lib.ptr(nA_u),
                         _lib.ptr(None if one else nA_l), _lib.ptr(nb_u), _lib.ptr(None if one else nb_l), stream)
-                if takes_parts(M, P, N, S, st.A_u, A_l_in):
+                if takes_parts(STORE, M, P, N, S, st.A_u, A_l_in):
                     _lib.call("bf_crown_linear_parts", _lib.ptr(st.A_u), _lib.ptr(A_l_in), S * N, B, S, N,
                               _lib.ptr(weight_parts(params[op.inputs[1]], False)), P, *rows)
                 else:
@@ -636,7 +636,7 @@ def lower_grad_pass(module: BFTaskModule, spec: InputSpec, trace: DagTrace, save
     G bias^T; relu through the relaxation (bf_relu_grad, which also reduces dL/dalpha and
     dL/dbeta); add the sum of its operands' gradients (plus G c^T for a constant c);
     concat the concatenation of its operands' gradients; flatten/reshape the same rows."""
-    from .crown import takes_parts, weight_parts
+    from .crown import STORE, takes_parts, weight_parts
 
     task = _module_task(module)
     params = module.params
@@ -669,12 +669,13 @@ def lower_grad_pass(module: BFTaskModule, spec: InputSpec, trace: DagTrace, save
             gt = torch.empty(M, n_out, device=dev)
             rank1 = (_lib.ptr(G if bias is not None else None), _lib.ptr(bias), 0)
             with _timed("grad_gemm", 2.0 * M * n_in * n_out, 4.0 * (M * n_in + M * n_out + n_in * n_out)):
-                if takes_parts(M, n_out, n_in, S, GA[x]):
+                wsz = int(_lib.load().bf_gemm_rank1_workspace(M, n_out, n_in))
+                # (a contraction the fp32 kernels split over K keeps the split)
+                if not wsz and takes_parts(STORE, M, n_out, n_in, S, GA[x]):
                     _lib.call("bf_gemm_rank1_parts", _lib.ptr(GA[x]), n_in,
                               _lib.ptr(weight_parts(params[op.inputs[1]], True)), _lib.ptr(gt), n_out, M, n_out, n_in,
                               S, *rank1, stream)
                 else:
-                    wsz = int(_lib.load().bf_gemm_rank1_workspace(M, n_out, n_in))
                     ws = torch.empty(wsz, device=dev) if wsz else None
                     _lib.call("bf_gemm_rank1", _lib.ptr(GA[x]), n_in, _lib.ptr(W), n_in, 1, _lib.ptr(gt), n_out, M,
                               n_out, n_in, S, *rank1, _lib.ptr(ws), wsz, stream)

@@ -130,20 +130,30 @@ int gemm_tile_choice(int64_t M, int64_t N, int nz, int64_t ks, int pro, bool dl)
 }
 
 int gemm_norm_cols(int64_t M, int64_t N, int pro);
-int launch_parts(const GemmArgs& a, int epi, int nz, hipStream_t stream);
+int launch_parts(const GemmArgs& a, int epi, int nz, bool small, hipStream_t stream);
 
-// Whether the three-part kernels take a plain contraction of this shape (packed weight, domains of
-// S rows): K whole float4s and at least four stages deep, rows within the 32-bit byte offsets of a
-// tile, and at least 128 tiles of 128 x 128.  A tile's stage takes about 0.64 us with one wave per
-// SIMD, so fewer tiles are bound by that latency and the fp32 tiles, which deal a short grid as 64 x
-// 64 over four times as many CUs, are level or faster (us on one MI355X, fp32 / parts): 72 tiles at
-// K = 512 26.2 / 27.3, at K = 256 16.6 / 16.8; 144 tiles 35.9 / 28.2 and 21.9 / 17.5, at K = 64
-// 10.6 / 9.3; 288 tiles 57.9 / 32.9; 1008 tiles 184.0 / 85.6.
-int gemm_parts_choice(int64_t M, int64_t N, int64_t K, int64_t S, int nz) {
-  if (kForcedTile || M <= 0 || N <= 0 || K < 64 || K % 4 != 0 || S <= 0 || N >= (1LL << 31) || K >= (1LL << 31))
+// The tile on which the three-part kernels take a plain contraction of this shape (packed weight,
+// domains of S rows, epilogue epi): 'P' (128 x 128), 'S' (64 x 64) or 0.  K must be whole float4s
+// and four stages deep and rows lie within the 32-bit byte offsets of a tile; a launch below 256 rows
+// is bound by its launch and its K loop on either kind (9 x 256 x 256: 10.0 / 9.9 us fp32 / 64 x 64).
+// us on one MI355X, fp32 / 64 x 64 / 128 x 128:
+//   576 x 256: K = 64 7.5 / 5.9 / 8.0, 256 11.7 / 10.6 / 14.9, 512 17.4 / 16.7 / 24.0, 1024 28.7 / 29.0 / 42.1
+//   2304 x 512 (288 64 x 64 tiles): K = 64 8.6 / 7.1 / 8.6, 256 16.1 / 13.0 / 15.6, 1024 44.2 / 37.2 / 43.1
+//   4608 x 784 (936): K = 256 26.8 / 17.0 / 17.8, 1024 81.3 / 51.1 / 51.0
+//   9216 x 784 (1872): K = 256 42.1 / 32.6 / 26.6;  36864 x 256 (2304): 54.9 / 35.7 / 34.9
+// so the store epilogue takes 64 x 64 below 1536 of them (six per CU, what is resident at once), and
+// past K = 512 leaves a grid that is not one tile per CU to the fp32 kernels.  The norm epilogue's tile
+// follows its partial norms' width; it and the relaxation epilogue take 128 x 128 from 128 tiles on
+// (72 tiles: level with fp32).
+int gemm_parts_choice(int64_t M, int64_t N, int64_t K, int64_t S, int nz, int epi) {
+  if (kForcedTile || M < 256 || N <= 0 || K < 64 || K % 4 != 0 || S <= 0 || N >= (1LL << 31) || K >= (1LL << 31))
     return 0;
   if (S >= (1LL << 29) / 4 || (512 + 4 * S) >= (1LL << 29) / K) return 0;
-  return ceil_div(M, (int64_t)128) * ceil_div(N, (int64_t)128) * nz >= 128 ? 1 : 0;
+  const int64_t t64 = ceil_div(M, (int64_t)64) * ceil_div(N, (int64_t)64) * nz;
+  const bool short_k = K <= 512 || t64 >= 256;
+  if (epi == EPI_STORE && t64 < 1536) return short_k ? 'S' : 0;
+  if (epi == EPI_ABSSUM && gemm_norm_cols(M, N, PRO_PLAIN) == NORM_BN / 2) return short_k ? 'S' : 0;
+  return ceil_div(M, (int64_t)128) * ceil_div(N, (int64_t)128) * nz >= 128 ? 'P' : 0;
 }
 
 int gemm_dispatch(const GemmArgs& a, int pro, int epi, int nz, hipStream_t stream) {
@@ -154,10 +164,11 @@ int gemm_dispatch(const GemmArgs& a, int pro, int epi, int nz, hipStream_t strea
   if (a.b_parts) {
     bool rows = a.lda == a.K && a.lda_d >= 0 && a.lda_d % 4 == 0 && a.lda_d <= 2 * a.S * a.K;
     for (int z = 0; z < nz; ++z) rows = rows && ((uintptr_t)a.A[z] & 15) == 0;
-    BF_REQUIRE(gemm_parts_choice(a.M, a.N, a.K, a.S, nz) && rows && pro == PRO_PLAIN && a.ksplit <= 1,
+    const int tile = gemm_parts_choice(a.M, a.N, a.K, a.S, nz, epi);
+    BF_REQUIRE(tile && rows && pro == PRO_PLAIN && a.ksplit <= 1,
                "gemm: a packed weight does not serve M=%lld N=%lld K=%lld with these rows (bf_gemm_parts_config)",
                (long long)a.M, (long long)a.N, (long long)a.K);
-    return launch_parts(a, epi, nz, stream);
+    return launch_parts(a, epi, nz, tile == 'S', stream);
   }
   const int64_t ks = (pro == PRO_PLAIN && epi == EPI_STORE && a.ksplit > 1) ? a.ksplit : 1;
   const bool dl = gemm_dl_operands(a, nz);

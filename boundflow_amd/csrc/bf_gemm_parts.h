@@ -37,9 +37,9 @@ typedef uint32_t uint32x4 __attribute__((ext_vector_type(4)));
 // values (column l % 32, k 8 (l / 32) .. + 7) at 16 l; columns and k past the end are zero.
 constexpr int PARTS_BLOCK = 3 * 64 * 4;   // floats of one block and stage
 
-template <int FM_, int NWM_, int OCC_>
+template <int FM_, int FN_, int NWM_, int OCC_>
 struct TileParts {
-  static constexpr int FM = FM_, FN = 4, NWM = NWM_, NWN = 1, OCC = OCC_;
+  static constexpr int FM = FM_, FN = FN_, NWM = NWM_, NWN = 1, OCC = OCC_;
   static constexpr int WTM = 32 * FM, WTN = 32 * FN;   // wave tile
   static constexpr int BM = WTM * NWM, BN = WTN, BK = 16, NT = 64 * NWM;
   static constexpr int A_STAGE = BM * BK;              // floats of a stage of A rows
@@ -72,7 +72,7 @@ __device__ __forceinline__ void split_parts(float (&v)[8], uint32x4 (&part)[3]) 
 }
 
 template <int EPI, class T>
-__global__ void __launch_bounds__(T::NT, T::OCC * T::NWM / 4) gemm_parts_kernel(GemmArgs p) {
+__global__ void __launch_bounds__(T::NT, (T::OCC * T::NWM + 3) / 4) gemm_parts_kernel(GemmArgs p) {
   constexpr int FM = T::FM, FN = T::FN, GBM = T::BM, GBN = T::BN, GBK = T::BK;
   // three stages of A rows, two of B parts; the relaxation epilogue stages its operands over all of it
   constexpr int SMEM = 3 * T::A_STAGE + 2 * T::B_STAGE;
@@ -166,56 +166,89 @@ __global__ void __launch_bounds__(T::NT, T::OCC * T::NWM / 4) gemm_parts_kernel(
 #pragma unroll
   for (int jq = 0; jq < 2; ++jq) a_pos[jq] = 4 * (4 * lrow + ((2 * h + jq) ^ swz));
 
+  // One stage: its MFMAs, between them the split of the next stage's A rows, a part of a pair of
+  // values (five VALU instructions) at a time, in the cycles the matrix cores take for the MFMA
+  // before it.  The fences pin that order and the B reads one column block ahead of their use; left
+  // to itself the compiler puts every split before the first MFMA.
   auto main_loop = [&](auto full_c) {
     constexpr bool FULL = decltype(full_c)::value;
+    uint32x4 ap[2][FM][3];   // the A parts of this stage and of the next
+    float v[FM][8];
+    auto read_a = [&](int slot) {
+#pragma unroll
+      for (int i = 0; i < FM; ++i) {
+        const float* src = a_wave + slot * T::A_STAGE + 512 * i;
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          const float4 f = *reinterpret_cast<const float4*>(src + a_pos[q]);
+          v[i][4 * q] = f.x; v[i][4 * q + 1] = f.y; v[i][4 * q + 2] = f.z; v[i][4 * q + 3] = f.w;
+        }
+      }
+    };
+    constexpr int SPLITS = 12 * FM;   // part u / 4 % 3 of value pair u % 4 of row block u / 12
+    auto split = [&](uint32x4 (&part)[FM][3], int u) {
+      part[u / 12][u / 4 % 3][u % 4] = take_part(v[u / 12][2 * (u % 4)], v[u / 12][2 * (u % 4) + 1]);
+    };
     copy_a(0, 0);
     copy_b(0, 0);
     if (nk > 1) copy_a(1, 1);
-    int sa = 0;   // A slot of stage kt
-    for (int kt = 0; kt < nk; ++kt) {
-      const int sb = kt & 1;
-      // this stage's copies have landed; the next stage's A rows may still be in flight
-      if (kt + 1 < nk) wait_vmem<CHUNKS>(); else wait_vmem<0>();
+    if (nk > 2) copy_a(2, 2);
+    if (nk > 2) wait_vmem<2 * CHUNKS>(); else if (nk > 1) wait_vmem<CHUNKS>(); else wait_vmem<0>();
+    read_a(0);
+#pragma unroll
+    for (int u = 0; u < SPLITS; ++u) split(ap[0], u);
+    int sa = 0;   // A slot of the stage
+    auto stage = [&](int kt, auto parity) {
+      constexpr int cur = decltype(parity)::value;
+      // the next stage's A rows and this one's B parts have landed; the A rows after them may not have
+      if (kt + 2 < nk) wait_vmem<CHUNKS>(); else wait_vmem<0>();
       lds_barrier();   // every wave's B parts are there; no wave reads the slots refilled next
-      if (kt + 1 < nk) copy_b(sb ^ 1, kt + 1);
-      if (kt + 2 < nk) copy_a(sa == 0 ? 2 : sa - 1, kt + 2);
-      const float* __restrict__ bst = bs + sb * T::B_STAGE + 4 * lane;
-      uint32x4 ap[FM][3], bp[2][3];
+      if (kt + 1 < nk) copy_b(cur ^ 1, kt + 1);
+      if (kt + 3 < nk) copy_a(sa, kt + 3);
+      sa = sa == 2 ? 0 : sa + 1;
+      const float* __restrict__ bst = bs + cur * T::B_STAGE + 4 * lane;
+      uint32x4 bp[2][3];
       auto read_b = [&](int j) {
 #pragma unroll
-        for (int s = 0; s < 3; ++s)
-          bp[j & 1][s] = *reinterpret_cast<const uint32x4*>(bst + j * PARTS_BLOCK + 256 * s);
+        for (int q = 0; q < 3; ++q)
+          bp[j & 1][q] = *reinterpret_cast<const uint32x4*>(bst + j * PARTS_BLOCK + 256 * q);
       };
-#pragma unroll
-      for (int i = 0; i < FM; ++i) {
-        const float* src = a_wave + sa * T::A_STAGE + 512 * i;
-        const float4 lo = *reinterpret_cast<const float4*>(src + a_pos[0]);
-        const float4 hi = *reinterpret_cast<const float4*>(src + a_pos[1]);
-        if (i == FM - 1) read_b(0);
-        float v[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
-        split_parts(v, ap[i]);
-      }
-      // the B parts of a column block are read one block ahead of their MFMAs (the fences keep
-      // the compiler from moving the reads to where they are used)
+      read_b(0);
+      read_a(sa);   // (past the last stage: what the slot held, split for nothing)
       __builtin_amdgcn_sched_barrier(0);
+      constexpr int MFMAS = 6 * FM;   // of a column block
 #pragma unroll
       for (int j = 0; j < FN; ++j) {
-        if (!FULL && j >= fn_act) continue;
+        const bool on = FULL || j < fn_act;
         if (j + 1 < FN && (FULL || j + 1 < fn_act)) read_b(j + 1);
         __builtin_amdgcn_sched_barrier(0);
         // the smallest products first
         constexpr int PA[6] = {2, 0, 1, 1, 0, 0}, PB[6] = {0, 2, 1, 0, 1, 0};
 #pragma unroll
-        for (int q = 0; q < 6; ++q)
-#pragma unroll
-          for (int i = 0; i < FM; ++i)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, ap[i][PA[q]]),
+        for (int m = 0; m < MFMAS; ++m) {
+          const int q = m / FM, i = m % FM;
+          if (on)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, ap[cur][i][PA[q]]),
                                                                 __builtin_bit_cast(bf16x8, bp[j & 1][PB[q]]),
                                                                 acc[i][j], 0, 0, 0);
-        __builtin_amdgcn_sched_barrier(0);
+          // (the first block leaves the A reads time to land)
+          constexpr int FIRST = FN > 2 ? 1 : 0;
+          if (j >= FIRST) {
+            constexpr int N = (FN - FIRST) * MFMAS;
+            const int at = (j - FIRST) * MFMAS + m;
+#pragma unroll
+            for (int u = at * SPLITS / N; u < (at + 1) * SPLITS / N; ++u) split(ap[cur ^ 1], u);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
       }
-      sa = sa == 2 ? 0 : sa + 1;
+    };
+    int kt = 0;
+    for (; kt + 2 <= nk; kt += 2) {
+      stage(kt, std::integral_constant<int, 0>{});
+      stage(kt + 1, std::integral_constant<int, 1>{});
     }
+    if (kt < nk) stage(kt, std::integral_constant<int, 0>{});
   };
   if (fn_act == FN) main_loop(std::true_type{});
   else main_loop(std::false_type{});
@@ -265,9 +298,9 @@ __global__ void __launch_bounds__(T::NT, T::OCC * T::NWM / 4) gemm_parts_kernel(
   parts_epilogue<EPI, T, SMEM>(p, acc, smem_ab, red, m0, n0, tile_n, wave, 0, lane, z, lower);
 }
 
-// 128 x 128, 4 waves of 32 x 128, 3 workgroups per CU
-using TileP = TileParts<1, 4, 3>;
+using TileP = TileParts<1, 4, 4, 3>;    // 128 x 128, 4 waves of 32 x 128, 3 workgroups per CU
+using TilePS = TileParts<1, 2, 2, 6>;   // 64 x 64, 2 waves of 32 x 64, 6 workgroups per CU
 
-int launch_parts(const GemmArgs& a, int epi, int nz, hipStream_t stream);
+int launch_parts(const GemmArgs& a, int epi, int nz, bool small, hipStream_t stream);
 
 }  // namespace bf

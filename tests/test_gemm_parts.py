@@ -23,12 +23,21 @@ def test_shapes_taken():
         pytest.skip("library not built (run python -m boundflow_amd.build)")
     if os.environ.get("BOUNDFLOW_GEMM_TILE"):
         pytest.skip("tile forced by the environment")
-    assert config(128000, 500, 500, 500, 2) and config(36864, 256, 256, 9, 1)
-    assert config(128 * 127 + 1, 1, 64, 9, 1) and not config(128 * 127, 1, 64, 9, 1)      # 128 tiles
-    assert config(128 * 63 + 1, 128, 64, 9, 2) and not config(128 * 63 + 1, 128, 64, 9, 1)
-    assert not config(36864, 256, 60, 9, 1) and not config(36864, 256, 254, 9, 1)         # K short, K ragged
-    assert not config(10 ** 7, 256, 256, 10 ** 6, 1)                                      # rows past 32-bit offsets
-    assert not config(0, 256, 256, 9, 1) and not config(36864, 256, 256, 9, 3) and not config(36864, 256, 256, 0, 1)
+    tile = lambda *a: chr(config(*a)) if config(*a) else ""   # noqa: E731
+    for form in (0, 1, 2):
+        assert tile(128000, 500, 500, 500, 2, form) == "P" and tile(36864, 256, 256, 9, 1, form) == "P"
+        assert not tile(36864, 256, 60, 9, 1, form) and not tile(36864, 256, 254, 9, 1, form)   # K short, K ragged
+        assert not tile(10 ** 7, 256, 256, 10 ** 6, 1, form)                        # rows past 32-bit offsets
+        assert not tile(0, 256, 256, 9, 1, form) and not tile(36864, 256, 256, 9, 3, form)
+        assert not tile(36864, 256, 256, 0, 1, form) and not tile(255, 256, 256, 9, 1, form)
+    # stores: 64 x 64 below 1536 such tiles, past K = 512 only with one per CU
+    assert tile(64 * 1536, 64, 256, 9, 1, 0) == "P" and tile(64 * 1535, 64, 256, 9, 1, 0) == "S"
+    assert tile(256, 64, 512, 9, 1, 0) == "S" and not tile(256, 64, 516, 9, 1, 0) and tile(64 * 128, 64, 516, 9, 2, 0) == "S"
+    # the norm epilogue's tile is its partial norms' width (64 columns on short grids); the others 128 tiles
+    assert tile(576, 784, 256, 9, 2, 1) == "S" and not tile(576, 784, 256, 9, 2, 2)
+    assert tile(64 * 128, 128, 256, 9, 2, 1) == "P" and not tile(64 * 128, 128, 256, 9, 1, 1)
+    assert tile(128 * 127 + 1, 128, 64, 9, 1, 2) == "P" and not tile(128 * 127, 128, 64, 9, 1, 2)
+    assert not config(36864, 256, 256, 9, 1, 3)
 
 
 def pack(W, trans_b):
@@ -44,16 +53,17 @@ def gen(*key):
     return torch.Generator().manual_seed(sum((i + 1) * int(k) for i, k in enumerate(key)))
 
 
-# tiles of 128 x 128 x 16: one row past a tile and one short of it, one column past a 32-column
-# block and past a tile, K of one to three whole float4s past a stage
+# tiles of 128 x 128 and 64 x 64, stages of 16 k: one row past a tile and one short of it, one column
+# past a 32-column block and past a tile, K of one to three whole float4s past a stage
 @gpu
-@pytest.mark.parametrize("M,N,K,S", [(16257, 128, 64, 9), (16384, 127, 68, 16384), (8321, 161, 76, 1),
-                                     (12672, 129, 252, 9), (4608, 500, 500, 512)])
+@pytest.mark.parametrize("M,N,K,S", [(49153, 128, 64, 9), (98303, 127, 68, 16384), (32897, 161, 76, 1),
+                                     (32769, 129, 252, 9), (12800, 500, 500, 512), (256, 1, 64, 9), (257, 65, 68, 300),
+                                     (575, 97, 508, 9), (2304, 256, 512, 9), (8191, 127, 1028, 1)])
 @pytest.mark.parametrize("trans_b", [True, False])
 def test_store_matches_fp64(M, N, K, S, trans_b):
     dev = device()
     announce(f"parts store M={M} N={N} K={K} S={S} trans_b={trans_b}")
-    assert config(M, N, K, S, 1)
+    assert config(M, N, K, S, 1, 0)
     g = gen(M, N, K, trans_b)
     A = torch.randn(M, K, generator=g)
     B = torch.randn(N, K, generator=g)
@@ -74,7 +84,7 @@ def test_store_matches_fp64(M, N, K, S, trans_b):
 
 
 @gpu
-@pytest.mark.parametrize("M,N,K", [(36864, 256, 256), (16384, 129, 500)])
+@pytest.mark.parametrize("M,N,K", [(36864, 256, 256), (16384, 129, 500), (2304, 256, 512)])
 @pytest.mark.parametrize("positive", [False, True])
 def test_error_is_not_above_the_fp32_tiles(M, N, K, positive):
     """Root mean square error against float64, beside that of the fp32 MFMA contraction."""
@@ -102,7 +112,7 @@ def test_relaxation_epilogue_matches_fp64(D, S, N, P, cvec, extra, bounds):
     dev = device()
     M = D * S
     announce(f"parts relaxation epilogue D={D} S={S} N={N} P={P} cvec={cvec} extra={extra} bounds={bounds}")
-    assert config(M, P, N, S, bounds)
+    assert config(M, P, N, S, bounds, 2)
     g = gen(D, S, N, P)
     W = torch.randn(N, P, generator=g) / N ** 0.5
     lo = torch.randn(D, P, generator=g)
@@ -163,12 +173,13 @@ def test_relaxation_epilogue_matches_fp64(D, S, N, P, cvec, extra, bounds):
 
 @gpu
 @pytest.mark.parametrize("D,S,N,I,box,norm_p", [(1600, 9, 64, 129, False, 0), (900, 9, 100, 784, True, 0),
-                                                (1025, 9, 256, 65, False, 1), (700, 13, 68, 161, False, 2)])
+                                                (1025, 9, 256, 65, False, 1), (700, 13, 68, 161, False, 2),
+                                                (64, 9, 256, 784, True, 0), (29, 9, 64, 65, False, 2)])
 def test_concretize_matches_fp64(D, S, N, I, box, norm_p):
     dev = device()
     M = D * S
     announce(f"parts concretize D={D} S={S} N={N} I={I} box={box} norm_p={norm_p}")
-    assert config(M, I, N, S, 2)
+    assert config(M, I, N, S, 2, 1)
     g = gen(D, S, N, I)
     A = {q: torch.randn(M, N, generator=g) for q in "ul"}
     W = torch.randn(N, I, generator=g) * 0.1
@@ -203,11 +214,11 @@ def test_concretize_matches_fp64(D, S, N, I, box, norm_p):
 
 
 @gpu
-def test_operands_that_are_not_finite():
+@pytest.mark.parametrize("M,N,K", [(65536, 128, 68), (9100, 128, 68)])   # 128 x 128 and 64 x 64 tiles
+def test_operands_that_are_not_finite(M, N, K):
     """Infinities, NaN and values between the largest bf16 and the largest fp32 give what the fp32
     contraction gives, and leave every other row and column alone."""
     dev = device()
-    M, N, K = 16384, 128, 68
     g = gen(M, N, K)
     A = torch.randn(M, K, generator=g)
     B = torch.randn(N, K, generator=g)
@@ -240,6 +251,6 @@ def test_refused_operands_raise():
     call = lambda a, M, K: _lib.call("bf_gemm_rank1_parts", _lib.ptr(a), K, _lib.ptr(W), _lib.ptr(C), 256, M, 256, K, 9,
                                      None, None, 0, _lib.stream_handle())   # noqa: E731
     with pytest.raises(_lib.HipError):
-        call(A, 64, 256)                                   # too few tiles
+        call(A, 64, 256)                                   # too few rows
     with pytest.raises(_lib.HipError):
         call(A.reshape(-1)[1:36864 * 256 + 1], 36864, 256)   # rows off 16-byte alignment
