@@ -220,7 +220,7 @@ def _grad_pass(spec: InputSpec, chain: Chain, trace: ForwardTrace, saved: dict, 
             with _timed("grad_gemm", 2.0 * M * n_in * n_out, 4.0 * (M * n_in + M * n_out + n_in * n_out)):
                 wsz = int(_lib.load().bf_gemm_rank1_workspace(M, n_out, n_in))
                 # (a contraction the fp32 kernels split over K keeps the split)
-                if not wsz and takes_parts(STORE, M, n_out, n_in, S, g):
+                if not wsz and takes_parts(STORE, M, n_out, n_in, S, 1):
                     _lib.call("bf_gemm_rank1_parts", _lib.ptr(g), n_in, _lib.ptr(weight_parts(layer.weight, True)),
                               _lib.ptr(gt), n_out, M, n_out, n_in, S, *rank1, stream)
                 else:

@@ -206,9 +206,9 @@ def chain_parts(layers: List[AffineLayer], layer: AffineLayer, M: int, S: int, n
             if other.kind != "linear":
                 continue
             n, p = _numel(other.out_shape), _numel(other.in_shape)
-            if takes_parts(CONCRETIZE if k == 0 else STORE, M, p, n, S, nz=nz):
+            if takes_parts(CONCRETIZE if k == 0 else STORE, M, p, n, S, nz):
                 yield other.weight, False
-            if save is not None and save.get("grad_rows") is not None and takes_parts(STORE, M, n, p, S, nz=1):
+            if save is not None and save.get("grad_rows") is not None and takes_parts(STORE, M, n, p, S, 1):
                 yield other.weight, True
     return weight_parts(layer.weight, trans_b, also())
 
@@ -217,15 +217,12 @@ def chain_parts(layers: List[AffineLayer], layer: AffineLayer, M: int, S: int, n
 STORE, CONCRETIZE, RELAX = 0, 1, 2
 
 
-def takes_parts(form: int, M: int, N: int, K: int, S: int, *coeffs: Optional[torch.Tensor], nz: int = 0) -> bool:
+def takes_parts(form: int, M: int, N: int, K: int, S: int, nz: int) -> bool:
     """Whether the contraction of M coefficient rows (S per domain) of K values into N runs on
-    packed weight parts: the library's rule on the form and the shape, and 16-byte aligned rows
-    (``nz`` in place of ``coeffs``: that many bounds, whose rows are still to be made)."""
-    if K < 64 or K % 4 or M < 256:   # (most small queries end here, without a call into the library)
+    packed weight parts: the library's rule on the form and the shape (``nz`` bounds)."""
+    if K < 16 or M < 256:   # (most small queries end here, without a call into the library)
         return False
-    nz = nz or sum(t is not None for t in coeffs)
-    return (all(t is None or t.data_ptr() % 16 == 0 for t in coeffs)
-            and _lib.load().bf_gemm_parts_config(M, N, K, S, nz, form) != 0)
+    return _lib.load().bf_gemm_parts_config(M, N, K, S, nz, form) != 0
 
 
 # ---------------------------------------------------------------------------
@@ -668,7 +665,7 @@ def crown_backward(
         small_grid = M < EPILOGUE_MIN_M and N >= RELAX_PASS_MIN_K
         # (few rows per domain: no epilogue relaxed them, and the packed weight takes no prologue)
         packed = relaxes and takes_parts(CONCRETIZE if k == 0 else STORE, M, P, N, S,
-                                         nz=int(A_u is not None) + int(A_l is not None))
+                                         int(A_u is not None) + int(A_l is not None))
         if relaxes and (shared_first or small_grid or relax_pass_next or packed):
             # A coefficient shared by every domain (the first region of a C = I query):
             # its relaxation differs per domain, so one bandwidth-bound pass writes it
@@ -716,7 +713,7 @@ def crown_backward(
                 save["h"] = h_out
                 save["cvec"] = trace.input_center_proj.get(layer.out_name)
             nz = int(A_u is not None) + int(A_l is not None)
-            in_parts = takes_parts(CONCRETIZE, M, P, N, S, A_u, A_l)
+            in_parts = takes_parts(CONCRETIZE, M, P, N, S, nz)
             # bytes: the coefficient rows and the weight read, the row partial norms written, the
             # gradient seed [M, P] written when asked
             with _timed("crown_linear_concretize", 2.0 * nz * M * N * P,
@@ -808,7 +805,7 @@ def crown_backward(
                 after = (_lib.ptr(b_u), _lib.ptr(b_l), _lib.ptr(n_table), _lib.ptr(n_add), n_add_ld, _lib.ptr(n_bias),
                          _lib.ptr(cvec), P, _lib.ptr(ws), _lib.ptr(nA_u), _lib.ptr(nA_l), None, _lib.ptr(pre_l),
                          _lib.ptr(nb_u), _lib.ptr(nb_l), _lib.ptr(nc_u), _lib.ptr(nc_l), stream)
-                if plain and takes_parts(RELAX, M, P, N, S, A_u, A_l):
+                if plain and takes_parts(RELAX, M, P, N, S, nz):
                     _lib.call("bf_crown_linear_relu_fwd_parts", _lib.ptr(A_u), _lib.ptr(A_l), stride, B, S, N,
                               _lib.ptr(chain_parts(layers, layer, M, S, nz, save)), P, *after)
                 else:
@@ -840,7 +837,7 @@ def crown_backward(
                         _lib.ptr(nA_u), _lib.ptr(nA_l), None if keep_b else _lib.ptr(nb_u),
                         None if keep_b else _lib.ptr(nb_l), stream)
                 with _timed("crown_relu_linear_fwd", flops, nbytes):
-                    if plain and takes_parts(STORE, M, P, N, S, A_u, A_l):
+                    if plain and takes_parts(STORE, M, P, N, S, nz):
                         _lib.call("bf_crown_linear_parts", _lib.ptr(A_u), _lib.ptr(A_l), stride, B, S, N,
                                   _lib.ptr(chain_parts(layers, layer, M, S, nz, save)), P, *rows)
                     else:

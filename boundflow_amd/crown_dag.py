@@ -471,7 +471,7 @@ def crown_backward_dag(
             with _timed("crown_linear", 2.0 * nz * M * N * P, 4.0 * nz * (M * N + N * P + M * P)):
                 rows = (_lib.ptr(bias), _lib.ptr(st.b_u), _lib.ptr(None if one else st.b_l), _lib.ptr(nA_u),
                         _lib.ptr(None if one else nA_l), _lib.ptr(nb_u), _lib.ptr(None if one else nb_l), stream)
-                if takes_parts(STORE, M, P, N, S, st.A_u, A_l_in):
+                if takes_parts(STORE, M, P, N, S, nz):
                     _lib.call("bf_crown_linear_parts", _lib.ptr(st.A_u), _lib.ptr(A_l_in), S * N, B, S, N,
                               _lib.ptr(weight_parts(params[op.inputs[1]], False)), P, *rows)
                 else:
@@ -671,7 +671,7 @@ def lower_grad_pass(module: BFTaskModule, spec: InputSpec, trace: DagTrace, save
             with _timed("grad_gemm", 2.0 * M * n_in * n_out, 4.0 * (M * n_in + M * n_out + n_in * n_out)):
                 wsz = int(_lib.load().bf_gemm_rank1_workspace(M, n_out, n_in))
                 # (a contraction the fp32 kernels split over K keeps the split)
-                if not wsz and takes_parts(STORE, M, n_out, n_in, S, GA[x]):
+                if not wsz and takes_parts(STORE, M, n_out, n_in, S, 1):
                     _lib.call("bf_gemm_rank1_parts", _lib.ptr(GA[x]), n_in,
                               _lib.ptr(weight_parts(params[op.inputs[1]], True)), _lib.ptr(gt), n_out, M, n_out, n_in,
                               S, *rank1, stream)

@@ -133,20 +133,23 @@ int gemm_norm_cols(int64_t M, int64_t N, int pro);
 int launch_parts(const GemmArgs& a, int epi, int nz, bool small, hipStream_t stream);
 
 // The tile on which the three-part kernels take a plain contraction of this shape (packed weight,
-// domains of S rows, epilogue epi): 'P' (128 x 128), 'S' (64 x 64) or 0.  K must be whole float4s
-// and four stages deep and rows lie within the 32-bit byte offsets of a tile; a launch below 256 rows
-// is bound by its launch and its K loop on either kind (9 x 256 x 256: 10.0 / 9.9 us fp32 / 64 x 64).
+// domains of S rows, epilogue epi): 'P' (128 x 128), 'S' (64 x 64) or 0.  K must fill a stage and
+// rows lie within the 32-bit byte offsets of a tile; a launch below 256 rows is bound by its launch
+// and its K loop on either kind (9 x 256 x 256: 10.0 / 9.9 us fp32 / 64 x 64).
 // us on one MI355X, fp32 / 64 x 64 / 128 x 128:
 //   576 x 256: K = 64 7.5 / 5.9 / 8.0, 256 11.7 / 10.6 / 14.9, 512 17.4 / 16.7 / 24.0, 1024 28.7 / 29.0 / 42.1
 //   2304 x 512 (288 64 x 64 tiles): K = 64 8.6 / 7.1 / 8.6, 256 16.1 / 13.0 / 15.6, 1024 44.2 / 37.2 / 43.1
 //   4608 x 784 (936): K = 256 26.8 / 17.0 / 17.8, 1024 81.3 / 51.1 / 51.0
 //   9216 x 784 (1872): K = 256 42.1 / 32.6 / 26.6;  36864 x 256 (2304): 54.9 / 35.7 / 34.9
+// and where K is no multiple of four (the fp32 tiles then read their operands float by float), fp32 /
+// the tile taken: 2304 x 50: K = 30 7.3 / 6.4, 50 8.6 / 7.6, 333 19.9 / 17.7; 36864 x 250: K = 30
+// 23.0 / 14.6, 50 33.0 / 17.9, 250 93.6 / 39.2; 100000 x 50: K = 50 32.4 / 21.0;
 // so the store epilogue takes 64 x 64 below 1536 of them (six per CU, what is resident at once), and
 // past K = 512 leaves a grid that is not one tile per CU to the fp32 kernels.  The norm epilogue's tile
 // follows its partial norms' width; it and the relaxation epilogue take 128 x 128 from 128 tiles on
 // (72 tiles: level with fp32).
 int gemm_parts_choice(int64_t M, int64_t N, int64_t K, int64_t S, int nz, int epi) {
-  if (kForcedTile || M < 256 || N <= 0 || K < 64 || K % 4 != 0 || S <= 0 || N >= (1LL << 31) || K >= (1LL << 31))
+  if (kForcedTile || M < 256 || N <= 0 || K < 16 || S <= 0 || N >= (1LL << 31) || K >= (1LL << 31))
     return 0;
   if (S >= (1LL << 29) / 4 || (512 + 4 * S) >= (1LL << 29) / K) return 0;
   const int64_t t64 = ceil_div(M, (int64_t)64) * ceil_div(N, (int64_t)64) * nz;
@@ -162,8 +165,7 @@ int gemm_dispatch(const GemmArgs& a, int pro, int epi, int nz, hipStream_t strea
     return BF_EINVAL;
   }
   if (a.b_parts) {
-    bool rows = a.lda == a.K && a.lda_d >= 0 && a.lda_d % 4 == 0 && a.lda_d <= 2 * a.S * a.K;
-    for (int z = 0; z < nz; ++z) rows = rows && ((uintptr_t)a.A[z] & 15) == 0;
+    const bool rows = a.lda == a.K && a.lda_d >= 0 && a.lda_d <= 2 * a.S * a.K;
     const int tile = gemm_parts_choice(a.M, a.N, a.K, a.S, nz, epi);
     BF_REQUIRE(tile && rows && pro == PRO_PLAIN && a.ksplit <= 1,
                "gemm: a packed weight does not serve M=%lld N=%lld K=%lld with these rows (bf_gemm_parts_config)",

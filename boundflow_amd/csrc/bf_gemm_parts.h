@@ -54,6 +54,16 @@ __device__ __forceinline__ void lds_copy16_at(const float* base, uint32_t byte_o
   asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(byte_off), "s"(base), "s"(off) : "memory");
 }
 
+// The same, four bytes a lane (256 of LDS in a row), from a scalar base or a lane's own address.
+__device__ __forceinline__ void lds_copy4_at(const float* base, uint32_t byte_off, float* lds_dst) {
+  const uint32_t off = (uint32_t)(uintptr_t)((lds_float*)lds_dst);
+  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dword %0, %1" ::"v"(byte_off), "s"(base), "s"(off) : "memory");
+}
+__device__ __forceinline__ void lds_copy4(const float* src, float* lds_dst) {
+  const uint32_t off = (uint32_t)(uintptr_t)((lds_float*)lds_dst);
+  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dword %0, off" ::"v"(src), "s"(off) : "memory");
+}
+
 // (x, y) -> the packed bf16 pair nearest to it, and what the pair leaves of both.
 __device__ __forceinline__ uint32_t take_part(float& x, float& y) {
   const floatx2 xy = {x, y};
@@ -71,7 +81,9 @@ __device__ __forceinline__ void split_parts(float (&v)[8], uint32x4 (&part)[3]) 
     for (int e = 0; e < 4; ++e) part[q][e] = take_part(v[2 * e], v[2 * e + 1]);
 }
 
-template <int EPI, class T>
+// VEC: coefficient rows of whole 16-byte aligned float4s; else they are copied float by float (a row
+// length that is no multiple of four), the same stage in four times as many copies.
+template <int EPI, class T, bool VEC>
 __global__ void __launch_bounds__(T::NT, (T::OCC * T::NWM + 3) / 4) gemm_parts_kernel(GemmArgs p) {
   constexpr int FM = T::FM, FN = T::FN, GBM = T::BM, GBN = T::BN, GBK = T::BK;
   // three stages of A rows, two of B parts; the relaxation epilogue stages its operands over all of it
@@ -106,30 +118,41 @@ __global__ void __launch_bounds__(T::NT, (T::OCC * T::NWM + 3) / 4) gemm_parts_k
   // at position 4 r + (kq ^ (r / 2 % 4)) of the chunk, as in gemm_kernel's direct-to-LDS loop.
   // Byte offsets from the tile's first domain (below 2^32, checked at launch): a stage advances
   // the scalar base alone.
-  constexpr int CHUNKS = T::WTM / 16;
+  constexpr int CHUNKS = VEC ? T::WTM / 16 : T::WTM / 4;   // copies of a stage: of 16 rows, or of 4
+  constexpr int CHUNK = VEC ? 256 : 64;                    // floats of one
   const int64_t d0 = div_rows(m0, p.S, fits32);
   const float* __restrict__ a_base = p.A[z] + d0 * p.lda_d;
   uint32_t a_off[CHUNKS];
-  const int a_kq = (lane & 3) ^ ((lane >> 3) & 3);
+  int a_k[VEC ? 1 : 2];   // this lane's k of a stage (float by float: of even and of odd chunks)
+  if constexpr (VEC) {
+    a_k[0] = 4 * ((lane & 3) ^ ((lane >> 3) & 3));
+  } else {
+#pragma unroll
+    for (int j = 0; j < 2; ++j) a_k[j] = 4 * (((lane >> 2) & 3) ^ (2 * j + (lane >> 5))) + (lane & 3);
+  }
 #pragma unroll
   for (int j = 0; j < CHUNKS; ++j) {
-    const int64_t mr = m0 + wave * T::WTM + 16 * j + (lane >> 2);
+    const int64_t mr = m0 + wave * T::WTM + (VEC ? 16 * j + (lane >> 2) : 4 * j + (lane >> 4));
     const int64_t m = mr < M ? mr : M - 1;
     const int64_t d = div_rows(m, p.S, fits32);
-    a_off[j] = (uint32_t)(4 * ((d - d0) * p.lda_d + (m - d * p.S) * p.lda + 4 * a_kq));
+    a_off[j] = (uint32_t)(4 * ((d - d0) * p.lda_d + (m - d * p.S) * p.lda + a_k[VEC ? 0 : j & 1]));
   }
   float* const a_wave = smem_ab + wave * T::WTM * GBK;
   auto copy_a = [&](int slot, int kt) {
     float* dst = a_wave + slot * T::A_STAGE;
     const float* src = a_base + (int64_t)kt * GBK;
-    if (kt * GBK + GBK <= K) {
+    const bool whole = kt * GBK + GBK <= K;
 #pragma unroll
-      for (int j = 0; j < CHUNKS; ++j) lds_copy16_at(src, a_off[j], dst + 256 * j);
-    } else {
-      // quads past K read the row start: they meet the zeros that B's parts hold there
-      const int back = kt * GBK + 4 * a_kq < K ? 0 : kt * GBK + 4 * a_kq;
-#pragma unroll
-      for (int j = 0; j < CHUNKS; ++j) lds_copy16(src + (int64_t)(a_off[j] / 4) - back, dst + 256 * j);
+    for (int j = 0; j < CHUNKS; ++j) {
+      // k past the end reads the row start: it meets the zeros that B's parts hold there
+      const int k = kt * GBK + a_k[VEC ? 0 : j & 1];
+      if constexpr (VEC) {
+        if (whole) lds_copy16_at(src, a_off[j], dst + CHUNK * j);
+        else lds_copy16(src + (int64_t)(a_off[j] / 4) - (k < K ? 0 : k), dst + CHUNK * j);
+      } else {
+        if (whole) lds_copy4_at(src, a_off[j], dst + CHUNK * j);
+        else lds_copy4(src + (int64_t)(a_off[j] / 4) - (k < K ? 0 : k), dst + CHUNK * j);
+      }
     }
   };
   // this wave's copies of a B stage: block * 3 + part = B_COPIES wave .. ; blocks past N copy the

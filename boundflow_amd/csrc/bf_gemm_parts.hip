@@ -79,18 +79,18 @@ int pack_parts(int count, const float* const* B, const int64_t* ldb, const int* 
   return BF_OK;
 }
 
-template <class T>
+template <class T, bool VEC>
 static int launch_tile(const GemmArgs& a, int epi, int nz, hipStream_t stream) {
   const int64_t ntiles = ceil_div(a.M, (int64_t)T::BM) * ceil_div(a.N, (int64_t)T::BN);
   BF_REQUIRE(ntiles + 8 < (1LL << 31), "gemm grid too large (M=%lld N=%lld)", (long long)a.M, (long long)a.N);
   const dim3 grid((unsigned)(ceil_div(ntiles, 8) * 8), (unsigned)nz), block(T::NT);
   if (epi == EPI_STORE) {
-    hipLaunchKernelGGL((gemm_parts_kernel<EPI_STORE, T>), grid, block, 0, stream, a);
+    hipLaunchKernelGGL((gemm_parts_kernel<EPI_STORE, T, VEC>), grid, block, 0, stream, a);
   } else if (epi == EPI_ABSSUM) {
-    hipLaunchKernelGGL((gemm_parts_kernel<EPI_ABSSUM, T>), grid, block, 0, stream, a);
+    hipLaunchKernelGGL((gemm_parts_kernel<EPI_ABSSUM, T, VEC>), grid, block, 0, stream, a);
   } else {
     if constexpr (T::BN == NORM_BN) {
-      hipLaunchKernelGGL((gemm_parts_kernel<EPI_RELAX, T>), grid, block, 0, stream, a);
+      hipLaunchKernelGGL((gemm_parts_kernel<EPI_RELAX, T, VEC>), grid, block, 0, stream, a);
     } else {
       set_error("gemm: the relaxation epilogue takes 128-column tiles");
       return BF_EINVAL;
@@ -101,7 +101,10 @@ static int launch_tile(const GemmArgs& a, int epi, int nz, hipStream_t stream) {
 }
 
 int launch_parts(const GemmArgs& a, int epi, int nz, bool small, hipStream_t stream) {
-  return small ? launch_tile<TilePS>(a, epi, nz, stream) : launch_tile<TileP>(a, epi, nz, stream);
+  bool vec = a.K % 4 == 0 && a.lda % 4 == 0 && a.lda_d % 4 == 0;
+  for (int z = 0; z < nz; ++z) vec = vec && ((uintptr_t)a.A[z] & 15) == 0;
+  if (vec) return small ? launch_tile<TilePS, true>(a, epi, nz, stream) : launch_tile<TileP, true>(a, epi, nz, stream);
+  return small ? launch_tile<TilePS, false>(a, epi, nz, stream) : launch_tile<TileP, false>(a, epi, nz, stream);
 }
 
 }  // namespace bf

@@ -675,6 +675,88 @@ relu_relax_rows_kernel(const float* __restrict__ Au, const float* __restrict__ A
   }
 }
 
+// The scalar pass for many rows per domain (a row length that is no multiple of four, at most 64 NQ):
+// a workgroup takes rows_per_wg rows of one domain and each lane keeps that domain's relaxation
+// entries, split term, bias and center of its k in registers across them, up to four rows'
+// coefficients in flight per wave.  The row kernel above repeats the box's loads and division and the
+// row's domain for every row.  It stays bound by its four-byte stores: 50 x 50 coefficients shared by
+// 1000 domains, both bounds with all sums, 27.3 -> 21.9 us; 333 x 333 by 256 144 -> 113 us (2.0 TB/s
+// written); 250 x 250 by 40 16.2 -> 13.5 us.  (With the row kernel's shuffles in place of wave_sum 35.7,
+// 133 and 17.1 us.)
+template <int NQ>
+__global__ void __launch_bounds__(256)
+relu_relax_domain_kernel(const float* __restrict__ Au, const float* __restrict__ Al, int64_t a_dstride, int64_t S,
+                         int64_t K, int64_t chunks, int rows_per_wg, RelaxSrc relax, const float* __restrict__ add_l,
+                         int64_t add_ld, const float* __restrict__ kbias, const float* __restrict__ cvec,
+                         const float* __restrict__ bu_in, const float* __restrict__ bl_in,
+                         float* __restrict__ Au_out, float* __restrict__ Al_out, float* __restrict__ bu_out,
+                         float* __restrict__ bl_out, float* __restrict__ cu_out, float* __restrict__ cl_out) {
+  constexpr int R = NQ <= 2 ? 4 : 2;   // rows in flight per wave
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t d = (int64_t)blockIdx.x / chunks;
+  const int64_t s0 = ((int64_t)blockIdx.x - d * chunks) * rows_per_wg;
+  const int64_t s_end = s0 + rows_per_wg < S ? s0 + rows_per_wg : S;
+  float4 e[NQ];
+  float kbv[NQ], cvv[NQ], adv[NQ];
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) {
+    const int64_t k = lane + 64 * q;
+    const bool ok = k < K;
+    e[q] = ok ? relax.at(d, K, k) : make_float4(1.f, 0.f, 1.f, 0.f);
+    kbv[q] = ok && kbias ? kbias[k] : 0.f;
+    cvv[q] = ok && cvec ? cvec[d * K + k] : 0.f;
+    adv[q] = ok && add_l ? add_l[d * add_ld + k] : 0.f;
+  }
+  const bool same = Au == Al;
+  // one bound of one row: the relaxed coefficient stored, its sums into the row outputs
+  auto bound = [&](const float (&v)[NQ], int64_t m, bool lower, float* __restrict__ out, const float* __restrict__ b_in,
+                   float* __restrict__ b_out, float* __restrict__ c_out) {
+    float sb = 0.f, sk = 0.f, sc = 0.f;
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+      const int64_t k = lane + 64 * q;
+      if (k >= K) continue;
+      const bool first = (v[q] >= 0.f) != lower;   // the upper entry of a nonnegative upper coefficient, ...
+      float o = v[q] * (first ? e[q].x : e[q].z);
+      sb += v[q] * (first ? e[q].y : e[q].w);
+      if (lower && add_l) o = o + adv[q];
+      if (kbias) sk += o * kbv[q];
+      if (cvec) sc += o * cvv[q];
+      if (out) out[m * K + k] = o;
+    }
+    if (b_out) {
+      sb = wave_sum(sb);
+      if (kbias) sk = wave_sum(sk);
+      if (lane == 0) b_out[m] = ((b_in ? b_in[m] : 0.f) + sb) + sk;
+    }
+    if (c_out) {
+      sc = wave_sum(sc);
+      if (lane == 0) c_out[m] = sc;
+    }
+  };
+  for (int64_t base = s0 + wave * R; base < s_end; base += 4 * R) {
+    float vu[R][NQ], vl[R][NQ];
+#pragma unroll
+    for (int u = 0; u < R; ++u) {
+      const int64_t at = d * a_dstride + (base + u < s_end ? base + u : s_end - 1) * K;
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) {
+        const int64_t k = lane + 64 * q;
+        vu[u][q] = Au && k < K ? Au[at + k] : 0.f;
+        vl[u][q] = Al && !same && k < K ? Al[at + k] : vu[u][q];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < R; ++u) {
+      if (base + u >= s_end) break;   // uniform
+      const int64_t m = d * S + base + u;
+      if (Au) bound(vu[u], m, false, Au_out, bu_in, bu_out, cu_out);
+      if (Al) bound(vl[u], m, true, Al_out, bl_in, bl_out, cl_out);
+    }
+  }
+}
+
 // The same pass, vectorized: TPR threads per row (256 / TPR rows per
 // workgroup), each thread handling 4 consecutive k per step, so a row of K
 // coefficients is covered in ceil(K / (4 TPR)) steps with two 16-byte loads per
@@ -1919,6 +2001,21 @@ static int relax_pass(const float* A_u, const float* A_l, int64_t a_dstride, int
                        a_dstride, M, S, K, src, add_l, add_ld, kbias, cvec, b_u_in, b_l_in, A_u_out, A_l_out, b_u_out,
                        b_l_out, c_u_out, c_l_out);
     BF_LAUNCH_CHECK("relu_relax_rows4_kernel<64>");
+  } else if (!vec && K <= 512 && S >= 16 && M >= 1024) {
+    // (fewer rows: 16 rows of 77 in 100 domains 9.2 / 9.0 us, row / domain kernel)
+    const int rpw = 16;
+    const int64_t chunks = ceil_div(S, rpw);
+    BF_REQUIRE(D * chunks < (1LL << 31), "bf_crown_relu_relax: too many rows");
+    auto launch = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3((unsigned)(D * chunks)), dim3(256), 0, stream, A_u, A_l, a_dstride, S, K, chunks,
+                         rpw, src, add_l, add_ld, kbias, cvec, b_u_in, b_l_in, A_u_out, A_l_out, b_u_out, b_l_out,
+                         c_u_out, c_l_out);
+    };
+    if (K <= 64) launch(relu_relax_domain_kernel<1>);
+    else if (K <= 128) launch(relu_relax_domain_kernel<2>);
+    else if (K <= 256) launch(relu_relax_domain_kernel<4>);
+    else launch(relu_relax_domain_kernel<8>);
+    BF_LAUNCH_CHECK("relu_relax_domain_kernel");
   } else {
     hipLaunchKernelGGL(relu_relax_rows_kernel, dim3((unsigned)ceil_div(M, 4)), dim3(256), 0, stream, A_u, A_l,
                        a_dstride, M, S, K, src, add_l, add_ld, kbias, cvec, b_u_in, b_l_in, A_u_out, A_l_out, b_u_out,

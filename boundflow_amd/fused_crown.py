@@ -284,7 +284,7 @@ class HipFusedCrownExecutor:
             table = torch.empty(D * N * 4, device=dev, dtype=torch.float32)
             with _timed("executor_relax_table", 0.0, 4.0 * 8 * D * N):
                 _lib.call("bf_relu_relax_table_from_planes", *[_lib.ptr(t) for t in planes], D * N, _lib.ptr(table), st)
-            packed = takes_parts(STORE, M, P, N, S, nz=2)
+            packed = takes_parts(STORE, M, P, N, S, 2)
             if packed or (M < EPILOGUE_MIN_M and N >= RELAX_PASS_MIN_K):
                 # the relaxation pass, then the plain contraction: on the packed weight, or, for a
                 # region of few rows, as 64 x 64 tiles that spread the short grid over more CUs (as

@@ -57,11 +57,11 @@ int bf_gemm_tile_config(int64_t M, int64_t N, int nz, int ksplit, int relax_prol
  * below, each the arithmetic of its namesake with the products of the parts down to
  * 2^-24 of a product, summed in fp32.
  * bf_gemm_parts_config: the tile on which they take M rows (domains of S rows) x N outputs
- * over K with nz bounds, 'P' (128 x 128) or 'S' (64 x 64), else 0 (K below 64 or no
- * multiple of 4, a grid the fp32 kernels run as fast, or rows past 32-bit offsets): the
- * caller then takes the namesake.  form: 0 the stores (bf_gemm_rank1_parts,
+ * over K with nz bounds, 'P' (128 x 128) or 'S' (64 x 64), else 0 (K below 16, a grid
+ * the fp32 kernels run as fast, or rows past 32-bit offsets): the caller then takes the
+ * namesake.  form: 0 the stores (bf_gemm_rank1_parts,
  * bf_crown_linear_parts), 1 bf_crown_linear_concretize_parts, 2 bf_crown_linear_relu_fwd_parts.
- * Coefficient rows must be 16-byte aligned and dense.
+ * Coefficient rows must be dense.
  * bf_gemm_pack_parts: count weights in one launch, B[j] as [N, K] (trans_b) or [K, N]
  * row-major with row stride ldb -> parts[j], bf_gemm_parts_floats(N, K) floats, 16-byte
  * aligned (host arrays of device pointers).

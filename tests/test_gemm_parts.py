@@ -26,7 +26,7 @@ def test_shapes_taken():
     tile = lambda *a: chr(config(*a)) if config(*a) else ""   # noqa: E731
     for form in (0, 1, 2):
         assert tile(128000, 500, 500, 500, 2, form) == "P" and tile(36864, 256, 256, 9, 1, form) == "P"
-        assert not tile(36864, 256, 60, 9, 1, form) and not tile(36864, 256, 254, 9, 1, form)   # K short, K ragged
+        assert tile(36864, 256, 16, 9, 1, form) == "P" and not tile(36864, 256, 15, 9, 1, form)   # a whole stage
         assert not tile(10 ** 7, 256, 256, 10 ** 6, 1, form)                        # rows past 32-bit offsets
         assert not tile(0, 256, 256, 9, 1, form) and not tile(36864, 256, 256, 9, 3, form)
         assert not tile(36864, 256, 256, 0, 1, form) and not tile(255, 256, 256, 9, 1, form)
@@ -58,7 +58,9 @@ def gen(*key):
 @gpu
 @pytest.mark.parametrize("M,N,K,S", [(49153, 128, 64, 9), (98303, 127, 68, 16384), (32897, 161, 76, 1),
                                      (32769, 129, 252, 9), (12800, 500, 500, 512), (256, 1, 64, 9), (257, 65, 68, 300),
-                                     (575, 97, 508, 9), (2304, 256, 512, 9), (8191, 127, 1028, 1)])
+                                     (575, 97, 508, 9), (2304, 256, 512, 9), (8191, 127, 1028, 1),
+                                     # K no multiple of four: rows copied float by float
+                                     (49153, 129, 17, 9), (98303, 63, 50, 16384), (257, 65, 31, 300), (2303, 50, 333, 1)])
 @pytest.mark.parametrize("trans_b", [True, False])
 def test_store_matches_fp64(M, N, K, S, trans_b):
     dev = device()
@@ -106,7 +108,8 @@ def test_error_is_not_above_the_fp32_tiles(M, N, K, positive):
 
 @gpu
 @pytest.mark.parametrize("D,S,N,P,cvec,extra,bounds", [(1600, 9, 64, 129, True, True, 1), (300, 33, 100, 500, False, False, 2),
-                                                       (6000, 3, 128, 160, True, False, 2), (40, 500, 252, 96, True, True, 1)])
+                                                       (6000, 3, 128, 160, True, False, 2), (40, 500, 252, 96, True, True, 1),
+                                                                  (1000, 50, 50, 50, True, True, 1), (2000, 9, 77, 130, False, False, 2)])
 def test_relaxation_epilogue_matches_fp64(D, S, N, P, cvec, extra, bounds):
     """9 and 3 rows per domain: a tile spans 16 domains (entries in LDS) and 44 (read from memory)."""
     dev = device()
@@ -174,7 +177,8 @@ def test_relaxation_epilogue_matches_fp64(D, S, N, P, cvec, extra, bounds):
 @gpu
 @pytest.mark.parametrize("D,S,N,I,box,norm_p", [(1600, 9, 64, 129, False, 0), (900, 9, 100, 784, True, 0),
                                                 (1025, 9, 256, 65, False, 1), (700, 13, 68, 161, False, 2),
-                                                (64, 9, 256, 784, True, 0), (29, 9, 64, 65, False, 2)])
+                                                (64, 9, 256, 784, True, 0), (29, 9, 64, 65, False, 2),
+                                                (400, 50, 50, 5, True, 0), (64, 9, 77, 784, False, 1)])
 def test_concretize_matches_fp64(D, S, N, I, box, norm_p):
     dev = device()
     M = D * S
@@ -214,7 +218,7 @@ def test_concretize_matches_fp64(D, S, N, I, box, norm_p):
 
 
 @gpu
-@pytest.mark.parametrize("M,N,K", [(65536, 128, 68), (9100, 128, 68)])   # 128 x 128 and 64 x 64 tiles
+@pytest.mark.parametrize("M,N,K", [(65536, 128, 68), (9100, 128, 68), (9100, 128, 69)])   # both tiles, both copies
 def test_operands_that_are_not_finite(M, N, K):
     """Infinities, NaN and values between the largest bf16 and the largest fp32 give what the fp32
     contraction gives, and leave every other row and column alone."""
@@ -222,8 +226,8 @@ def test_operands_that_are_not_finite(M, N, K):
     g = gen(M, N, K)
     A = torch.randn(M, K, generator=g)
     B = torch.randn(N, K, generator=g)
-    A[5, 3], A[300, 66], A[5000, 0], A[9000, 67] = float("inf"), float("nan"), 3.4e38, -float("inf")
-    B[7, 2], B[40, 67], B[100, 1] = float("inf"), float("nan"), -3.4e38
+    A[5, 3], A[300, 66], A[5000, 0], A[9000, K - 1] = float("inf"), float("nan"), 3.4e38, -float("inf")
+    B[7, 2], B[40, K - 1], B[100, 1] = float("inf"), float("nan"), -3.4e38
     Ad, Bd = A.to(dev), B.to(dev)
     C, C32 = torch.empty(M, N, device=dev), torch.empty(M, N, device=dev)
     _lib.call("bf_gemm_rank1_parts", _lib.ptr(Ad), K, _lib.ptr(pack(Bd, True)), _lib.ptr(C), N, M, N, K, 9, None, None,
@@ -244,13 +248,19 @@ def test_operands_that_are_not_finite(M, N, K):
 
 
 @gpu
-def test_refused_operands_raise():
+def test_unaligned_rows_and_refused_shapes():
     dev = device()
-    A, C = torch.zeros(36865, 256, device=dev), torch.zeros(36864, 256, device=dev)
-    W = pack(torch.randn(256, 256, device=dev), True)
-    call = lambda a, M, K: _lib.call("bf_gemm_rank1_parts", _lib.ptr(a), K, _lib.ptr(W), _lib.ptr(C), 256, M, 256, K, 9,
-                                     None, None, 0, _lib.stream_handle())   # noqa: E731
+    g = torch.Generator(device=dev).manual_seed(3)
+    A, B = torch.randn(2304 * 64 + 1, generator=g, device=dev), torch.randn(128, 64, generator=g, device=dev)
+    W = pack(B, True)
+
+    def run(a, M, K):
+        C = torch.empty(M, 128, device=dev)
+        _lib.call("bf_gemm_rank1_parts", _lib.ptr(a), K, _lib.ptr(W), _lib.ptr(C), 128, M, 128, K, 9, None, None, 0,
+                  _lib.stream_handle())
+        return C
+
+    off = A[1:].reshape(2304, 64)                       # one float off 16-byte alignment: the same bits
+    assert torch.equal(run(off, 2304, 64), run(off.clone(), 2304, 64))
     with pytest.raises(_lib.HipError):
-        call(A, 64, 256)                                   # too few rows
-    with pytest.raises(_lib.HipError):
-        call(A.reshape(-1)[1:36864 * 256 + 1], 36864, 256)   # rows off 16-byte alignment
+        run(off, 64, 64)                                # too few rows

@@ -1,0 +1,61 @@
+"""The relaxation pass over rows whose length is no multiple of four and that come many to a domain
+(each lane keeps its domain's operands over 16 rows): against float64, on one lane's worth of columns
+past and short of a register of them, a shared coefficient and one per domain, either bound alone."""
+
+import pytest
+import torch
+
+from boundflow_amd import _lib
+from tests.gpu_util import announce, device
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("D,S,K,shared,sides", [(64, 16, 63, True, "ul"), (61, 17, 65, False, "ul"), (40, 50, 50, True, "l"),
+                                                (70, 16, 129, False, "u"), (30, 35, 257, True, "ul"), (33, 33, 510, False, "ul")])
+@pytest.mark.parametrize("extras", [True, False])
+def test_many_rows_per_domain_match_fp64(D, S, K, shared, sides, extras):
+    dev = device()
+    M = D * S
+    announce(f"relaxation pass D={D} S={S} K={K} shared={shared} sides={sides} extras={extras}")
+    g = torch.Generator().manual_seed(D + 3 * S + 7 * K + extras)
+    A = {q: torch.randn(S if shared else M, K, generator=g) for q in sides}
+    lo = torch.randn(D, K, generator=g)
+    hi = lo + torch.rand(D, K, generator=g) * 2
+    alpha = torch.rand(D, K, generator=g) if extras else None
+    add = torch.randn(D, K, generator=g) if extras else None
+    cen = torch.randn(D, K, generator=g) if extras else None
+    bias, b0 = torch.randn(K, generator=g), torch.randn(M, generator=g)
+    table = torch.empty(D, K, 4, device=dev)
+    d = lambda t: None if t is None else t.to(dev)   # noqa: E731
+    lo_d, hi_d, al_d, add_d, cen_d, bias_d, b0_d = (d(t) for t in (lo, hi, alpha, add, cen, bias, b0))
+    _lib.call("bf_relu_relax_table", _lib.ptr(lo_d), _lib.ptr(hi_d), _lib.ptr(al_d), K, D, K, _lib.ptr(table),
+              _lib.stream_handle())
+    A_d = {q: d(A[q]) for q in sides}
+    out = {q: torch.empty(M, K, device=dev) for q in sides}
+    bo = {q: torch.empty(M, device=dev) for q in sides}
+    co = {q: torch.empty(M, device=dev) for q in sides} if extras else {}
+    p = lambda m, q: _lib.ptr(m.get(q))   # noqa: E731
+    _lib.call("bf_crown_relu_relax_lu", p(A_d, "u"), p(A_d, "l"), 0 if shared else S * K, D, S, K, _lib.ptr(lo_d),
+              _lib.ptr(hi_d), _lib.ptr(al_d), K, _lib.ptr(add_d), K, _lib.ptr(bias_d), _lib.ptr(cen_d), _lib.ptr(b0_d),
+              _lib.ptr(b0_d), p(out, "u"), p(out, "l"), p(bo, "u"), p(bo, "l"), p(co, "u"), p(co, "l"),
+              _lib.stream_handle())
+    torch.cuda.synchronize()
+    dom = torch.arange(M) // S
+    tab = table.cpu().double()[dom]
+    for q in sides:
+        a = (A[q].repeat(D, 1) if shared else A[q]).double()
+        take_u = a < 0 if q == "l" else a >= 0
+        nxt = a * torch.where(take_u, tab[..., 0], tab[..., 2])
+        beta = a * torch.where(take_u, tab[..., 1], tab[..., 3])
+        if q == "l" and extras:
+            nxt = nxt + add.double()[dom]
+        err = (out[q].cpu().double() - nxt).abs()
+        assert bool((err <= 2.0 ** -22 * (nxt.abs() + (add.double().abs()[dom] if extras else 0.0)) + 1e-30).all())
+        sums = [(bo[q], b0.double() + beta.sum(1) + (nxt * bias.double()).sum(1),
+                 b0.double().abs() + beta.abs().sum(1) + (nxt * bias.double()).abs().sum(1))]
+        if extras:
+            sums.append((co[q], (nxt * cen.double()[dom]).sum(1), (nxt * cen.double()[dom]).abs().sum(1)))
+        for got, want, size in sums:
+            err = (got.cpu().double() - want).abs()
+            assert bool((err <= (K + 8) * 2.0 ** -23 * size + 1e-30).all()), float((err / size).max())
