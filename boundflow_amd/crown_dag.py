@@ -352,7 +352,7 @@ def crown_backward_dag(
     kept for ``lower_grad_pass``.  With ``relu_influence`` each ReLU input x reached by the
     backward gets max over specs of max(|A_u|, |A_l|) of the coefficient of the ReLU's
     output, [B, *shape of x] (crown_ibp.py:1810-1833)."""
-    from .crown import STORE, _flat_param, _init_spec, takes_parts, transposed, weight_parts
+    from .crown import STORE, _flat_param, _init_spec, derived, takes_parts, transposed, weight_parts
 
     task = _module_task(module)
     params = module.params
@@ -402,9 +402,9 @@ def crown_backward_dag(
         return (zero_b if st.b_u is not None else None), (zero_b if st.b_l is not None else None)
 
     def rows_pass(st: _Rows, n: int, *, pre=None, alpha=None, alpha_ld=0, add=None, add_ld=0, kbias=None,
-                  cvec=None, name="crown_relu_relax"):
-        """bf_crown_relu_relax_lu over the bounds st carries: (A', b + sums, center sums).  Without a
-        relaxation, rows shared by both bounds are passed once."""
+                  cvec=None, name="crown_relu_relax", two: Optional[_Rows] = None):
+        """bf_crown_relu_relax_lu over the bounds st carries (``two``: over the sum of st and two):
+        (A', b + sums, center sums).  Without a relaxation, rows shared by both bounds are passed once."""
         one = pre is None and add is None and shared(st)
         rA_u, rA_l = like(st, n, one)
         nb_u, nb_l = like(_Rows(st.b_u, st.b_l, None, None), 1, one)
@@ -415,6 +415,15 @@ def crown_backward_dag(
         A_l_in = None if one else st.A_l
         nz = int(st.A_u is not None) + int(A_l_in is not None)
         reads = 1 if (nz == 2 and ptr_of(st.A_u) == ptr_of(st.A_l)) else nz
+        if two is not None:
+            with _timed(name, 0.0, 4.0 * (reads + 2 * nz) * M * n):
+                _lib.call("bf_crown_relu_relax_sum_lu", _lib.ptr(st.A_u), _lib.ptr(st.A_l), _lib.ptr(two.A_u),
+                          _lib.ptr(two.A_l), B, S, n, _lib.ptr(pre.lower.reshape(B, n)),
+                          _lib.ptr(pre.upper.reshape(B, n)), _lib.ptr(alpha), alpha_ld,
+                          _lib.ptr(add if st.A_l is not None else None), add_ld, _lib.ptr(kbias), _lib.ptr(st.b_u),
+                          _lib.ptr(st.b_l), _lib.ptr(two.b_u), _lib.ptr(two.b_l), _lib.ptr(rA_u), _lib.ptr(rA_l),
+                          _lib.ptr(nb_u), _lib.ptr(nb_l), stream)
+            return _Rows(rA_u, rA_l, nb_u, nb_l), (None, None)
         with _timed(name, 0.0, 4.0 * (reads + nz) * M * n):
             _lib.call("bf_crown_relu_relax_lu", _lib.ptr(st.A_u), _lib.ptr(A_l_in), S * n, B, S, n,
                       _lib.ptr(None if pre is None else pre.lower.reshape(B, n)),
@@ -433,11 +442,23 @@ def crown_backward_dag(
         return out
 
     def accumulate(name: str, upd: _Rows) -> None:
-        """crown_ibp.py:892-909: current + update, coefficients and bias rows."""
+        """crown_ibp.py:892-909: current + update, coefficients and bias rows.  A ReLU's second
+        adjoint waits for the ReLU, whose pass adds the two as it reads them."""
         cur = adjoints.get(name)
         if cur is None:
             adjoints[name] = upd
             return
+        if name in relu_out and name not in pending:
+            pending[name] = upd
+            return
+        if name in pending:
+            first = pending.pop(name)
+            adjoints.pop(name)
+            accumulate_now(name, cur, first)
+            cur = adjoints[name]
+        accumulate_now(name, cur, upd)
+
+    def accumulate_now(name: str, cur: _Rows, upd: _Rows) -> None:
         n = int((upd.A_u if upd.A_u is not None else upd.A_l).shape[1])
         both = shared(cur) and shared(upd)
         with _timed("dag_accumulate", 0.0, 4.0 * 3 * M * n * (1 if both else 2)):
@@ -447,30 +468,81 @@ def crown_backward_dag(
         b_l = b_u if both else add_rows(cur.b_l, upd.b_l, 1)
         adjoints[name] = _Rows(A_u, A_l, b_u, b_l)
 
+    pending: Dict[str, _Rows] = {}
+    # (a gradient pass and the influences read the coefficient that enters the relaxation)
+    relu_out = set() if save is not None or relu_influence is not None else {
+        op.outputs[0] for op in task.ops if op.op_type == "relu"}
+    readers: Dict[str, int] = {}
+    for op in task.ops:
+        for name in op.inputs:
+            readers[name] = readers.get(name, 0) + 1
+    maker = {op.outputs[0]: (i, op) for i, op in enumerate(task.ops)}
+    folded = set()   # the affine ops whose bias a ReLU's pass has summed
+
+    def bias_of(x: str):
+        """The biases of the affine ops whose coefficient is the relaxed one of the ReLU reading x:
+        x's own maker's or, through adds and reshapes, those of the values x is the sum of, where
+        nothing else reads them."""
+        if readers.get(x) != 1 or x == output_value or x not in maker:
+            return
+        i, op = maker[x]
+        if op.op_type in ("linear", "conv2d"):
+            if len(op.inputs) == 3:
+                yield i, op
+        elif op.op_type in ("add", "flatten", "reshape"):
+            for v in op.inputs:
+                if v in dynamic and _numel(trace.shapes[v]) == _numel(trace.shapes[x]):
+                    yield from bias_of(v)
+
+    def relu_bias(x: str) -> Optional[torch.Tensor]:
+        """Their sum as one value per element of x (kept across queries)."""
+        ops = list(bias_of(x))
+        folded.update(i for i, _op in ops)
+        if not ops:
+            return None
+        maps = [(params[op.inputs[2]], trace.shapes[op.outputs[0]] if op.op_type == "conv2d" else None)
+                for _i, op in ops]
+
+        def make():
+            flat = [b.detach().contiguous() if shape is None else _conv_bias_map(b.detach(), shape)
+                    for b, shape in maps]
+            return flat[0] if len(flat) == 1 else torch.stack(flat).sum(dim=0)
+
+        if len(maps) == 1 and maps[0][1] is None:
+            return make()
+        return derived("dag_bias:" + ":".join(str(shape) for _b, shape in maps), tuple(b for b, _s in maps), make)
+
     for op_index in range(len(task.ops) - 1, -1, -1):
         op = task.ops[op_index]
         out = op.outputs[0]
         st = adjoints.pop(out, None)
         if st is None:
             continue
+        two = pending.pop(out, None)
         if save is not None:
             save["ran"].add(op_index)
         t = op.op_type
         x = op.inputs[0]
         if t == "linear":
             W = params[op.inputs[1]].contiguous()
-            bias = params[op.inputs[2]].contiguous() if len(op.inputs) == 3 else None
+            keep_b = len(op.inputs) != 3 or op_index in folded   # the bias rows pass through
+            bias = None if keep_b else params[op.inputs[2]].contiguous()
             N, P = int(W.shape[0]), int(W.shape[1])
             one = shared(st)
             nA_u, nA_l = like(st, P, one)
-            nb_u, nb_l = like(_Rows(st.b_u, st.b_l, None, None), 1, one)
-            nb_u = None if nb_u is None else nb_u.reshape(M)
-            nb_l = None if nb_l is None else nb_l.reshape(M)
+            if keep_b:
+                nb_u, nb_l = st.b_u, st.b_l
+            else:
+                nb_u, nb_l = like(_Rows(st.b_u, st.b_l, None, None), 1, one)
+                nb_u = None if nb_u is None else nb_u.reshape(M)
+                nb_l = None if nb_l is None else nb_l.reshape(M)
             A_l_in = None if one else st.A_l
             nz = int(st.A_u is not None) + int(A_l_in is not None)
             with _timed("crown_linear", 2.0 * nz * M * N * P, 4.0 * nz * (M * N + N * P + M * P)):
-                rows = (_lib.ptr(bias), _lib.ptr(st.b_u), _lib.ptr(None if one else st.b_l), _lib.ptr(nA_u),
-                        _lib.ptr(None if one else nA_l), _lib.ptr(nb_u), _lib.ptr(None if one else nb_l), stream)
+                out_b = (None, None) if keep_b else (_lib.ptr(nb_u), _lib.ptr(None if one else nb_l))
+                rows = (_lib.ptr(bias), _lib.ptr(None if keep_b else st.b_u),
+                        _lib.ptr(None if one or keep_b else st.b_l), _lib.ptr(nA_u),
+                        _lib.ptr(None if one else nA_l), *out_b, stream)
                 if takes_parts(STORE, M, P, N, S, nz):
                     _lib.call("bf_crown_linear_parts", _lib.ptr(st.A_u), _lib.ptr(A_l_in), S * N, B, S, N,
                               _lib.ptr(weight_parts(params[op.inputs[1]], False)), P, *rows)
@@ -486,8 +558,10 @@ def crown_backward_dag(
             Co, Ho, Wo = out_shape
             Ci, Hi, Wi = in_shape
             n_out = Co * Ho * Wo
-            if len(op.inputs) == 3:
-                st, _ = rows_pass(st, n_out, kbias=_conv_bias_map(params[op.inputs[2]], out_shape),
+            if len(op.inputs) == 3 and op_index not in folded:
+                bias = params[op.inputs[2]]
+                st, _ = rows_pass(st, n_out, kbias=derived(f"conv_bias_map:{Ho}x{Wo}", (bias,),
+                                                           lambda b=bias: _conv_bias_map(b.detach(), out_shape)),
                                   name="conv_bias_rows")
             one = shared(st)
             y_u, y_l = like(st, Ci * Hi * Wi, one)
@@ -517,7 +591,8 @@ def crown_backward_dag(
                 relu_influence[x] = infl
             if save is not None:
                 save["relu_A"][op_index] = st.A_l      # the coefficient before the relaxation
-            new, _ = rows_pass(st, n, pre=pre, alpha=alpha, alpha_ld=alpha_ld, add=add, add_ld=add_ld)
+            new, _ = rows_pass(st, n, pre=pre, alpha=alpha, alpha_ld=alpha_ld, add=add, add_ld=add_ld,
+                               kbias=relu_bias(x), two=two)
             accumulate(x, new)
         elif t in ("flatten", "reshape"):
             accumulate(x, st)          # the rows are already laid out in the input's element order

@@ -570,6 +570,17 @@ ibp_batched_linear_kernel(const float* __restrict__ lo, const float* __restrict_
   }
 }
 
+// Optional second coefficient of the relaxation pass and its bias rows, added to the first as the
+// rows are read: the sum of a DAG value's two adjoints (crown_ibp.py:892-909) without a pass of its
+// own.  The launches are short of work, not of bandwidth: a residual query of 64 x 10 rows (4 blocks of
+// 512, both bounds) took 449 us with the sums as launches (16 of about 4.3 us) and the affine ops' bias
+// sums as passes (8 of about 5.6 us), 365 us with both inside the relaxation pass; a residual conv
+// net of 16 x 10 rows 431 and 332 us.
+struct RowAddend {
+  const float* A[2];   // [M, K] of the upper and the lower bound, or null
+  const float* b[2];   // [M]
+};
+
 // ---------------------------------------------------------------------------
 // Where a relaxation pass reads the slopes/intercepts {alpha_u, beta_u, alpha_l,
 // beta_l} of (domain d, neuron k): a table of bf_relu_relax_table, or computed in
@@ -629,7 +640,7 @@ relu_relax_rows_kernel(const float* __restrict__ Au, const float* __restrict__ A
                        const float* __restrict__ kbias, const float* __restrict__ cvec,
                        const float* __restrict__ bu_in, const float* __restrict__ bl_in, float* __restrict__ Au_out,
                        float* __restrict__ Al_out, float* __restrict__ bu_out, float* __restrict__ bl_out,
-                       float* __restrict__ cu_out, float* __restrict__ cl_out) {
+                       float* __restrict__ cu_out, float* __restrict__ cl_out, RowAddend two) {
   const int lane = threadIdx.x & 63;
   const int64_t m = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (m >= M) return;
@@ -641,6 +652,7 @@ relu_relax_rows_kernel(const float* __restrict__ Au, const float* __restrict__ A
     const float4 r = relax.at(d, K, k);
     if (Au) {
       float v = Au[a_row + k];
+      if (two.A[0]) v = v + two.A[0][m * K + k];
       bool nn = v >= 0.f;
       float o = v * (nn ? r.x : r.z);
       su += v * (nn ? r.y : r.w);
@@ -650,6 +662,7 @@ relu_relax_rows_kernel(const float* __restrict__ Au, const float* __restrict__ A
     }
     if (Al) {
       float v = Al[a_row + k];
+      if (two.A[1]) v = v + two.A[1][m * K + k];
       bool nn = v >= 0.f;
       float o = v * (nn ? r.z : r.x);
       sl += v * (nn ? r.w : r.y);
@@ -668,8 +681,8 @@ relu_relax_rows_kernel(const float* __restrict__ Au, const float* __restrict__ A
     cl += __shfl_xor(cl, off, 64);
   }
   if (lane == 0) {
-    if (bu_out) bu_out[m] = ((bu_in ? bu_in[m] : 0.f) + su) + ku;
-    if (bl_out) bl_out[m] = ((bl_in ? bl_in[m] : 0.f) + sl) + kl;
+    if (bu_out) bu_out[m] = ((bu_in ? bu_in[m] : 0.f) + (two.b[0] ? two.b[0][m] : 0.f) + su) + ku;
+    if (bl_out) bl_out[m] = ((bl_in ? bl_in[m] : 0.f) + (two.b[1] ? two.b[1][m] : 0.f) + sl) + kl;
     if (cu_out) cu_out[m] = cu;
     if (cl_out) cl_out[m] = cl;
   }
@@ -763,6 +776,10 @@ relu_relax_domain_kernel(const float* __restrict__ Au, const float* __restrict__
 // bound and four table entries in flight per thread.  Needs K % 4 == 0 and
 // 16-byte aligned rows.  Row sums: per-thread partials in k order, then a fixed
 // tree (wave shuffles, then the workgroup's waves through LDS when TPR > 64).
+__device__ __forceinline__ float4 add4(float4 a, float4 b) {
+  return make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w);
+}
+
 template <int TPR>
 __global__ void __launch_bounds__(256)
 relu_relax_rows4_kernel(const float* __restrict__ Au, const float* __restrict__ Al, int64_t a_dstride, int64_t M,
@@ -771,7 +788,7 @@ relu_relax_rows4_kernel(const float* __restrict__ Au, const float* __restrict__ 
                         const float* __restrict__ kbias, const float* __restrict__ cvec,
                         const float* __restrict__ bu_in, const float* __restrict__ bl_in, float* __restrict__ Au_out,
                         float* __restrict__ Al_out, float* __restrict__ bu_out, float* __restrict__ bl_out,
-                        float* __restrict__ cu_out, float* __restrict__ cl_out) {
+                        float* __restrict__ cu_out, float* __restrict__ cl_out, RowAddend two) {
   constexpr int RPB = 256 / TPR;   // rows per workgroup
   constexpr int WPR = TPR / 64;    // waves per row
   __shared__ float red[6][256 / 64];
@@ -793,7 +810,8 @@ relu_relax_rows4_kernel(const float* __restrict__ Au, const float* __restrict__ 
       // one load serves both bounds when they share the coefficient (the first region of a C = I query)
       const float4 vu4 = Au ? *reinterpret_cast<const float4*>(Au + a_row + k) : make_float4(0.f, 0.f, 0.f, 0.f);
       if (Au) {
-        const float4 v4 = vu4;
+        float4 v4 = vu4;
+        if (two.A[0]) v4 = add4(v4, *reinterpret_cast<const float4*>(two.A[0] + m * K + k));
         const float v[4] = {v4.x, v4.y, v4.z, v4.w};
         float o[4];
 #pragma unroll
@@ -807,7 +825,8 @@ relu_relax_rows4_kernel(const float* __restrict__ Au, const float* __restrict__ 
         if (Au_out) *reinterpret_cast<float4*>(Au_out + m * K + k) = make_float4(o[0], o[1], o[2], o[3]);
       }
       if (Al) {
-        const float4 v4 = Al == Au ? vu4 : *reinterpret_cast<const float4*>(Al + a_row + k);
+        float4 v4 = Al == Au ? vu4 : *reinterpret_cast<const float4*>(Al + a_row + k);
+        if (two.A[1]) v4 = add4(v4, *reinterpret_cast<const float4*>(two.A[1] + m * K + k));
         const float v[4] = {v4.x, v4.y, v4.z, v4.w};
         const float4 ad =
             add_l ? *reinterpret_cast<const float4*>(add_l + d * add_ld + k) : make_float4(0.f, 0.f, 0.f, 0.f);
@@ -846,8 +865,8 @@ relu_relax_rows4_kernel(const float* __restrict__ Au, const float* __restrict__ 
       }
   }
   if (live && t == 0) {
-    if (bu_out) bu_out[m] = ((bu_in ? bu_in[m] : 0.f) + s[0]) + s[2];
-    if (bl_out) bl_out[m] = ((bl_in ? bl_in[m] : 0.f) + s[1]) + s[3];
+    if (bu_out) bu_out[m] = ((bu_in ? bu_in[m] : 0.f) + (two.b[0] ? two.b[0][m] : 0.f) + s[0]) + s[2];
+    if (bl_out) bl_out[m] = ((bl_in ? bl_in[m] : 0.f) + (two.b[1] ? two.b[1][m] : 0.f) + s[1]) + s[3];
     if (cu_out) cu_out[m] = s[4];
     if (cl_out) cl_out[m] = s[5];
   }
@@ -1542,7 +1561,8 @@ int bf_relu_relax_table_multi(int count, const float* const* pre_lo, const float
 static int relax_pass(const float* A_u, const float* A_l, int64_t a_dstride, int64_t D, int64_t S, int64_t K,
                       const RelaxSrc& src, const float* add_l, int64_t add_ld, const float* kbias, const float* cvec,
                       const float* b_u_in, const float* b_l_in, float* A_u_out, float* A_l_out, float* b_u_out,
-                      float* b_l_out, float* c_u_out, float* c_l_out, hipStream_t stream, bool sums_only);
+                      float* b_l_out, float* c_u_out, float* c_l_out, hipStream_t stream, bool sums_only,
+                      const RowAddend& two = RowAddend{});
 
 int bf_crown_relu_linear_fwd(const float* A_u, const float* A_l, int64_t a_dstride, int64_t D, int64_t S, int64_t N,
                              const float* relax, const float* add_l, int64_t add_ld, const float* W, int64_t P,
@@ -1957,7 +1977,8 @@ int64_t bf_crown_linear_concretize_workspace(int64_t D, int64_t S, int64_t I) {
 static int relax_pass(const float* A_u, const float* A_l, int64_t a_dstride, int64_t D, int64_t S, int64_t K,
                       const RelaxSrc& src, const float* add_l, int64_t add_ld, const float* kbias, const float* cvec,
                       const float* b_u_in, const float* b_l_in, float* A_u_out, float* A_l_out, float* b_u_out,
-                      float* b_l_out, float* c_u_out, float* c_l_out, hipStream_t stream, bool sums_only) {
+                      float* b_l_out, float* c_u_out, float* c_l_out, hipStream_t stream, bool sums_only,
+                      const RowAddend& two) {
   BF_REQUIRE(D >= 0 && S >= 0 && K > 0, "bf_crown_relu_relax: bad sizes");
   const int64_t M = D * S;
   if (M == 0) return BF_OK;
@@ -1970,8 +1991,9 @@ static int relax_pass(const float* A_u, const float* A_l, int64_t a_dstride, int
   const bool vec = (K % 4 == 0) && (a_dstride % 4 == 0) && al16(A_u) && al16(A_l) && al16(A_u_out) &&
                    al16(A_l_out) && al16(kbias) &&
                    al16(cvec) && al16(add_l) && (add_l == nullptr || add_ld % 4 == 0) && al16(src.lo) &&
-                   al16(src.hi) && al16(src.alpha) && (src.alpha_ld % 4 == 0);
-  if (vec && K <= 512 && (a_dstride == 0 ? S >= 16 : (S >= 8 && M >= 8192))) {
+                   al16(src.hi) && al16(src.alpha) && (src.alpha_ld % 4 == 0) && al16(two.A[0]) && al16(two.A[1]);
+  const bool one = !two.A[0] && !two.A[1];   // (the kernels that keep a domain's operands take no second coefficient)
+  if (one && vec && K <= 512 && (a_dstride == 0 ? S >= 16 : (S >= 8 && M >= 8192))) {
     // a shared coefficient: 16 rows of one domain per workgroup (4 per wave), the
     // domain's operands held in registers across them (C2's 500 x 500 shape: 8, 16 and
     // 64 rows per workgroup measured 150, 129 and 141 us, the per-row kernel 156 us).
@@ -1994,14 +2016,14 @@ static int relax_pass(const float* A_u, const float* A_l, int64_t a_dstride, int
   } else if (vec && K >= 1024) {
     hipLaunchKernelGGL(relu_relax_rows4_kernel<256>, dim3((unsigned)M), dim3(256), 0, stream, A_u, A_l, a_dstride, M, S,
                        K, src, add_l, add_ld, kbias, cvec, b_u_in, b_l_in, A_u_out, A_l_out, b_u_out, b_l_out, c_u_out,
-                       c_l_out);
+                       c_l_out, two);
     BF_LAUNCH_CHECK("relu_relax_rows4_kernel<256>");
   } else if (vec) {
     hipLaunchKernelGGL(relu_relax_rows4_kernel<64>, dim3((unsigned)ceil_div(M, 4)), dim3(256), 0, stream, A_u, A_l,
                        a_dstride, M, S, K, src, add_l, add_ld, kbias, cvec, b_u_in, b_l_in, A_u_out, A_l_out, b_u_out,
-                       b_l_out, c_u_out, c_l_out);
+                       b_l_out, c_u_out, c_l_out, two);
     BF_LAUNCH_CHECK("relu_relax_rows4_kernel<64>");
-  } else if (!vec && K <= 512 && S >= 16 && M >= 1024) {
+  } else if (one && !vec && K <= 512 && S >= 16 && M >= 1024) {
     // (fewer rows: 16 rows of 77 in 100 domains 9.2 / 9.0 us, row / domain kernel)
     const int rpw = 16;
     const int64_t chunks = ceil_div(S, rpw);
@@ -2019,7 +2041,7 @@ static int relax_pass(const float* A_u, const float* A_l, int64_t a_dstride, int
   } else {
     hipLaunchKernelGGL(relu_relax_rows_kernel, dim3((unsigned)ceil_div(M, 4)), dim3(256), 0, stream, A_u, A_l,
                        a_dstride, M, S, K, src, add_l, add_ld, kbias, cvec, b_u_in, b_l_in, A_u_out, A_l_out, b_u_out,
-                       b_l_out, c_u_out, c_l_out);
+                       b_l_out, c_u_out, c_l_out, two);
     BF_LAUNCH_CHECK("relu_relax_rows_kernel");
   }
   return BF_OK;
@@ -2044,6 +2066,20 @@ int bf_crown_relu_relax_lu(const float* A_u, const float* A_l, int64_t a_dstride
   const RelaxSrc src{nullptr, pre_lo, pre_hi, alpha, alpha_ld};
   return relax_pass(A_u, A_l, a_dstride, D, S, K, src, add_l, add_ld, kbias, cvec, b_u_in, b_l_in, A_u_out, A_l_out,
                     b_u_out, b_l_out, c_u_out, c_l_out, stream, false);
+}
+
+int bf_crown_relu_relax_sum_lu(const float* A_u, const float* A_l, const float* A2_u, const float* A2_l, int64_t D,
+                               int64_t S, int64_t K, const float* pre_lo, const float* pre_hi, const float* alpha,
+                               int64_t alpha_ld, const float* add_l, int64_t add_ld, const float* kbias,
+                               const float* b_u_in, const float* b_l_in, const float* b2_u, const float* b2_l,
+                               float* A_u_out, float* A_l_out, float* b_u_out, float* b_l_out, hipStream_t stream) {
+  BF_REQUIRE(alpha == nullptr || alpha_ld == 0 || alpha_ld >= K, "bf_crown_relu_relax_sum_lu: bad alpha_ld");
+  BF_REQUIRE((A_u == nullptr) == (A2_u == nullptr) && (A_l == nullptr) == (A2_l == nullptr),
+             "bf_crown_relu_relax_sum_lu: a bound's two coefficients go together");
+  const RelaxSrc src{nullptr, pre_lo, pre_hi, alpha, alpha_ld};
+  const RowAddend two{{A2_u, A2_l}, {b2_u, b2_l}};
+  return relax_pass(A_u, A_l, S * K, D, S, K, src, add_l, add_ld, kbias, nullptr, b_u_in, b_l_in, A_u_out, A_l_out,
+                    b_u_out, b_l_out, nullptr, nullptr, stream, false, two);
 }
 
 int bf_concretize_dense(const float* A, int64_t D, int64_t S, int64_t I, const float* center, const float* rad,

@@ -430,6 +430,14 @@ int64_t bf_gemm_rank1_workspace(int64_t M, int64_t N, int64_t K);
 
 /* ---- kernel #4: concretization -------------------------------------------- */
 
+/* bf_crown_relu_relax_lu (per-domain rows) of the sum of two coefficients and of their bias rows, added
+ * as they are read: a DAG value's two adjoints (runtime/crown_ibp.py:892-909) through its ReLU. */
+int bf_crown_relu_relax_sum_lu(const float* A_u, const float* A_l, const float* A2_u, const float* A2_l, int64_t D,
+                               int64_t S, int64_t K, const float* pre_lo, const float* pre_hi, const float* alpha,
+                               int64_t alpha_ld, const float* add_l, int64_t add_ld, const float* kbias,
+                               const float* b_u_in, const float* b_l_in, const float* b2_u, const float* b2_l,
+                               float* A_u_out, float* A_l_out, float* b_u_out, float* b_l_out, hipStream_t stream);
+
 /* Dense coefficient rows A [M, I] against the input set:
  * out = A . center[d] -/+ eps * sum |A| (Linf, rad NULL) or -/+ sum |A| * rad[d] (box), + b;
  * norm_p 2 / 1 (rad NULL): eps times the row's L2 norm / max |A| (L2 / L1 ball).

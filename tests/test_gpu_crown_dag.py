@@ -152,6 +152,34 @@ def test_dag_crown_constant_add_operand():
     _check(w, dev, "constant add")
 
 
+def test_dag_crown_fan_out_of_four_and_unshared_biases():
+    """A ReLU read by four ops (its adjoints beyond two are summed ahead of it), an affine value read by a
+    ReLU and by an add (its bias is its own pass's), and a sum of two affine values behind a reshape
+    (their biases join in the ReLU's pass)."""
+    from boundflow_amd.ir import BFTaskModule, BoundTask, TaskKind, TaskOp
+    from boundflow_amd.spec import InputSpec
+    dev = device()
+    announce("DAG CROWN with a fan-out of four")
+    g = torch.Generator().manual_seed(21)
+    B, n = 5, 18
+    params = {f"W{i}": torch.randn(n, 12 if i == 0 else n, generator=g) * 0.2 for i in range(5)}
+    params.update({f"b{i}": torch.randn(n, generator=g) for i in range(5)}, Wo=torch.randn(10, n, generator=g) * 0.2)
+    lin = lambda i, x: TaskOp("linear", f"lin{i}", [x, f"W{i}", f"b{i}"], [f"h{i}"])   # noqa: E731
+    ops = [lin(0, "input"), TaskOp("relu", "relu0", ["h0"], ["r"]), lin(1, "r"), lin(2, "r"), lin(3, "r"),
+           TaskOp("add", "add0", ["h1", "h2"], ["s"]), TaskOp("flatten", "flat", ["s"], ["f"]),
+           TaskOp("relu", "relu1", ["f"], ["r1"]), TaskOp("relu", "relu3", ["h3"], ["r3"]),
+           TaskOp("add", "add1", ["r", "h3"], ["s1"]), TaskOp("add", "add2", ["s1", "r3"], ["s2"]),
+           TaskOp("add", "add3", ["s2", "r1"], ["s3"]), lin(4, "s3"), TaskOp("relu", "relu4", ["h4"], ["r4"]),
+           TaskOp("linear", "lin5", ["r4", "Wo"], ["out"])]
+    task = BoundTask(task_id="t0", kind=TaskKind.INTERVAL_IBP, ops=ops, input_values=["input"],
+                     output_values=["out"])
+    module = BFTaskModule(tasks=[task], entry_task_id="t0", bindings={"params": params})
+    labels = torch.tensor([1, 4, 7, 0, 9])
+    w = wl.Workload("fan_out", module, InputSpec.linf(value_name="input", center=torch.rand(B, 12, generator=g), eps=0.05),
+                    wl.margin_spec(labels), labels)
+    _check(w, dev, "fan-out")
+
+
 def test_dag_crown_rejects_broadcast_add():
     from boundflow_amd.ir import BFTaskModule, BoundTask, TaskKind, TaskOp
     from boundflow_amd.spec import InputSpec

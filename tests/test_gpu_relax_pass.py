@@ -59,3 +59,37 @@ def test_many_rows_per_domain_match_fp64(D, S, K, shared, sides, extras):
         for got, want, size in sums:
             err = (got.cpu().double() - want).abs()
             assert bool((err <= (K + 8) * 2.0 ** -23 * size + 1e-30).all()), float((err / size).max())
+
+
+@pytest.mark.parametrize("D,S,K,sides", [(1, 1, 1, "ul"), (3, 5, 20, "ul"), (2, 7, 255, "l"), (4, 9, 256, "ul"),
+                                         (2, 3, 516, "u"), (1030, 9, 64, "ul"), (70, 16, 63, "ul")])
+@pytest.mark.parametrize("one", [True, False])
+def test_sum_of_two_coefficients_matches_the_summed_one(D, S, K, sides, one):
+    """The pass that adds a second coefficient and its bias rows as it reads them: the coefficients bit
+    for bit those of the pass over the sum, the bias rows within the rounding of their own sums; one
+    tensor for both bounds and one each."""
+    dev = device()
+    M = D * S
+    announce(f"relaxation of a sum D={D} S={S} K={K} sides={sides} one={one}")
+    g = torch.Generator().manual_seed(D + 3 * S + 7 * K + one)
+    r = lambda *shape: torch.randn(*shape, generator=g).to(dev)   # noqa: E731
+    A, A2, b, b2 = ({q: r(M, *cols) for q in sides} for cols in ((K,), (K,), (), ()))
+    if one:
+        A, A2 = ({q: m[sides[0]] for q in sides} for m in (A, A2))
+    lo, kbias, alpha = r(D, K), r(K), torch.rand(D, K, generator=g).to(dev)
+    hi = lo + torch.rand(D, K, generator=g).to(dev) * 2
+    out, want = ({q: torch.empty(M, K, device=dev) for q in sides} for _ in range(2))
+    bo, bw = ({q: torch.empty(M, device=dev) for q in sides} for _ in range(2))
+    p = lambda m, q: _lib.ptr(m.get(q))   # noqa: E731
+    tail = (_lib.ptr(lo), _lib.ptr(hi), _lib.ptr(alpha), K, None, 0, _lib.ptr(kbias))
+    _lib.call("bf_crown_relu_relax_sum_lu", p(A, "u"), p(A, "l"), p(A2, "u"), p(A2, "l"), D, S, K, *tail, p(b, "u"),
+              p(b, "l"), p(b2, "u"), p(b2, "l"), p(out, "u"), p(out, "l"), p(bo, "u"), p(bo, "l"), _lib.stream_handle())
+    added, b_added = {q: A[q] + A2[q] for q in sides}, {q: b[q] + b2[q] for q in sides}
+    _lib.call("bf_crown_relu_relax_lu", p(added, "u"), p(added, "l"), S * K, D, S, K, *tail, None, p(b_added, "u"),
+              p(b_added, "l"), p(want, "u"), p(want, "l"), p(bw, "u"), p(bw, "l"), None, None, _lib.stream_handle())
+    torch.cuda.synchronize()
+    for q in sides:
+        assert torch.equal(out[q], want[q])
+        # |beta| <= |A'| |lower|-like terms: both sides sum the same addends, in another order at most
+        size = b[q].abs() + b2[q].abs() + (added[q].abs() * (kbias.abs() + 3 * (1 + lo.abs().repeat_interleave(S, 0)))).sum(1)
+        assert bool(((bo[q] - bw[q]).abs() <= 2 * (K + 8) * 2.0 ** -24 * size).all())
