@@ -141,16 +141,24 @@ def load() -> ctypes.CDLL:
     return lib
 
 
-class DevicePtr(ctypes.c_void_p):
+class DevicePtr:
     """A tensor's address that keeps the tensor alive.  Arguments such as
     ``ptr(x.contiguous())`` may be temporaries; held here, they survive until
     the call that receives them has enqueued its kernels, so the caching
     allocator cannot hand their memory to a later argument of the same call
-    (later reuse is ordered after the launch on the stream)."""
+    (later reuse is ordered after the launch on the stream).  A query makes hundreds:
+    a plain object ctypes converts by its ``_as_parameter_`` takes half the time of a
+    c_void_p subclass (0.28 against 0.52 us)."""
+
+    __slots__ = ("_as_parameter_", "tensor")
 
     def __init__(self, t: torch.Tensor):
-        super().__init__(t.data_ptr())
+        self._as_parameter_ = t.data_ptr()
         self.tensor = t
+
+    @property
+    def value(self) -> Optional[int]:
+        return self._as_parameter_ or None
 
 
 def ptr(t: Optional[torch.Tensor]):
@@ -190,9 +198,15 @@ def f32_array(values) -> HostArray:
     return HostArray(ctypes.c_float, [float(v) for v in values])
 
 
+# the current stream's handle of a device index, without a Stream object around it
+current_raw_stream = torch._C._cuda_getCurrentRawStream if hasattr(torch._C, "_cuda_getCurrentRawStream") else (
+    lambda index: torch.cuda.current_stream(index).cuda_stream)
+
+
 def stream_handle(stream: Optional[torch.cuda.Stream] = None):
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return ctypes.c_void_p(s.cuda_stream)
+    if stream is not None:
+        return ctypes.c_void_p(stream.cuda_stream)
+    return ctypes.c_void_p(current_raw_stream(torch.cuda.current_device()))
 
 
 def call(name: str, *args) -> int:

@@ -30,6 +30,7 @@ behaviour.
 from __future__ import annotations
 
 import contextlib
+import functools
 import threading
 from collections import OrderedDict
 from dataclasses import dataclass, field
@@ -84,7 +85,7 @@ def _kept(tag: str, sources: Tuple[torch.Tensor, ...]) -> Optional[torch.Tensor]
     if scope is None:
         _DERIVED.move_to_end(key)
         out, stream, event = hit[2]
-        if event is not None and torch.cuda.current_stream(out.device) != stream:
+        if event is not None and _lib.current_raw_stream(out.device.index) != stream.cuda_stream:
             torch.cuda.current_stream(out.device).wait_event(event)
         return out
     return hit[2][0]
@@ -222,6 +223,11 @@ def takes_parts(form: int, M: int, N: int, K: int, S: int, nz: int) -> bool:
     packed weight parts: the library's rule on the form and the shape (``nz`` bounds)."""
     if K < 16 or M < 256:   # (most small queries end here, without a call into the library)
         return False
+    return _parts_rule(M, N, K, S, nz, form)
+
+
+@functools.lru_cache(maxsize=4096)
+def _parts_rule(M: int, N: int, K: int, S: int, nz: int, form: int) -> bool:
     return _lib.load().bf_gemm_parts_config(M, N, K, S, nz, form) != 0
 
 
@@ -255,6 +261,15 @@ class Chain:
         """Logical (per-example) shape of every ReLU input, in op order."""
         out = {layer.out_name: tuple(layer.out_shape) for layer in self.layers}
         return {name: out[name] for name in self.relu_names}
+
+    def until(self, output_value: str) -> "Chain":
+        """The chain that ends at the affine layer producing ``output_value``, what ``parse_chain``
+        makes of it."""
+        last = [layer.out_name for layer in self.layers].index(output_value)
+        layers = self.layers[:last + 1]
+        before = {layer.out_name for layer in layers[:-1]}
+        return Chain(layers=layers, relu_names=[r for r in self.relu_names if r in before],
+                     output_value=output_value)
 
 
 def _pair(v) -> Tuple[int, int]:
@@ -580,7 +595,15 @@ def crown_backward(
     stride = a_dstride
     tables: Dict[int, torch.Tensor] = {}
 
+    read: Dict[int, tuple] = {}
+
     def relax_params(k: int):
+        """``relax_params_of(k)``, read once (the relaxation before a region asks for it too)."""
+        if k not in read:
+            read[k] = relax_params_of(k)
+        return read[k]
+
+    def relax_params_of(k: int):
         """(alpha, alpha_ld, add, add_ld, pre_lo, pre_hi, N) of the ReLU after layer k."""
         layer = layers[k]
         relax_name = layer.out_name if k < len(layers) - 1 else None
@@ -1082,14 +1105,14 @@ def run_crown_all_intermediate(module: BFTaskModule, input_spec, *, linear_spec_
     stream = _lib.stream_handle()
     B = int(spec.center.shape[0])
     for name in names[1:]:
-        chain = parse_chain(module, spec, name)
+        chain = chain_full.until(name)
         b = crown_backward(module, spec, trace, chain=chain, linear_spec_C=None)
         cur = trace.relu_pre[name]
         n = int(cur.lower[0].numel())
         lo = cur.lower.reshape(B, n)
         hi = cur.upper.reshape(B, n)
-        flag = torch.zeros(B, dtype=torch.int32, device=spec.center.device)
+        # (no caller asks whether a refinement emptied a box: no flags)
         _lib.call("bf_interval_clip", _lib.ptr(lo), _lib.ptr(hi), _lib.ptr(b.lower.contiguous()),
-                  _lib.ptr(b.upper.contiguous()), None, 0, B, n, _lib.ptr(flag), stream)
+                  _lib.ptr(b.upper.contiguous()), None, 0, B, n, None, stream)
     final = crown_backward(module, spec, trace, chain=chain_full, linear_spec_C=linear_spec_C)
     return final, trace.relu_pre

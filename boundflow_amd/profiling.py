@@ -10,7 +10,7 @@ until ``summary()`` is called.
 from __future__ import annotations
 
 from collections import defaultdict
-from contextlib import contextmanager
+from contextlib import contextmanager, nullcontext
 from typing import Dict, List, Optional, Tuple
 
 import torch
@@ -64,17 +64,20 @@ def timing(timer: LaunchTimer):
 _pending: Optional[list] = None   # [name, flops, bytes, start event, end event] of the bracketed launch
 
 
-@contextmanager
+_OFF = nullcontext()
+
+
 def launch(name: str, flops: float, nbytes: float):
     """Time the first library call inside the block (no-op unless a
     LaunchTimer is active).  The events are recorded by the call itself,
     immediately around the foreign function, so host work that prepares the
     arguments -- during which a launch-bound device idles -- is not counted."""
+    return _OFF if _active is None else _launch(_active, name, flops, nbytes)
+
+
+@contextmanager
+def _launch(t: LaunchTimer, name: str, flops: float, nbytes: float):
     global _pending
-    t = _active
-    if t is None:
-        yield
-        return
     _pending = [name, float(flops), float(nbytes), None, None]
     try:
         yield
