@@ -230,7 +230,8 @@ struct GatherArgs {
   int Kc, Kc4, npad, nblk, nclasses, ntasks;
   FastDiv f_kstride, f_npad, f_T, f_nB, f_sw, f_KHKW, f_KW, f_HpWp, f_Wp;   // staging index divisions
   FastDiv f_HWm, f_Wm;                    // channel-last staging: divisions by Hm*Wm and Wm
-  FastDiv f_Kc4;                          // MODE_F weight staging in source order: division by Kc4
+  FastDiv f_kq;                           // conv2d weight staging: division by Kc4 / 16
+  int w_vec;                              // conv2d weights: 16-byte rows (Kc % 4 == 0, W aligned)
   const float* wpack;                     // channel-last: weights already in LDS order (or null)
   // MODE_F interval input (IBP): 0 X[z] as given; IVL_BOX X[0] = lo, ivl_hi = hi, operand z = 0
   // the center (l + u) / 2, z = 1 the radius (u - l) / 2 (IVL_RELU: of max(., 0)); IVL_BALL
@@ -252,7 +253,7 @@ static void gather_fdivs(GatherArgs& g) {
   g.f_KW = make_fdiv(g.KW);
   g.f_HpWp = make_fdiv(g.Hp * g.Wp);
   g.f_Wp = make_fdiv(g.Wp);
-  g.f_Kc4 = make_fdiv(g.Kc4 > 0 ? g.Kc4 : 1);
+  g.f_kq = make_fdiv(g.Kc4 >= 16 ? g.Kc4 / 16 : 1);
 }
 
 // LDS layout of the gather-GEMM operands.  The weights of class c, output channel n
@@ -272,10 +273,65 @@ __device__ __forceinline__ int koff_index(const GatherArgs& g, int k) {
   return (j * (g.Kc4 >> 4) + (s >> 2)) * 4 + (s & 3);
 }
 
+// Weights of conv2d channels ch0 .. ch0 + 16 nbl - 1 into the LDS order of ws_index (nbl channel
+// blocks), zero-padded in k and in channels: a thread takes 16 consecutive k of one channel
+// (k = 16 sq + 4 e + j), read as four 16-byte loads where the rows allow them, and transposes
+// them in registers into the four chunks (j; e = 0 .. 3) of its step quad.  The lanes of a chunk
+// are 16 consecutive channels, so the stores have no bank conflict; the scatter of single k values
+// it replaces met 16 of 64 lanes on one bank and worked out an index per value.  One row per
+// workgroup (the bound pass of 128 inputs, 16 x 18 x 18 -> 32 x 8 x 8): the interval conv went from 15.3 to
+// 12.7 us with this and with the map's loads issued ahead of it.
+__device__ __forceinline__ void stage_conv_weights(const GatherArgs& g, float* Ws, int ch0, int nbl, bool absw,
+                                                   int tid) {
+  const int kq = g.Kc4 >> 4;
+  for (int u = tid; u < nbl * kq * 16; u += GTM) {
+    const int col = u & 15, q = u >> 4;
+    const int cb = fdivq(q, g.f_kq), sq = q - cb * kq;
+    const int ch = ch0 + 16 * cb + col, k0 = 16 * sq;
+    const float* __restrict__ src = g.W + (int64_t)(ch < g.nch ? ch : 0) * g.Kc + k0;
+    float x[16];
+    if (g.w_vec) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const bool ok = ch < g.nch && k0 + 4 * e < g.Kc;   // (Kc % 4 == 0: a chunk is inside or outside)
+        const float4 v = *reinterpret_cast<const float4*>(ok ? src + 4 * e : g.W);
+        x[4 * e] = ok ? v.x : 0.f;
+        x[4 * e + 1] = ok ? v.y : 0.f;
+        x[4 * e + 2] = ok ? v.z : 0.f;
+        x[4 * e + 3] = ok ? v.w : 0.f;
+      }
+    } else {
+#pragma unroll
+      for (int k = 0; k < 16; ++k) {
+        const bool ok = ch < g.nch && k0 + k < g.Kc;
+        const float v = *(ok ? src + k : g.W);
+        x[k] = ok ? v : 0.f;
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      float4 v = make_float4(x[j], x[4 + j], x[8 + j], x[12 + j]);
+      if (absw) v = make_float4(fabsf(v.x), fabsf(v.y), fabsf(v.z), fabsf(v.w));
+      *reinterpret_cast<float4*>(Ws + ((((cb * 4 + j) * kq + sq) * 16 + col) << 2)) = v;
+    }
+  }
+}
+
+// Elements of a row's map a thread of the forward gather-GEMM stages at a time: the first batch of a
+// row is loaded ahead of the weights (the first row) or of the products of the row before, so
+// its way from memory runs beside them, and the maps of the networks at hand (16 x 18 x 18,
+// 3 x 34 x 34) are one batch.  The interval conv of 2048 inputs, 16 x 18 x 18 -> 32 x 8 x 8: 142.6 -> 104.2 us,
+// 3 x 34 x 34 -> 16 x 16 x 16 (8 at a time): 76.0 -> 62.3 us (12 at a time 70.8: fewer workgroups fit the
+// registers; so does a branch around the elements past the map, at 132 registers: 142 and 94 us).
+// The transposed direction keeps its 8 loads behind the weights (53 registers; 20.7 us over a residual
+// net's 3 x 3 layers, 26.3 us loaded ahead).
+constexpr int MAP_U = 12;
+
 template <int MODE>
 __global__ void __launch_bounds__(GTM)
 conv_mfma_kernel(GatherArgs g) {
   extern __shared__ __attribute__((aligned(16))) float smem[];
+  constexpr int U = MODE == MODE_F ? MAP_U : 8;
   float* Ws = smem;                                              // [nclasses][Kc4][npad]
   int* koff = reinterpret_cast<int*>(Ws + (size_t)g.nclasses * g.Kc4 * g.npad);   // [Kc4]
   float* As = reinterpret_cast<float*>(koff + g.Kc4);            // [Cm][Hp][Wp]
@@ -290,53 +346,90 @@ conv_mfma_kernel(GatherArgs g) {
   float* __restrict__ nrm = g.nrm[z];
   const int kstride = g.Kc4 * g.npad;
 
-  // weights of every class, zero-padded in k (to Kc4) and in channels (to npad);
-  // eight loads per thread in flight, from clamped addresses, before the stores.
-  // MODE_F (one class) walks them in the source order, k fastest, so a wave's loads
-  // are consecutive floats of one output channel's row (W[n * Kc + k]), and scatters
-  // them into the LDS order.
-  const int wtotal = g.nclasses * kstride;
-  auto w_coords = [&](int idx, int& c, int& k, int& n) {
-    if (MODE == MODE_F) {
-      c = 0;
-      n = fdivq(idx, g.f_Kc4);
-      k = idx - n * g.Kc4;
-    } else {
+  const int nin = g.Cm * g.Hm * g.Wm;
+  const int64_t nout = (int64_t)g.nch * g.HWout;
+  const int map = g.Cm * g.Hp * g.Wp;
+  // interval input: the operand is made from the bounds as the map is staged (the
+  // arithmetic of ibp_center_radius_kernel), uniform over the launch
+  const int ivl = MODE == MODE_F ? g.ivl : 0;
+  // elements base + u GTM + tid of row r's padded map; bit u of the result: inside the map
+  auto map_load = [&](int64_t r, int base, float (&xa)[U], float (&xb)[U]) {
+    const float* __restrict__ xr = X + (r / g.in_div) * nin;
+    const float* __restrict__ hr_row = (ivl & IVL_BOX) ? g.ivl_hi + (r / g.in_div) * nin : nullptr;
+    uint32_t in = 0;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int idx = base + u * GTM + tid;
+      const int c = fdivq(idx, g.f_HpWp), rem = idx - c * g.Hp * g.Wp;
+      const int hr = fdivq(rem, g.f_Wp);
+      const int hm = hr - g.pad_h, wm = (rem - hr * g.Wp) - g.pad_w;
+      const bool ok = idx < map && hm >= 0 && hm < g.Hm && wm >= 0 && wm < g.Wm;
+      const int src = ok ? (c * g.Hm + hm) * g.Wm + wm : 0;
+      xa[u] = xr[src];
+      if (MODE == MODE_F && (ivl & IVL_BOX)) xb[u] = hr_row[src];
+      in |= ok ? 1u << u : 0u;
+    }
+    return in;
+  };
+  auto map_store = [&](int base, uint32_t in, const float (&xa)[U], const float (&xb)[U]) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int idx = base + u * GTM + tid;
+      float x = xa[u];
+      if (ivl & IVL_BOX) {
+        float l = xa[u], h = xb[u];
+        if (ivl & IVL_RELU) {
+          l = fmaxf(l, 0.f);
+          h = fmaxf(h, 0.f);
+        }
+        x = z == 0 ? (l + h) / 2.0f : (h - l) / 2.0f;
+      } else if ((ivl & IVL_BALL) && z == 1) {
+        x = g.ivl_eps;
+      }
+      if (idx < map) As[idx] = (in >> u) & 1u ? x : 0.f;
+    }
+  };
+  float xa[U], xb[U];
+  uint32_t in = 0;
+  const int64_t r0 = (int64_t)blockIdx.x * g.rows_per_wg;
+  if (MODE == MODE_F && r0 < g.R) in = map_load(r0, 0, xa, xb);
+
+  if (MODE == MODE_F) {
+    stage_conv_weights(g, Ws, 0, g.nblk, (g.abs_w >> z) & 1, tid);
+  } else {
+    // weights of every class, zero-padded in k (to Kc4) and in channels (to npad);
+    // eight loads per thread in flight, from clamped addresses, before the stores
+    const int wtotal = g.nclasses * kstride;
+    auto w_coords = [&](int idx, int& c, int& k, int& n) {
       c = fdivq(idx, g.f_kstride);
       const int rem = idx - c * kstride;
       k = fdivq(rem, g.f_npad);
       n = rem - k * g.npad;
-    }
-  };
-  for (int base = 0; base < wtotal; base += 8 * GTM) {
-    float wv[8];
+    };
+    for (int base = 0; base < wtotal; base += 8 * GTM) {
+      float wv[8];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const int idx = base + u * GTM + tid;
-      int c, k, n;
-      w_coords(idx, c, k, n);
-      const bool ok = idx < wtotal && k < g.Kc && n < g.nch;
-      int64_t src;
-      if (MODE == MODE_T) {
+      for (int u = 0; u < 8; ++u) {
+        const int idx = base + u * GTM + tid;
+        int c, k, n;
+        w_coords(idx, c, k, n);
+        const bool ok = idx < wtotal && k < g.Kc && n < g.nch;
         const int co = fdivq(k, g.f_T), t = k - co * g.T;
         const int a = fdivq(t, g.f_nB), b = t - a * g.nB;
         const int cr = fdivq(c, g.f_sw);
         const int kh = cr + g.sh * a, kw = (c - cr * g.sw) + g.sw * b;
-        src = (((int64_t)co * g.Cin + n) * g.KH + kh) * g.KW + kw;
-      } else {
-        src = (int64_t)n * g.Kc + k;   // k = (ci * KH + kh) * KW + kw
+        const int64_t src = (((int64_t)co * g.Cin + n) * g.KH + kh) * g.KW + kw;
+        const float w = g.W[ok ? src : 0];
+        wv[u] = ok ? w : 0.f;
       }
-      float w = g.W[ok ? src : 0];
-      if (MODE == MODE_F && ((g.abs_w >> z) & 1)) w = fabsf(w);
-      wv[u] = ok ? w : 0.f;
-    }
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const int idx = base + u * GTM + tid;
-      if (idx < wtotal) {
-        int c, k, n;
-        w_coords(idx, c, k, n);
-        Ws[ws_index(g, c, n, k)] = wv[u];
+      for (int u = 0; u < 8; ++u) {
+        const int idx = base + u * GTM + tid;
+        if (idx < wtotal) {
+          int c, k, n;
+          w_coords(idx, c, k, n);
+          Ws[ws_index(g, c, n, k)] = wv[u];
+        }
       }
     }
   }
@@ -356,9 +449,6 @@ conv_mfma_kernel(GatherArgs g) {
     koff[koff_index(g, k)] = off;
   }
 
-  const int nin = g.Cm * g.Hm * g.Wm;
-  const int64_t nout = (int64_t)g.nch * g.HWout;
-  const int map = g.Cm * g.Hp * g.Wp;
   const int j = lane >> 4;     // k sub-index of the MFMA operands; output row group
   const int col = lane & 15;   // pixel column (B operand / D column); channel row (A operand)
 
@@ -366,43 +456,13 @@ conv_mfma_kernel(GatherArgs g) {
     const int64_t r = (int64_t)blockIdx.x * g.rows_per_wg + i;
     if (r >= g.R) break;   // uniform
     __syncthreads();       // weights staged / previous row's map and partial sums consumed
-    const float* __restrict__ xr = X + (r / g.in_div) * nin;
-    // interval input: the operand is made from the bounds as the map is staged (the
-    // arithmetic of ibp_center_radius_kernel), uniform over the launch
-    const int ivl = MODE == MODE_F ? g.ivl : 0;
-    const float* __restrict__ hr_row = (ivl & IVL_BOX) ? g.ivl_hi + (r / g.in_div) * nin : nullptr;
-    for (int base = 0; base < map; base += 8 * GTM) {
-      float xv[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const int idx = base + u * GTM + tid;
-        const int c = fdivq(idx, g.f_HpWp), rem = idx - c * g.Hp * g.Wp;
-        const int hr = fdivq(rem, g.f_Wp);
-        const int hm = hr - g.pad_h, wm = (rem - hr * g.Wp) - g.pad_w;
-        const bool ok = idx < map && hm >= 0 && hm < g.Hm && wm >= 0 && wm < g.Wm;
-        const int src = ok ? (c * g.Hm + hm) * g.Wm + wm : 0;
-        float x;
-        if (ivl & IVL_BOX) {
-          float l = xr[src], h = hr_row[src];
-          if (ivl & IVL_RELU) {
-            l = fmaxf(l, 0.f);
-            h = fmaxf(h, 0.f);
-          }
-          x = z == 0 ? (l + h) / 2.0f : (h - l) / 2.0f;
-        } else if ((ivl & IVL_BALL) && z == 1) {
-          x = g.ivl_eps;
-        } else {
-          x = xr[src];
-        }
-        xv[u] = ok ? x : 0.f;
-      }
-#pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const int idx = base + u * GTM + tid;
-        if (idx < map) As[idx] = xv[u];
-      }
+    if (MODE == MODE_F) map_store(0, in, xa, xb);
+    for (int base = MODE == MODE_F ? U * GTM : 0; base < map; base += U * GTM) {
+      in = map_load(r, base, xa, xb);
+      map_store(base, in, xa, xb);
     }
     __syncthreads();
+    if (MODE == MODE_F && i + 1 < g.rows_per_wg && r + 1 < g.R) in = map_load(r + 1, 0, xa, xb);
     const int64_t d = r / g.S;
     const float hs = (MODE == MODE_T && lower && g.h_out) ? g.h_scale[r] : 0.f;
     const float rsv = (MODE == MODE_F && g.rs) ? g.rs[r] : 0.f;
@@ -492,6 +552,7 @@ template <bool CB_SPLIT>
 __global__ void __launch_bounds__(GTM)
 conv_ibp_kernel(GatherArgs g, IbpConvOut o) {
   extern __shared__ __attribute__((aligned(16))) float smem[];
+  constexpr int U = CB_SPLIT ? MAP_U : 8;   // (one channel block: small maps, more workgroups per CU)
   const int half = blockIdx.y;
   const int nbl = CB_SPLIT ? g.nblk / 2 : g.nblk;   // channel blocks staged here
   const int cb0 = CB_SPLIT ? half * nbl : 0;
@@ -509,29 +570,53 @@ conv_ibp_kernel(GatherArgs g, IbpConvOut o) {
     const int cb = n >> 4, col = n & 15, j = k & 3, s = k >> 2, sq = s >> 2, e = s & 3;
     return (((cb * 4 + j) * kq + sq) * 16 + col) * 4 + e;
   };
-  // weights of this half's channels in the source order (k fastest: consecutive floats of
-  // one output channel's row), eight loads per thread in flight, scattered into the LDS order
-  const int wtotal = g.Kc4 * nloc;
-  for (int base = 0; base < wtotal; base += 8 * GTM) {
-    float wv[8];
+  const int nin = g.Cm * g.Hm * g.Wm;
+  const int64_t nout = (int64_t)g.nch * g.HWout;
+  const bool box = (g.ivl & IVL_BOX) != 0, relu = (g.ivl & IVL_RELU) != 0;
+  auto map_load = [&](int64_t r, int base, float (&xl)[U], float (&xh)[U]) {   // as conv_mfma_kernel's
+    const float* __restrict__ xr = g.X[0] + r * nin;
+    const float* __restrict__ hr_row = box ? g.ivl_hi + r * nin : nullptr;
+    uint32_t in = 0;
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
+    for (int u = 0; u < U; ++u) {
       const int idx = base + u * GTM + tid;
-      const int n = fdivq(idx, g.f_Kc4), k = idx - n * g.Kc4;
-      const int ch = 16 * cb0 + n;
-      const bool ok = idx < wtotal && k < g.Kc && ch < g.nch;
-      const float w = g.W[ok ? (int64_t)ch * g.Kc + k : 0];
-      wv[u] = ok ? w : 0.f;
+      const int c = fdivq(idx, g.f_HpWp), rem = idx - c * g.Hp * g.Wp;
+      const int hr = fdivq(rem, g.f_Wp);
+      const int hm = hr - g.pad_h, wm = (rem - hr * g.Wp) - g.pad_w;
+      const bool ok = idx < map && hm >= 0 && hm < g.Hm && wm >= 0 && wm < g.Wm;
+      const int src = ok ? (c * g.Hm + hm) * g.Wm + wm : 0;
+      xl[u] = xr[src];
+      if (box) xh[u] = hr_row[src];
+      in |= ok ? 1u << u : 0u;
     }
+    return in;
+  };
+  auto map_store = [&](int base, uint32_t in, const float (&xl)[U], const float (&xh)[U]) {
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
+    for (int u = 0; u < U; ++u) {
       const int idx = base + u * GTM + tid;
-      if (idx < wtotal) {
-        const int n = fdivq(idx, g.f_Kc4), k = idx - n * g.Kc4;
-        Ws[ws_at(n, k)] = wv[u];
+      float cx = xl[u], rx = g.ivl_eps;
+      if (box) {
+        float l = xl[u], h = xh[u];
+        if (relu) {
+          l = fmaxf(l, 0.f);
+          h = fmaxf(h, 0.f);
+        }
+        cx = (l + h) / 2.0f;
+        rx = (h - l) / 2.0f;
+      }
+      if (idx < map) {
+        const bool ok = (in >> u) & 1u;
+        Mc[idx] = ok ? cx : 0.f;
+        Mr[idx] = ok ? rx : 0.f;
       }
     }
-  }
+  };
+  float xl[U], xh[U];
+  uint32_t in = 0;
+  const int64_t r0 = (int64_t)blockIdx.x * g.rows_per_wg;
+  if (r0 < g.R) in = map_load(r0, 0, xl, xh);
+  stage_conv_weights(g, Ws, 16 * cb0, nbl, false, tid);   // this half's channels
   for (int k = tid; k < g.Kc4; k += GTM) {
     int off = 0;
     if (k < g.Kc) {
@@ -542,58 +627,24 @@ conv_ibp_kernel(GatherArgs g, IbpConvOut o) {
     koff[koff_index(g, k)] = off;
   }
 
-  const int nin = g.Cm * g.Hm * g.Wm;
-  const int64_t nout = (int64_t)g.nch * g.HWout;
   const int j = lane >> 4;
   const int col = lane & 15;
   const GatherClass& C = g.cls[0];
   const int npt = (C.np + 15) / 16;
   // tasks of this half: (pixel tile, local channel block)
   const int ntl = CB_SPLIT ? npt * nbl : ((npt - half + 1) / 2) * g.nblk;
-  const bool box = (g.ivl & IVL_BOX) != 0, relu = (g.ivl & IVL_RELU) != 0;
 
   for (int i = 0; i < g.rows_per_wg; ++i) {
     const int64_t r = (int64_t)blockIdx.x * g.rows_per_wg + i;
     if (r >= g.R) break;   // uniform
     __syncthreads();       // weights staged / the previous row's maps consumed
-    const float* __restrict__ xr = g.X[0] + r * nin;
-    const float* __restrict__ hr_row = box ? g.ivl_hi + r * nin : nullptr;
-    for (int base = 0; base < map; base += 8 * GTM) {
-      float cv[8], rv[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const int idx = base + u * GTM + tid;
-        const int c = fdivq(idx, g.f_HpWp), rem = idx - c * g.Hp * g.Wp;
-        const int hr = fdivq(rem, g.f_Wp);
-        const int hm = hr - g.pad_h, wm = (rem - hr * g.Wp) - g.pad_w;
-        const bool ok = idx < map && hm >= 0 && hm < g.Hm && wm >= 0 && wm < g.Wm;
-        const int src = ok ? (c * g.Hm + hm) * g.Wm + wm : 0;
-        float cx, rx;
-        if (box) {
-          float l = xr[src], h = hr_row[src];
-          if (relu) {
-            l = fmaxf(l, 0.f);
-            h = fmaxf(h, 0.f);
-          }
-          cx = (l + h) / 2.0f;
-          rx = (h - l) / 2.0f;
-        } else {
-          cx = xr[src];
-          rx = g.ivl_eps;
-        }
-        cv[u] = ok ? cx : 0.f;
-        rv[u] = ok ? rx : 0.f;
-      }
-#pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const int idx = base + u * GTM + tid;
-        if (idx < map) {
-          Mc[idx] = cv[u];
-          Mr[idx] = rv[u];
-        }
-      }
+    map_store(0, in, xl, xh);
+    for (int base = U * GTM; base < map; base += U * GTM) {
+      in = map_load(r, base, xl, xh);
+      map_store(base, in, xl, xh);
     }
     __syncthreads();
+    if (i + 1 < g.rows_per_wg && r + 1 < g.R) in = map_load(r + 1, 0, xl, xh);
     for (int tl = wave; tl < ntl; tl += GTM / 64) {
       int pt, cbl;
       if (CB_SPLIT) {
@@ -1680,6 +1731,11 @@ static bool conv_f_mfma_plan(GatherArgs& g, int64_t R, int Ci, int Hi, int Wi, i
   return true;
 }
 
+// conv2d weight rows of whole 16-byte chunks
+static int conv_rows_vec(const GatherArgs& g) {
+  return g.Kc % 4 == 0 && (reinterpret_cast<uintptr_t>(g.W) & 15) == 0 ? 1 : 0;
+}
+
 // rows per workgroup: amortize the weight stage, keep >= ~3 workgroups per CU
 static int gather_rows_per_wg(int64_t work) {
   int64_t rpw = work / 768;
@@ -1728,6 +1784,7 @@ static int conv2d_launch(const float* x, int64_t in_div, int64_t R, int Ci, int 
       g.X[1] = x2;
       g.y[1] = y2;
       g.W = W;
+      g.w_vec = conv_rows_vec(g);
       g.abs_w = (abs_w ? 1 : 0) | (abs_w2 ? 2 : 0);   // bit z: operand pair z uses |W|
       g.in_div = in_div;
       g.rs = rs;
@@ -2169,6 +2226,7 @@ static int conv2d_ivl_launch(const float* lo, const float* hi, int ivl, float ep
   g.y[0] = yc;
   g.y[1] = yr;
   g.W = W;
+  g.w_vec = conv_rows_vec(g);
   g.abs_w = 2;   // the radius product takes |W|
   g.in_div = 1;
   g.S = 1;
@@ -2201,6 +2259,7 @@ static int conv_ibp_fused_launch(const float* lo, const float* hi, int ivl, floa
   *planned = true;
   g.X[0] = lo;
   g.W = W;
+  g.w_vec = conv_rows_vec(g);
   g.ivl = ivl;
   g.ivl_hi = hi;
   g.ivl_eps = eps;

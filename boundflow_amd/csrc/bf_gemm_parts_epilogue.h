@@ -33,8 +33,10 @@ struct EpilogueRows {
 };
 
 // The store, norm or relaxation epilogue of one workgroup tile: gemm_kernel's arithmetic in its
-// order, taken column block by column block so that a lane's store is one instruction (the same
-// epilogues with 64-bit addresses and bounds per element cost C = [128000, 500] x 2 ... see below).
+// order, taken column block by column block so that a lane's store is one instruction.  A whole
+// row block takes neither bounds nor 64-bit addresses per element: the relaxation epilogue's launch
+// on 128000 x 500 x 500, both bounds, went from 914 to 833 us by it, on 36864 x 256 x 256 with
+// the unrelaxed product stored too from 77.6 to 59.6 us.
 // smem_ab: SMEM floats of LDS no wave reads any more; m0, n0: the tile's first row and column,
 // tile_n its column tile; wm, wn: the wave's place in the tile.
 template <int EPI, class T, int SMEM>

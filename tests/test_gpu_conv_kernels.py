@@ -389,3 +389,46 @@ def test_relu_conv_transpose_concretize_matches_pass_then_conv(shape, variant):
         if z == 1 and norm_p == 0:
             sure = y.abs() > ytol
             assert torch.equal(hf.cpu()[sure], hp.cpu()[sure]), "gradient seed differs where sign(y) is certain"
+
+
+# (Ci, k, stride, size, Co, R, offset): weight rows of no whole 16-byte chunk (9, 27) and of whole ones
+# that end inside a step quad (108) or on one (48, 256), a weight tensor off a 16-byte address, maps of
+# one, of two and of a part of a staged batch (up to 10 x 30 x 30), rows that leave a workgroup a remainder
+@pytest.mark.parametrize("Ci,k,stride,size,Co,R,offset", [
+    (1, 3, 1, 5, 3, 7, 0), (3, 3, 1, 16, 12, 33, 0), (3, 4, 2, 32, 16, 20, 0), (3, 4, 2, 32, 16, 20, 1),
+    (12, 3, 1, 16, 12, 1600, 0), (16, 4, 2, 16, 32, 801, 0), (16, 4, 2, 16, 20, 40, 0), (10, 3, 2, 28, 17, 5, 0),
+    (8, 3, 1, 26, 16, 9, 3)])
+def test_conv_staging_matches_fp64(Ci, k, stride, size, Co, R, offset):
+    """The forward gather-GEMM and its interval form against float64, within the rounding of a
+    Ci k k term sum."""
+    dev = device()
+    announce(f"conv staging Ci={Ci} k={k} stride={stride} size={size} Co={Co} R={R} offset={offset}")
+    g = torch.Generator().manual_seed(Ci + 7 * k + R)
+    pad = 1
+    ho = (size + 2 * pad - k) // stride + 1
+    W = torch.randn(Co, Ci, k, k, generator=g)
+    Wd = torch.zeros(W.numel() + offset, device=dev)[offset:]
+    Wd.copy_(W.reshape(-1))
+    lo = torch.randn(R, Ci, size, size, generator=g)
+    hi = lo + torch.rand(R, Ci, size, size, generator=g)
+    bias = torch.randn(Co, generator=g)
+    lo_d, hi_d, b_d = lo.to(dev), hi.to(dev), bias.to(dev)
+    y, ylo, yhi = (torch.empty(R, Co, ho, ho, device=dev) for _ in range(3))
+    geo = (Co, k, k, stride, stride, pad, pad, ho, ho)
+    _lib.call("bf_conv2d_rows", _lib.ptr(lo_d), 1, R, Ci, size, size, _lib.ptr(Wd), 0, *geo, _lib.ptr(y), None, None, 1, 0,
+              _lib.stream_handle())
+    ws = torch.empty(int(_lib.load().bf_ibp_conv2d_workspace(R, Ci * size * size, Co * ho * ho)), device=dev)
+    _lib.call("bf_ibp_conv2d", _lib.ptr(lo_d), _lib.ptr(hi_d), R, Ci, size, size, 0, 0.0, 1, _lib.ptr(Wd), _lib.ptr(b_d), *geo,
+              None, 0, _lib.ptr(ws), _lib.ptr(ylo), _lib.ptr(yhi), None, None, _lib.stream_handle())
+    torch.cuda.synchronize()
+    conv = lambda x, w: torch.nn.functional.conv2d(x.double(), w.double(), stride=stride, padding=pad)   # noqa: E731
+    unit = (Ci * k * k + 4) * 2.0 ** -24
+    err = (y.cpu().double() - conv(lo, W)).abs()
+    assert bool((err <= unit * conv(lo.abs(), W.abs()) + 1e-30).all())
+    l, h = lo.clamp(min=0), hi.clamp(min=0)
+    c, r = conv((l.double() + h.double()) / 2, W), conv((h.double() - l.double()) / 2, W.abs())
+    # (center and radius round once, their products and the two additions after them; |l|, |h| <= l + h)
+    size_ = 4 * unit * (conv(l.double() + h.double(), W.abs()) + bias.double().abs().reshape(1, Co, 1, 1))
+    for got, want in ((ylo, c - r), (yhi, c + r)):
+        err = (got.cpu().double() - (want + bias.double().reshape(1, Co, 1, 1))).abs()
+        assert bool((err <= size_ + 1e-30).all())
