@@ -739,7 +739,7 @@ def crown_backward(
             in_parts = takes_parts(CONCRETIZE, M, P, N, S, nz)
             # bytes: the coefficient rows and the weight read, the row partial norms written, the
             # gradient seed [M, P] written when asked
-            with _timed("crown_linear_concretize", 2.0 * nz * M * N * P,
+            with _timed("crown_linear_concretize_parts" if in_parts else "crown_linear_concretize", 2.0 * nz * M * N * P,
                         4.0 * nz * (M * N + N * P + M * -(-P // 128)) + (4.0 * M * P if h_out is not None else 0.0)):
                 _lib.call("bf_crown_linear_concretize_parts" if in_parts else "bf_crown_linear_concretize",
                           _lib.ptr(A_u), _lib.ptr(A_l), stride, B, S, N,
@@ -823,12 +823,13 @@ def crown_backward(
             e_bytes = (16.0 * B * P + (4.0 * B * P if (n_add is not None and A_l is not None) else 0.0)
                        + (4.0 * B * P if cvec is not None else 0.0)
                        + 4.0 * nz * M * -(-P // 128) * (2 if cvec is not None else 1))
-            with _timed("crown_relu_linear_relu_fwd", flops,
+            packed = plain and takes_parts(RELAX, M, P, N, S, nz)
+            with _timed("crown_linear_relu_fwd_parts" if packed else "crown_relu_linear_relu_fwd", flops,
                         nbytes + e_bytes + (4.0 * M * P if pre_l is not None else 0.0)):
                 after = (_lib.ptr(b_u), _lib.ptr(b_l), _lib.ptr(n_table), _lib.ptr(n_add), n_add_ld, _lib.ptr(n_bias),
                          _lib.ptr(cvec), P, _lib.ptr(ws), _lib.ptr(nA_u), _lib.ptr(nA_l), None, _lib.ptr(pre_l),
                          _lib.ptr(nb_u), _lib.ptr(nb_l), _lib.ptr(nc_u), _lib.ptr(nc_l), stream)
-                if plain and takes_parts(RELAX, M, P, N, S, nz):
+                if packed:
                     _lib.call("bf_crown_linear_relu_fwd_parts", _lib.ptr(A_u), _lib.ptr(A_l), stride, B, S, N,
                               _lib.ptr(chain_parts(layers, layer, M, S, nz, save)), P, *after)
                 else:
@@ -859,8 +860,9 @@ def crown_backward(
                 rows = (_lib.ptr(bias), None if keep_b else _lib.ptr(b_u), None if keep_b else _lib.ptr(b_l),
                         _lib.ptr(nA_u), _lib.ptr(nA_l), None if keep_b else _lib.ptr(nb_u),
                         None if keep_b else _lib.ptr(nb_l), stream)
-                with _timed("crown_relu_linear_fwd", flops, nbytes):
-                    if plain and takes_parts(STORE, M, P, N, S, nz):
+                packed = plain and takes_parts(STORE, M, P, N, S, nz)
+                with _timed("crown_linear_parts" if packed else "crown_relu_linear_fwd", flops, nbytes):
+                    if packed:
                         _lib.call("bf_crown_linear_parts", _lib.ptr(A_u), _lib.ptr(A_l), stride, B, S, N,
                                   _lib.ptr(chain_parts(layers, layer, M, S, nz, save)), P, *rows)
                     else:

@@ -538,12 +538,14 @@ def crown_backward_dag(
                 nb_l = None if nb_l is None else nb_l.reshape(M)
             A_l_in = None if one else st.A_l
             nz = int(st.A_u is not None) + int(A_l_in is not None)
-            with _timed("crown_linear", 2.0 * nz * M * N * P, 4.0 * nz * (M * N + N * P + M * P)):
+            packed = takes_parts(STORE, M, P, N, S, nz)
+            with _timed("crown_linear_parts" if packed else "crown_linear", 2.0 * nz * M * N * P,
+                        4.0 * nz * (M * N + N * P + M * P)):
                 out_b = (None, None) if keep_b else (_lib.ptr(nb_u), _lib.ptr(None if one else nb_l))
                 rows = (_lib.ptr(bias), _lib.ptr(None if keep_b else st.b_u),
                         _lib.ptr(None if one or keep_b else st.b_l), _lib.ptr(nA_u),
                         _lib.ptr(None if one else nA_l), *out_b, stream)
-                if takes_parts(STORE, M, P, N, S, nz):
+                if packed:
                     _lib.call("bf_crown_linear_parts", _lib.ptr(st.A_u), _lib.ptr(A_l_in), S * N, B, S, N,
                               _lib.ptr(weight_parts(params[op.inputs[1]], False)), P, *rows)
                 else:
@@ -743,10 +745,12 @@ def lower_grad_pass(module: BFTaskModule, spec: InputSpec, trace: DagTrace, save
             n_out, n_in = int(W.shape[0]), int(W.shape[1])
             gt = torch.empty(M, n_out, device=dev)
             rank1 = (_lib.ptr(G if bias is not None else None), _lib.ptr(bias), 0)
-            with _timed("grad_gemm", 2.0 * M * n_in * n_out, 4.0 * (M * n_in + M * n_out + n_in * n_out)):
-                wsz = int(_lib.load().bf_gemm_rank1_workspace(M, n_out, n_in))
-                # (a contraction the fp32 kernels split over K keeps the split)
-                if not wsz and takes_parts(STORE, M, n_out, n_in, S, 1):
+            wsz = int(_lib.load().bf_gemm_rank1_workspace(M, n_out, n_in))
+            # (a contraction the fp32 kernels split over K keeps the split)
+            packed = not wsz and takes_parts(STORE, M, n_out, n_in, S, 1)
+            with _timed("grad_gemm_parts" if packed else "grad_gemm", 2.0 * M * n_in * n_out,
+                        4.0 * (M * n_in + M * n_out + n_in * n_out)):
+                if packed:
                     _lib.call("bf_gemm_rank1_parts", _lib.ptr(GA[x]), n_in,
                               _lib.ptr(weight_parts(params[op.inputs[1]], True)), _lib.ptr(gt), n_out, M, n_out, n_in,
                               S, *rank1, stream)

@@ -295,7 +295,8 @@ class HipFusedCrownExecutor:
                     _lib.call("bf_crown_relu_relax", _lib.ptr(request.A_u), _lib.ptr(request.A_l), S * N, D, S, N,
                               _lib.ptr(table), None, 0, _lib.ptr(bias), None, None, None, _lib.ptr(ru), _lib.ptr(rl),
                               _lib.ptr(du), _lib.ptr(dl), None, None, st)
-                with _timed("executor_linear", 4.0 * M * N * P, 4.0 * (2 * M * N + N * P + 2 * M * P)):
+                with _timed("executor_linear_parts" if packed else "executor_linear", 4.0 * M * N * P,
+                            4.0 * (2 * M * N + N * P + 2 * M * P)):
                     rows = (None, None, None, _lib.ptr(pu), _lib.ptr(pl), None, None, st)
                     if packed:
                         _lib.call("bf_crown_linear_parts", _lib.ptr(ru), _lib.ptr(rl), S * N, D, S, N,
