@@ -317,21 +317,23 @@ __device__ __forceinline__ void stage_conv_weights(const GatherArgs& g, float* W
   }
 }
 
-// Elements of a row's map a thread of the forward gather-GEMM stages at a time: the first batch of a
-// row is loaded ahead of the weights (the first row) or of the products of the row before, so
+// Elements of a row's map a thread of the interval conv stages at a time: the first batch of a row
+// is loaded ahead of the weights (the first row) or of the products of the row before, so
 // its way from memory runs beside them, and the maps of the networks at hand (16 x 18 x 18,
 // 3 x 34 x 34) are one batch.  The interval conv of 2048 inputs, 16 x 18 x 18 -> 32 x 8 x 8: 142.6 -> 104.2 us,
 // 3 x 34 x 34 -> 16 x 16 x 16 (8 at a time): 76.0 -> 62.3 us (12 at a time 70.8: fewer workgroups fit the
 // registers; so does a branch around the elements past the map, at 132 registers: 142 and 94 us).
-// The transposed direction keeps its 8 loads behind the weights (53 registers; 20.7 us over a residual
-// net's 3 x 3 layers, 26.3 us loaded ahead).
+// conv_mfma_kernel loads a map in place, 8 at a time: its maps are small and its launches short, and what a
+// load ahead holds in registers (109 against 57) costs more than it hides.  Slope optimisation on a CNN of 8
+// channels, 8 steps: 4 inputs 766 us ahead, 735 in place; 32 inputs 970, 925; of 16 channels, 32 inputs
+// 1136, 1105; the transposed direction over a residual net's 3 x 3 layers 26.3 us, 20.7.
 constexpr int MAP_U = 12;
 
 template <int MODE>
 __global__ void __launch_bounds__(GTM)
 conv_mfma_kernel(GatherArgs g) {
   extern __shared__ __attribute__((aligned(16))) float smem[];
-  constexpr int U = MODE == MODE_F ? MAP_U : 8;
+  constexpr int U = 8;   // map elements a thread loads at a time
   float* Ws = smem;                                              // [nclasses][Kc4][npad]
   int* koff = reinterpret_cast<int*>(Ws + (size_t)g.nclasses * g.Kc4 * g.npad);   // [Kc4]
   float* As = reinterpret_cast<float*>(koff + g.Kc4);            // [Cm][Hp][Wp]
@@ -389,10 +391,6 @@ conv_mfma_kernel(GatherArgs g) {
       if (idx < map) As[idx] = (in >> u) & 1u ? x : 0.f;
     }
   };
-  float xa[U], xb[U];
-  uint32_t in = 0;
-  const int64_t r0 = (int64_t)blockIdx.x * g.rows_per_wg;
-  if (MODE == MODE_F && r0 < g.R) in = map_load(r0, 0, xa, xb);
 
   if (MODE == MODE_F) {
     stage_conv_weights(g, Ws, 0, g.nblk, (g.abs_w >> z) & 1, tid);
@@ -456,13 +454,12 @@ conv_mfma_kernel(GatherArgs g) {
     const int64_t r = (int64_t)blockIdx.x * g.rows_per_wg + i;
     if (r >= g.R) break;   // uniform
     __syncthreads();       // weights staged / previous row's map and partial sums consumed
-    if (MODE == MODE_F) map_store(0, in, xa, xb);
-    for (int base = MODE == MODE_F ? U * GTM : 0; base < map; base += U * GTM) {
-      in = map_load(r, base, xa, xb);
+    for (int base = 0; base < map; base += U * GTM) {
+      float xa[U], xb[U];
+      const uint32_t in = map_load(r, base, xa, xb);
       map_store(base, in, xa, xb);
     }
     __syncthreads();
-    if (MODE == MODE_F && i + 1 < g.rows_per_wg && r + 1 < g.R) in = map_load(r + 1, 0, xa, xb);
     const int64_t d = r / g.S;
     const float hs = (MODE == MODE_T && lower && g.h_out) ? g.h_scale[r] : 0.f;
     const float rsv = (MODE == MODE_F && g.rs) ? g.rs[r] : 0.f;
