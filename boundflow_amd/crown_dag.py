@@ -562,9 +562,10 @@ def crown_backward_dag(
             n_out = Co * Ho * Wo
             if len(op.inputs) == 3 and op_index not in folded:
                 bias = params[op.inputs[2]]
-                st, _ = rows_pass(st, n_out, kbias=derived(f"conv_bias_map:{Ho}x{Wo}", (bias,),
-                                                           lambda b=bias: _conv_bias_map(b.detach(), out_shape)),
-                                  name="conv_bias_rows")
+                # (bound here: a captured query remakes the map long after this loop has moved on)
+                kbias = derived(f"conv_bias_map:{Ho}x{Wo}", (bias,),
+                                lambda b=bias, shape=out_shape: _conv_bias_map(b.detach(), shape))
+                st, _ = rows_pass(st, n_out, kbias=kbias, name="conv_bias_rows")
             one = shared(st)
             y_u, y_l = like(st, Ci * Hi * Wi, one)
             A_l_in = None if one else st.A_l
