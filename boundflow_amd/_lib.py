@@ -34,6 +34,7 @@ SIGNATURES = {
     "bf_gemm_rank1": (I32, [P, I64, P, I64, I32, P, I64, I64, I64, I64, I64, P, P, I64, P, I64, P]),
     "bf_gemm_rank1_workspace": (I64, [I64, I64, I64]),
     "bf_gemm_parts_config": (I32, [I64, I64, I64, I64, I32, I32]),
+    "bf_gemm_parts_pays": (I32, [I64, I64, I64, I64, I32, I32]),
     "bf_gemm_parts_floats": (I64, [I64, I64]),
     "bf_gemm_pack_parts": (I32, [I32, P, P, P, P, P, P, P]),
     "bf_gemm_rank1_parts": (I32, [P, I64, P, P, I64, I64, I64, I64, I64, P, P, I64, P]),

@@ -228,7 +228,7 @@ def takes_parts(form: int, M: int, N: int, K: int, S: int, nz: int) -> bool:
 
 @functools.lru_cache(maxsize=4096)
 def _parts_rule(M: int, N: int, K: int, S: int, nz: int, form: int) -> bool:
-    return _lib.load().bf_gemm_parts_config(M, N, K, S, nz, form) != 0
+    return _lib.load().bf_gemm_parts_pays(M, N, K, S, nz, form) != 0
 
 
 # ---------------------------------------------------------------------------

@@ -136,18 +136,11 @@ int launch_parts(const GemmArgs& a, int epi, int nz, bool small, hipStream_t str
 // domains of S rows, epilogue epi): 'P' (128 x 128), 'S' (64 x 64) or 0.  K must fill a stage and
 // rows lie within the 32-bit byte offsets of a tile; a launch below 256 rows is bound by its launch
 // and its K loop on either kind (9 x 256 x 256: 10.0 / 9.9 us fp32 / 64 x 64).
-// us on one MI355X, fp32 / 64 x 64 / 128 x 128:
-//   576 x 256: K = 64 7.5 / 5.9 / 8.0, 256 11.7 / 10.6 / 14.9, 512 17.4 / 16.7 / 24.0, 1024 28.7 / 29.0 / 42.1
-//   2304 x 512 (288 64 x 64 tiles): K = 64 8.6 / 7.1 / 8.6, 256 16.1 / 13.0 / 15.6, 1024 44.2 / 37.2 / 43.1
-//   4608 x 784 (936): K = 256 26.8 / 17.0 / 17.8, 1024 81.3 / 51.1 / 51.0
-//   9216 x 784 (1872): K = 256 42.1 / 32.6 / 26.6;  36864 x 256 (2304): 54.9 / 35.7 / 34.9
-// and where K is no multiple of four (the fp32 tiles then read their operands float by float), fp32 /
-// the tile taken: 2304 x 50: K = 30 7.3 / 6.4, 50 8.6 / 7.6, 333 19.9 / 17.7; 36864 x 250: K = 30
-// 23.0 / 14.6, 50 33.0 / 17.9, 250 93.6 / 39.2; 100000 x 50: K = 50 32.4 / 21.0;
-// so the store epilogue takes 64 x 64 below 1536 of them (six per CU, what is resident at once), and
-// past K = 512 leaves a grid that is not one tile per CU to the fp32 kernels.  The norm epilogue's tile
-// follows its partial norms' width; it and the relaxation epilogue take 128 x 128 from 128 tiles on
-// (72 tiles: level with fp32).
+// The store epilogue takes 64 x 64 below 1536 of them (six per CU, what is resident at once): the faster
+// tile up to 1280 at every K measured, 128 x 128 from 1872 on but for grids whose second round of
+// 128 x 128 workgroups is mostly empty (36864 x 256: 8 % slower).  The norm epilogue's tile follows its
+// partial norms' width; it and the relaxation epilogue take 128 x 128 from 128 tiles on.  Which of these
+// shapes gain by it is gemm_parts_pays' to say.
 int gemm_parts_choice(int64_t M, int64_t N, int64_t K, int64_t S, int nz, int epi) {
   if (kForcedTile || M < 256 || N <= 0 || K < 16 || S <= 0 || N >= (1LL << 31) || K >= (1LL << 31))
     return 0;
@@ -157,6 +150,44 @@ int gemm_parts_choice(int64_t M, int64_t N, int64_t K, int64_t S, int nz, int ep
   if (epi == EPI_STORE && t64 < 1536) return short_k ? 'S' : 0;
   if (epi == EPI_ABSSUM && gemm_norm_cols(M, N, PRO_PLAIN) == NORM_BN / 2) return short_k ? 'S' : 0;
   return ceil_div(M, (int64_t)128) * ceil_div(N, (int64_t)128) * nz >= 128 ? 'P' : 0;
+}
+
+// Where the three-part kernel is the faster one.  us on one MI355X:
+// stores, fp32 / 64 x 64 / 128 x 128 tiles (in brackets the 64 x 64 tiles):
+//   576 x 256 (36):       K = 64 7.4 / 6.6 / 9.1, 128 8.8 / 8.5 / 12.0, 256 11.6 / 12.3 / 17.9, 512 17.5 / 20.0 / 29.1
+//   2304 x 512 (288):     K = 64 8.8 / 8.1 / 9.7, 256 16.6 / 15.8 / 18.5, 512 26.3 / 26.3 / 29.9, 1024 45.6 / 46.0 / 51.9
+//   4608 x 784 (936):     K = 256 28.3 / 20.4 / 22.1, 1024 83.4 / 60.3 / 60.3
+//   9216 x 784 (1872):    K = 256 42.5 / 38.0 / 31.5
+//   36864 x 256 (2304):   K = 16 13.3 / 12.1 / 15.0, 64 21.6 / 18.4 / 22.1, 256 53.6 / 41.7 / 45.0
+// stores where K is no multiple of 32 (the fp32 tiles then check their loads) or of four (float by float):
+//   576 x 256:   K = 50 8.4 / 8.3 / 10.3, 100 10.1 / 7.9 / 11.1, 250 16.2 / 16.2 / 21.6, 500 23.0 / 20.1 / 29.4
+//   36864 x 256: K = 50 32.2 / 22.4 / 23.6, 250 93.0 / 47.6 / 50.7, 500 94.5 / 76.6 / 78.3
+// norms, both bounds, fp32 / three-part:
+//   288 x 784 (130 64 x 64 tiles): K = 128 15.9 / 15.1, 256 19.7 / 20.2, 512 24.9 / 27.6
+//   36864 x 5 (576 128 x 128 tiles): K = 50 24.6 / 22.8, 256 33.5 / 41.6
+// relaxation, fp32 / three-part (in brackets the 128 x 128 tiles, 512 of which are resident at once):
+//   9216 x 256 (144):   K = 64 19.8 / 19.0, 256 32.6 / 27.5
+//   36864 x 256 (576):  K = 64 30.0 / 37.0, 128 40.9 / 44.0, 256 62.2 / 59.8
+//   36864 x 256, both bounds (1152): K = 64 51.7 / 58.0, 128 71.3 / 68.9, 256 111.5 / 95.1
+bool gemm_parts_pays(int64_t M, int64_t N, int64_t K, int64_t S, int nz, int epi) {
+  const int tile = gemm_parts_choice(M, N, K, S, nz, epi);
+  if (!tile) return false;
+  const int64_t t64 = ceil_div(M, (int64_t)64) * ceil_div(N, (int64_t)64) * nz;
+  const int64_t t128 = ceil_div(M, (int64_t)128) * ceil_div(N, (int64_t)128) * nz;
+  if (epi == EPI_STORE) {
+    if (tile == 'P') return K > 64 || K % 4 || t64 < 2048 || t64 >= 3072;
+    // fewer tiles than CUs: a tile's own K loop is the time, and fp32's is the shorter one past K = 128
+    if (t64 < 256) return K <= 128 || (K % 32 && K % 4 == 0);
+    return t64 >= 512 || K <= 256 || K % 32;
+  }
+  if (epi == EPI_ABSSUM) {
+    if (tile == 'S') return K <= 128 || K % 4 || (t64 >= 256 && N > 32);
+    return N > 64 || K % 4;   // (columns past N cost a 128 x 128 tile what those inside do)
+  }
+  // a second round of 128 x 128 workgroups, mostly empty, outweighs what a short K gains
+  const bool fills = t128 <= 512 || t128 > 768;
+  if (K % 4) return t128 >= 256 || K >= 100;
+  return (K >= 100 && fills) || (K >= 256 && N > 64);
 }
 
 int gemm_dispatch(const GemmArgs& a, int pro, int epi, int nz, hipStream_t stream) {

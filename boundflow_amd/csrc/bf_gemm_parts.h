@@ -5,13 +5,17 @@
 //
 // Every operand value is split into three bf16 parts, each the nearest bf16 of what the
 // parts before it leave: x = x0 + x1 + x2 exactly (8 + 8 + 8 significant bits against 24;
-// the exponent range of bf16 is fp32's).  A product is the sum of the six part products
-// above 2^-24 of it,
-//   x0 y0 + (x0 y1 + x1 y0) + (x1 y1 + x0 y2 + x2 y0),
-// each exact, summed in fp32 by v_mfma_f32_32x32x16_bf16: six of these take 192 cycles for
-// the 16 k steps that eight v_mfma_f32_32x32x2f32 take 512 for.  What is left out is below
-// 2^-24 of a product, the rounding of one fp32 addition, and the 6 roundings of a sum per
-// 16 k stand against 8.
+// the exponent range of bf16 is fp32's).  A product is the sum of eight part products,
+//   x0 y0 + (x0 y1 + x1 y0) + (x1 y1 + x0 y2 + x2 y0) + (x1 y2 + x2 y1),
+// each exact; x2 y2, the ninth, is below 2^-32 of it.  They are summed in fp32 by
+// v_mfma_f32_32x32x16_bf16: eight of these take 256 cycles for the 16 k steps that eight
+// v_mfma_f32_32x32x2f32 take 512 for.  The x0 y0 products and the others have a sum of their own
+// each, joined at the end: the low one is 2^-8 of the other, so its roundings do not count, and
+// the high one rounds once per 16 k (the fp32 tiles: once per k that has a product).  Relative
+// error (2-norm) against float64 on 9216 x 256 x 256, fp32 tiles / these: dense rows 2.9e-7 /
+// 0.9e-7; rows of 16, 4, 2 and 1 nonzeros 7.4 / 3.4, 4.0 / 2.6, 3.1 / 2.6 and 2.5 / 2.5e-8.  (All
+// products into one sum: 2.4e-7, 13.8, 7.3, 5.1 and 3.5e-8, with six, eight or nine of them: a row's
+// few products are rounded up to nine times where the fp32 tiles round once.)
 //
 // B (a layer's weight) comes packed: its parts made once per weight (pack_parts_kernel), in
 // the MFMA operand order, so that a stage's parts go straight from global memory to LDS.  A
@@ -37,6 +41,7 @@ typedef uint32_t uint32x4 __attribute__((ext_vector_type(4)));
 // values (column l % 32, k 8 (l / 32) .. + 7) at 16 l; columns and k past the end are zero.
 constexpr int PARTS_BLOCK = 3 * 64 * 4;   // floats of one block and stage
 
+// OCC: workgroups resident per CU (the two sums of a 32 x 128 wave tile are 128 registers).
 template <int FM_, int FN_, int NWM_, int OCC_>
 struct TileParts {
   static constexpr int FM = FM_, FN = FN_, NWM = NWM_, NWN = 1, OCC = OCC_;
@@ -172,16 +177,17 @@ __global__ void __launch_bounds__(T::NT, (T::OCC * T::NWM + 3) / 4) gemm_parts_k
     for (int c = 0; c < T::B_COPIES; ++c) lds_copy16_at(src + b_src[c], b_lane, dst + 256 * c);
   };
 
-  floatx16 acc[FM][FN];
-  auto clear = [&]() {
+  floatx16 acc[FM][FN], low[FM][FN];   // sums of the x0 y0 products and of the others
+  auto clear = [&](floatx16 (&sum)[FM][FN]) {
 #pragma unroll
     for (int i = 0; i < FM; ++i)
 #pragma unroll
       for (int j = 0; j < FN; ++j)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+        for (int r = 0; r < 16; ++r) sum[i][j][r] = 0.f;
   };
-  clear();
+  clear(acc);
+  clear(low);
 
   // operand positions of this lane in its wave's A stage: row 32 i + lrow, k quads 2 h and 2 h + 1
   const int swz = (lrow >> 1) & 3;
@@ -239,21 +245,23 @@ __global__ void __launch_bounds__(T::NT, (T::OCC * T::NWM + 3) / 4) gemm_parts_k
       read_b(0);
       read_a(sa);   // (past the last stage: what the slot held, split for nothing)
       __builtin_amdgcn_sched_barrier(0);
-      constexpr int MFMAS = 6 * FM;   // of a column block
+      // the smallest products first
+      constexpr int NP = 8;
+      constexpr int PA[NP] = {2, 1, 2, 0, 1, 1, 0, 0}, PB[NP] = {1, 2, 0, 2, 1, 0, 1, 0};
+      constexpr int MFMAS = NP * FM;   // of a column block
 #pragma unroll
       for (int j = 0; j < FN; ++j) {
         const bool on = FULL || j < fn_act;
         if (j + 1 < FN && (FULL || j + 1 < fn_act)) read_b(j + 1);
         __builtin_amdgcn_sched_barrier(0);
-        // the smallest products first
-        constexpr int PA[6] = {2, 0, 1, 1, 0, 0}, PB[6] = {0, 2, 1, 0, 1, 0};
 #pragma unroll
         for (int m = 0; m < MFMAS; ++m) {
           const int q = m / FM, i = m % FM;
-          if (on)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, ap[cur][i][PA[q]]),
-                                                                __builtin_bit_cast(bf16x8, bp[j & 1][PB[q]]),
-                                                                acc[i][j], 0, 0, 0);
+          if (on) {
+            floatx16& sum = q == NP - 1 ? acc[i][j] : low[i][j];
+            sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, ap[cur][i][PA[q]]),
+                                                          __builtin_bit_cast(bf16x8, bp[j & 1][PB[q]]), sum, 0, 0, 0);
+          }
           // (the first block leaves the A reads time to land)
           constexpr int FIRST = FN > 2 ? 1 : 0;
           if (j >= FIRST) {
@@ -283,9 +291,12 @@ __global__ void __launch_bounds__(T::NT, (T::OCC * T::NWM + 3) / 4) gemm_parts_k
 #pragma unroll
     for (int j = 0; j < FN; ++j)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) probe = __builtin_fmaf(acc[i][j][r], 0.f, probe);
+      for (int r = 0; r < 16; ++r) {
+        acc[i][j][r] += low[i][j][r];
+        probe = __builtin_fmaf(acc[i][j][r], 0.f, probe);
+      }
   if (__any(probe != 0.f)) {
-    clear();
+    clear(acc);
     const float* arow[FM];
 #pragma unroll
     for (int i = 0; i < FM; ++i) {
@@ -321,7 +332,9 @@ __global__ void __launch_bounds__(T::NT, (T::OCC * T::NWM + 3) / 4) gemm_parts_k
   parts_epilogue<EPI, T, SMEM>(p, acc, smem_ab, red, m0, n0, tile_n, wave, 0, lane, z, lower);
 }
 
-using TileP = TileParts<1, 4, 4, 3>;    // 128 x 128, 4 waves of 32 x 128, 3 workgroups per CU
+// (a 64 x 128 tile of two waves, four workgroups per CU: 3 to 9 % slower on grids past 1000 tiles, and no
+// better where 128 x 128 tiles leave a second round of workgroups mostly empty)
+using TileP = TileParts<1, 4, 4, 2>;    // 128 x 128, 4 waves of 32 x 128, 2 workgroups per CU
 using TilePS = TileParts<1, 2, 2, 6>;   // 64 x 64, 2 waves of 32 x 64, 6 workgroups per CU
 
 int launch_parts(const GemmArgs& a, int epi, int nz, bool small, hipStream_t stream);

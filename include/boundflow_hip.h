@@ -55,11 +55,11 @@ int bf_gemm_tile_config(int64_t M, int64_t N, int nz, int ksplit, int relax_prol
  * value as three bf16 parts whose sum is the value, in the matrix operand order) serves
  * contractions at fp32 accuracy at more than the fp32 MFMA rate: the *_parts entry points
  * below, each the arithmetic of its namesake with the products of the parts down to
- * 2^-24 of a product, summed in fp32.
+ * 2^-32 of a product, summed in fp32 (the leading ones apart from the others).
  * bf_gemm_parts_config: the tile on which they take M rows (domains of S rows) x N outputs
- * over K with nz bounds, 'P' (128 x 128) or 'S' (64 x 64), else 0 (K below 16, a grid
- * the fp32 kernels run as fast, or rows past 32-bit offsets): the caller then takes the
- * namesake.  form: 0 the stores (bf_gemm_rank1_parts,
+ * over K with nz bounds, 'P' (128 x 128) or 'S' (64 x 64), else 0 (K below 16, a short
+ * grid, or rows past 32-bit offsets): the caller then takes the namesake.
+ * bf_gemm_parts_pays: whether that is also faster than the namesake.  form: 0 the stores (bf_gemm_rank1_parts,
  * bf_crown_linear_parts), 1 bf_crown_linear_concretize_parts, 2 bf_crown_linear_relu_fwd_parts.
  * Coefficient rows must be dense.
  * bf_gemm_pack_parts: count weights in one launch, B[j] as [N, K] (trans_b) or [K, N]
@@ -68,6 +68,7 @@ int bf_gemm_tile_config(int64_t M, int64_t N, int nz, int ksplit, int relax_prol
  * No counterpart in the reference (its contractions are torch matmuls,
  * runtime/crown_ibp.py:1371-1700). */
 int bf_gemm_parts_config(int64_t M, int64_t N, int64_t K, int64_t S, int nz, int form);
+int bf_gemm_parts_pays(int64_t M, int64_t N, int64_t K, int64_t S, int nz, int form);
 int64_t bf_gemm_parts_floats(int64_t N, int64_t K);
 int bf_gemm_pack_parts(int count, const float* const* B, const int64_t* ldb, const int* trans_b, const int64_t* N,
                        const int64_t* K, float* const* parts, hipStream_t stream);

@@ -40,6 +40,26 @@ def test_shapes_taken():
     assert not config(36864, 256, 256, 9, 1, 3)
 
 
+@pytest.mark.parametrize("gains,M,N,K,nz,form", [
+    # stores: fewer 64 x 64 tiles than CUs, one or two a CU, 128 x 128 tiles
+    (True, 2304, 256, 128, 1, 0), (False, 2304, 256, 256, 1, 0), (True, 2304, 256, 500, 1, 0), (False, 2304, 256, 250, 1, 0),
+    (True, 4096, 256, 256, 1, 0), (False, 4096, 256, 512, 1, 0), (True, 4096, 256, 500, 1, 0), (True, 8192, 256, 512, 1, 0),
+    (False, 36864, 256, 64, 1, 0), (True, 36864, 256, 50, 1, 0), (True, 49152, 256, 64, 1, 0), (True, 128000, 500, 500, 2, 0),
+    # norms: the 64-column tile, the 128-column one over a few columns
+    (True, 288, 784, 128, 2, 1), (False, 288, 784, 256, 2, 1), (True, 100000, 5, 50, 2, 1), (False, 100000, 5, 256, 2, 1),
+    # relaxation: a second round of workgroups that fills, one that does not
+    (False, 9216, 256, 64, 1, 2), (True, 9216, 256, 128, 1, 2), (False, 36864, 256, 128, 1, 2), (True, 36864, 256, 256, 1, 2),
+    (True, 36864, 256, 128, 2, 2), (True, 50000, 50, 50, 2, 2), (False, 8192, 256, 50, 1, 2),
+    (False, 255, 256, 64, 1, 0), (False, 36864, 256, 256, 3, 0)])
+def test_shapes_that_gain(gains, M, N, K, nz, form):
+    if not _lib.LIB_PATH.exists():
+        pytest.skip("library not built (run python -m boundflow_amd.build)")
+    if os.environ.get("BOUNDFLOW_GEMM_TILE"):
+        pytest.skip("tile forced by the environment")
+    assert bool(_lib.load().bf_gemm_parts_pays(M, N, K, 9, nz, form)) == gains
+    assert not gains or config(M, N, K, 9, nz, form)
+
+
 def pack(W, trans_b):
     n, p = W.shape
     N, K = (n, p) if trans_b else (p, n)
@@ -104,6 +124,33 @@ def test_error_is_not_above_the_fp32_tiles(M, N, K, positive):
     err, err32 = (float((c.double() - ref).norm() / ref.norm()) for c in (C, C32))
     announce(f"parts error {err:.3e}, fp32 tiles {err32:.3e} (M={M} N={N} K={K} positive={positive})")
     assert err <= err32
+
+
+@gpu
+@pytest.mark.parametrize("M,N,K", [(36864, 256, 256), (2304, 256, 64), (9216, 97, 50), (2304, 500, 100), (36864, 129, 500)])
+@pytest.mark.parametrize("nonzeros", [1, 2, 4, 16])
+def test_sparse_rows_are_no_further_off_than_the_fp32_tiles(M, N, K, nonzeros):
+    """Rows of few nonzero coefficients (stable-off ReLUs leave such): the fp32 contraction rounds a sum
+    once per nonzero.  One product alone is within fp32's own rounding: what is left out of it and the
+    rounding of its low sum are below 9 x 2^-33 of it, 2^-6 of half a unit in the last place."""
+    dev = device()
+    announce(f"parts sparse rows M={M} N={N} K={K} nonzeros={nonzeros}")
+    assert config(M, N, K, 9, 1, 0)
+    g = torch.Generator(device=dev).manual_seed(M + N + K + nonzeros)
+    A, B = torch.randn(M, K, generator=g, device=dev), torch.randn(N, K, generator=g, device=dev)
+    at = torch.rand(M, K, generator=g, device=dev).topk(nonzeros, dim=1).indices
+    A = A * torch.zeros_like(A).scatter_(1, at, 1.0)
+    C, C32 = torch.empty(M, N, device=dev), torch.empty(M, N, device=dev)
+    _lib.call("bf_gemm_rank1_parts", _lib.ptr(A), K, _lib.ptr(pack(B, True)), _lib.ptr(C), N, M, N, K, 9, None, None,
+              0, _lib.stream_handle())
+    _lib.call("bf_gemm", _lib.ptr(A), K, _lib.ptr(B), K, 1, 0, _lib.ptr(C32), N, M, N, K, _lib.stream_handle())
+    torch.cuda.synchronize()
+    ref = A.double() @ B.double().t()
+    err, err32 = (float((c.double() - ref).norm() / ref.norm()) for c in (C, C32))
+    announce(f"parts error {err:.4e}, fp32 tiles {err32:.4e}")
+    assert err <= err32 * (1 + 2.0 ** -6)
+    if nonzeros == 1:
+        assert bool(((C.double() - ref).abs() <= 2.0 ** -24 * (1 + 2.0 ** -6) * ref.abs()).all())
 
 
 @gpu
