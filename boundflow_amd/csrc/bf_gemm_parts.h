@@ -4,8 +4,10 @@
 //   C[M, N] = A[M, K] x B[N, K]^T
 //
 // Every operand value is split into three bf16 parts, each the nearest bf16 of what the
-// parts before it leave: x = x0 + x1 + x2 exactly (8 + 8 + 8 significant bits against 24;
-// the exponent range of bf16 is fp32's).  A product is the sum of eight part products,
+// parts before it leave: x = x0 + x1 + x2 exactly (8 + 8 + 8 significant bits against 24).
+// The exponent range of bf16 is fp32's, so the lower parts of a small value would be subnormal,
+// which the matrix cores read as zero: values are split times 2^24, which leaves the least part
+// of the least subnormal at 2^-125, and the sums are multiplied by 2^-48 at the end.  A product is the sum of eight part products,
 //   x0 y0 + (x0 y1 + x1 y0) + (x1 y1 + x0 y2 + x2 y0) + (x1 y2 + x2 y1),
 // each exact; x2 y2, the ninth, is below 2^-32 of it.  They are summed in fp32 by
 // v_mfma_f32_32x32x16_bf16: eight of these take 256 cycles for the 16 k steps that eight
@@ -23,9 +25,9 @@
 // are (global_load_lds_dwordx4, private to the wave, so no barrier guards them) and it splits
 // them once, in registers.  Stages are 16 k deep, three of A and two of B; one barrier each.
 //
-// A tile with a sum that is not finite (an operand that is not, or a coefficient above the
-// largest bf16, whose parts are then not defined) is computed again by v_mfma_f32_32x32x2f32
-// from the fp32 values, so such operands give what they give on the fp32 tiles.
+// A tile with a sum that is not finite (an operand that is not, a value of 2^103 or more, which
+// has no parts, or a sum past 2^79) is computed again by v_mfma_f32_32x32x2f32 from the fp32
+// values, so such operands give what they give on the fp32 tiles.
 #pragma once
 
 #include "bf_gemm_parts_epilogue.h"
@@ -39,7 +41,11 @@ typedef uint32_t uint32x4 __attribute__((ext_vector_type(4)));
 
 // Packed parts of B: per 32-column block and 16-k stage 3 KB, part by part, lane l's eight
 // values (column l % 32, k 8 (l / 32) .. + 7) at 16 l; columns and k past the end are zero.
+// A value that has no parts lies there as the NaN PARTS_RAW and the two halves of its 32 bits: the
+// NaN sends every tile that meets it to the fp32 MFMAs, which read it whole.
 constexpr int PARTS_BLOCK = 3 * 64 * 4;   // floats of one block and stage
+constexpr uint32_t PARTS_RAW = 0x7fff;
+constexpr float PARTS_SCALE = 16777216.f;   // 2^24
 
 // OCC: workgroups resident per CU (the two sums of a 32 x 128 wave tile are 128 registers).
 template <int FM_, int FN_, int NWM_, int OCC_>
@@ -216,7 +222,12 @@ __global__ void __launch_bounds__(T::NT, (T::OCC * T::NWM + 3) / 4) gemm_parts_k
     };
     constexpr int SPLITS = 12 * FM;   // part u / 4 % 3 of value pair u % 4 of row block u / 12
     auto split = [&](uint32x4 (&part)[FM][3], int u) {
-      part[u / 12][u / 4 % 3][u % 4] = take_part(v[u / 12][2 * (u % 4)], v[u / 12][2 * (u % 4) + 1]);
+      float &x = v[u / 12][2 * (u % 4)], &y = v[u / 12][2 * (u % 4) + 1];
+      if (u / 4 % 3 == 0) {
+        x *= PARTS_SCALE;
+        y *= PARTS_SCALE;
+      }
+      part[u / 12][u / 4 % 3][u % 4] = take_part(x, y);
     };
     copy_a(0, 0);
     copy_b(0, 0);
@@ -313,13 +324,13 @@ __global__ void __launch_bounds__(T::NT, (T::OCC * T::NWM + 3) / 4) gemm_parts_k
         for (int i = 0; i < FM; ++i) av[i] = k < K ? arow[i][k] : 0.f;
 #pragma unroll
         for (int j = 0; j < FN; ++j) {
-          // the fp32 value again: the sum of its parts, which is exact
+          // the fp32 value again: the sum of its parts, which is exact, or its bits
           const int blk = j < fn_act ? j : fn_act - 1;
           const uint16_t* src = reinterpret_cast<const uint16_t*>(b_base + ((int64_t)blk * nk + kt) * PARTS_BLOCK) +
                                 8 * lane + e;
-          const float x0 = __uint_as_float((uint32_t)src[0] << 16), x1 = __uint_as_float((uint32_t)src[512] << 16),
-                      x2 = __uint_as_float((uint32_t)src[1024] << 16);
-          bv[j] = (x0 + x1) + x2;
+          const uint32_t q0 = src[0], q1 = src[512], q2 = src[1024];
+          const float x0 = __uint_as_float(q0 << 16), x1 = __uint_as_float(q1 << 16), x2 = __uint_as_float(q2 << 16);
+          bv[j] = q0 == PARTS_RAW ? __uint_as_float(q1 << 16 | q2) : ((x0 + x1) + x2) * (1.f / PARTS_SCALE);
         }
 #pragma unroll
         for (int i = 0; i < FM; ++i)
@@ -327,6 +338,13 @@ __global__ void __launch_bounds__(T::NT, (T::OCC * T::NWM + 3) / 4) gemm_parts_k
           for (int j = 0; j < FN; ++j)
             acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[i], bv[j], acc[i][j], 0, 0, 0);
       }
+  } else {
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < FN; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[i][j][r] *= 1.f / (PARTS_SCALE * PARTS_SCALE);
   }
   __syncthreads();   // every wave is done with the stages before an epilogue reuses them
   parts_epilogue<EPI, T, SMEM>(p, acc, smem_ab, red, m0, n0, tile_n, wave, 0, lane, z, lower);

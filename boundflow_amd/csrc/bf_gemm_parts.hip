@@ -18,11 +18,10 @@ struct PackSegs {
   int count;
 };
 
-// One thread per lane of a column block and stage: its eight values of B, split and written as the
-// MFMA operands of the three parts.  Unlike the kernels' own split it also takes a value above the
-// largest bf16 (its first part cut, not rounded) and one that is not finite (the value and zeros),
-// so the sum of the parts is the value whatever it is.  A weight is packed once: nothing here is
-// worth more than its one launch (500 x 500: 4 us).
+// One thread per lane of a column block and stage: its eight values of B, split (times PARTS_SCALE, as the
+// kernels split theirs) and written as the MFMA operands of the three parts, or as PARTS_RAW and their bits
+// where the first part is no finite bf16.  A weight is packed once: nothing here is worth more than its one
+// launch (500 x 500: 4 us).
 __global__ void pack_parts_kernel(PackSegs p) {
   int s = 0;
   while (s + 1 < p.count && (int64_t)blockIdx.x >= p.bstart[s + 1]) ++s;
@@ -37,15 +36,21 @@ __global__ void pack_parts_kernel(PackSegs p) {
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
     const int64_t k = k0 + e;
-    float x = n < N && k < K ? (p.trans_b[s] ? B[n * ldb + k] : B[k * ldb + n]) : 0.f;
-    const bool finite = fabsf(x) < __builtin_inff();
+    const float x = n < N && k < K ? (p.trans_b[s] ? B[n * ldb + k] : B[k * ldb + n]) : 0.f;
+    float left = x * PARTS_SCALE;
+    uint32_t bits[3];
 #pragma unroll
     for (int q = 0; q < 3; ++q) {
-      uint32_t bits = __builtin_bit_cast(uint16_t, (__bf16)x);
-      if ((bits & 0x7fff) == 0x7f80 && finite) bits = __float_as_uint(x) >> 16;
-      x = finite ? x - __uint_as_float(bits << 16) : 0.f;
-      part[q][e / 2] = e & 1 ? part[q][e / 2] | bits << 16 : bits;
+      bits[q] = __builtin_bit_cast(uint16_t, (__bf16)left);
+      left -= __uint_as_float(bits[q] << 16);
     }
+    if ((bits[0] & 0x7fff) >= 0x7f80) {
+      bits[0] = PARTS_RAW;
+      bits[1] = __float_as_uint(x) >> 16;
+      bits[2] = __float_as_uint(x) & 0xffff;
+    }
+#pragma unroll
+    for (int q = 0; q < 3; ++q) part[q][e / 2] = e & 1 ? part[q][e / 2] | bits[q] << 16 : bits[q];
   }
 #pragma unroll
   for (int q = 0; q < 3; ++q) p.out[s][(i >> 6) * 192 + 64 * q + lane] = part[q];

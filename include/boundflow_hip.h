@@ -52,7 +52,7 @@ const char* bf_last_error(void);
 int bf_gemm_tile_config(int64_t M, int64_t N, int nz, int ksplit, int relax_prologue, int dl_operands);
 
 /* Contractions on the bf16 matrix cores.  A weight packed by bf_gemm_pack_parts (every
- * value as three bf16 parts whose sum is the value, in the matrix operand order) serves
+ * value as three bf16 parts whose sum is 2^24 times it, or whole, in the matrix operand order) serves
  * contractions at fp32 accuracy at more than the fp32 MFMA rate: the *_parts entry points
  * below, each the arithmetic of its namesake with the products of the parts down to
  * 2^-32 of a product, summed in fp32 (the leading ones apart from the others).

@@ -294,6 +294,31 @@ def test_operands_that_are_not_finite(M, N, K):
     assert bool((err[rest] <= 1e-4 * want.double().abs()[rest]).all())
 
 
+# powers of two on A and on B: subnormal values and those whose third bf16 part would be, on either side;
+# values past 2^103 and sums past 2^79, which the tiles compute again
+@gpu
+@pytest.mark.parametrize("a_exp,b_exp", [(-118, 100), (-140, 120), (100, -118), (120, -140), (-60, -80), (-110, -16),
+                                         (104, -90), (-90, 104), (50, 40), (-126, 102), (123, -146)])
+@pytest.mark.parametrize("M,N,K", [(36864, 256, 64), (2304, 97, 50)])   # both tiles, both copies
+def test_operands_of_any_size_keep_their_bits(a_exp, b_exp, M, N, K):
+    dev = device()
+    announce(f"parts operands of 2^{a_exp} and 2^{b_exp} M={M} N={N} K={K}")
+    g = gen(M, N, K, abs(a_exp), abs(b_exp))
+    scale = lambda t, e: (t.double() * 2.0 ** e).float()   # noqa: E731
+    A, B = scale(torch.randn(M, K, generator=g), a_exp), scale(torch.randn(N, K, generator=g), b_exp)
+    Ad, Bd = A.to(dev), B.to(dev)
+    C, C32 = torch.empty(M, N, device=dev), torch.empty(M, N, device=dev)
+    _lib.call("bf_gemm_rank1_parts", _lib.ptr(Ad), K, _lib.ptr(pack(Bd, True)), _lib.ptr(C), N, M, N, K, 9, None, None,
+              0, _lib.stream_handle())
+    _lib.call("bf_gemm", _lib.ptr(Ad), K, _lib.ptr(Bd), K, 1, 0, _lib.ptr(C32), N, M, N, K, _lib.stream_handle())
+    torch.cuda.synchronize()
+    # (float64 of the scaled products: past float32's range at either end they would be neither's)
+    ref = (A.double() * 2.0 ** -a_exp) @ (B.double() * 2.0 ** -b_exp).t()
+    err, err32 = (float((c.cpu().double() * 2.0 ** -(a_exp + b_exp) - ref).norm() / ref.norm()) for c in (C, C32))
+    announce(f"parts error {err:.4e}, fp32 tiles {err32:.4e}")
+    assert err <= err32 * (1 + 2.0 ** -6)
+
+
 @gpu
 def test_unaligned_rows_and_refused_shapes():
     dev = device()
