@@ -84,14 +84,6 @@ __device__ __forceinline__ uint32_t take_part(float& x, float& y) {
   return pk;
 }
 
-// Eight values -> their three parts as MFMA operands.
-__device__ __forceinline__ void split_parts(float (&v)[8], uint32x4 (&part)[3]) {
-#pragma unroll
-  for (int q = 0; q < 3; ++q)
-#pragma unroll
-    for (int e = 0; e < 4; ++e) part[q][e] = take_part(v[2 * e], v[2 * e + 1]);
-}
-
 // VEC: coefficient rows of whole 16-byte aligned float4s; else they are copied float by float (a row
 // length that is no multiple of four), the same stage in four times as many copies.
 template <int EPI, class T, bool VEC>

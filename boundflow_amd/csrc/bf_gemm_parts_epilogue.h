@@ -182,10 +182,9 @@ __device__ __forceinline__ void parts_epilogue(const GemmArgs& p, floatx16 (&acc
     // it is stored, so the next contraction reads A' directly; every coefficient
     // is relaxed once here instead of once per column tile of its consumer.
     static_assert(GBN == NORM_BN, "the relaxation epilogue needs BN == NORM_BN");
-    // As / Bs are free once every wave has left the main loop: As holds the
-    // relaxation entries of the tile's domains x columns, Bs the split term,
-    // the center vector, the bias and the domain of each row.
-    // per (domain, column) entry: the float4 relaxation, the split term and the center
+    // smem_ab, free by now, holds an entry per domain and column of the tile: the float4 relaxations of all
+    // of them (Te), then the split terms (Ae), then the centers (Ce).  The bias of a column (Ke) and the
+    // domain of a row (Re) have arrays of their own.
     constexpr int E_DOMS = SMEM / (6 * GBN);
     __shared__ float Ke[GBN];
     __shared__ int Re[GBM];
