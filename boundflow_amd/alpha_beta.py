@@ -32,7 +32,6 @@ import torch
 
 from . import _lib
 from .crown import (
-    STORE,
     Chain,
     ForwardTrace,
     _broadcast_split,
@@ -43,7 +42,7 @@ from .crown import (
     forward_ibp_trace,
     NotAChain,
     parse_chain,
-    takes_parts,
+    reverse_takes_parts,
     weight_parts,
 )
 from .profiling import launch as _timed
@@ -217,15 +216,14 @@ def _grad_pass(spec: InputSpec, chain: Chain, trace: ForwardTrace, saved: dict, 
         gt = torch.empty(M, n_out, device=dev)
         if layer.kind == "linear":
             rank1 = (_lib.ptr(G if vec is not None else None), _lib.ptr(vec), vec_ld)
-            wsz = int(_lib.load().bf_gemm_rank1_workspace(M, n_out, n_in))
-            # (a contraction the fp32 kernels split over K keeps the split)
-            packed = not wsz and takes_parts(STORE, M, n_out, n_in, S, 1)
+            packed = reverse_takes_parts(M, n_out, n_in, S)
             with _timed("grad_gemm_parts" if packed else "grad_gemm", 2.0 * M * n_in * n_out,
                         4.0 * (M * n_in + M * n_out + n_in * n_out)):
                 if packed:
                     _lib.call("bf_gemm_rank1_parts", _lib.ptr(g), n_in, _lib.ptr(weight_parts(layer.weight, True)),
                               _lib.ptr(gt), n_out, M, n_out, n_in, S, *rank1, stream)
                 else:
+                    wsz = int(_lib.load().bf_gemm_rank1_workspace(M, n_out, n_in))
                     ws = torch.empty(wsz, device=dev) if wsz else None
                     _lib.call("bf_gemm_rank1", _lib.ptr(g), n_in, _lib.ptr(layer.weight.contiguous()), n_in, 1,
                               _lib.ptr(gt), n_out, M, n_out, n_in, S, *rank1, _lib.ptr(ws), wsz, stream)

@@ -197,21 +197,27 @@ def _pack(todo) -> List[torch.Tensor]:
     return outs
 
 
-def chain_parts(layers: List[AffineLayer], layer: AffineLayer, M: int, S: int, nz: int, save: Optional[dict],
-                trans_b: bool = False) -> torch.Tensor:
-    """``weight_parts`` of a chain's linear layer; when it is not kept yet, with those of the
-    other layers the query will read: the backward's, and with a gradient to follow the reverse
-    pass's."""
+def chain_parts(layers: List[AffineLayer], k: int, M: int, S: int, nz: int, save: Optional[dict]) -> torch.Tensor:
+    """``weight_parts`` of layer ``k`` of a chain; when it is not kept yet, with those of what the
+    query will read after it: the layers below, as the backward contracts them, and with a
+    gradient to follow the reverse pass's."""
     def also():
-        for k, other in enumerate(layers):
+        for j, other in enumerate(layers[:k]):
             if other.kind != "linear":
                 continue
-            n, p = _numel(other.out_shape), _numel(other.in_shape)
-            if takes_parts(CONCRETIZE if k == 0 else STORE, M, p, n, S, nz):
+            form = CONCRETIZE if j == 0 else RELAX if relaxes_in_epilogue(layers, j, M, S) else STORE
+            if takes_parts(form, M, _numel(other.in_shape), _numel(other.out_shape), S, nz):
                 yield other.weight, False
-            if save is not None and save.get("grad_rows") is not None and takes_parts(STORE, M, n, p, S, 1):
-                yield other.weight, True
-    return weight_parts(layer.weight, trans_b, also())
+        if save is not None and save.get("grad_rows") is not None:
+            for other in layers[:-1]:
+                if other.kind == "linear" and reverse_takes_parts(M, _numel(other.out_shape), _numel(other.in_shape), S):
+                    yield other.weight, True
+    return weight_parts(layers[k].weight, False, also())
+
+
+def relaxes_in_epilogue(layers: List[AffineLayer], k: int, M: int, S: int) -> bool:
+    """Whether the contraction of layer ``k`` (not the input layer) relaxes its result for the layer below."""
+    return layers[k - 1].kind == "linear" and S >= EPILOGUE_MIN_ROWS and M >= EPILOGUE_MIN_M
 
 
 # forms of a contraction on packed parts (bf_gemm_parts_config)
@@ -224,6 +230,12 @@ def takes_parts(form: int, M: int, N: int, K: int, S: int, nz: int) -> bool:
     if K < 16 or M < 256:   # (most small queries end here, without a call into the library)
         return False
     return _parts_rule(M, N, K, S, nz, form)
+
+
+def reverse_takes_parts(M: int, N: int, K: int, S: int) -> bool:
+    """Whether the reverse pass's contraction of M rows of K values into N (bf_gemm_rank1) runs on packed
+    weight parts: one that the fp32 kernels split over K keeps the split."""
+    return takes_parts(STORE, M, N, K, S, 1) and not _lib.load().bf_gemm_rank1_workspace(M, N, K)
 
 
 @functools.lru_cache(maxsize=4096)
@@ -743,7 +755,7 @@ def crown_backward(
                         4.0 * nz * (M * N + N * P + M * -(-P // 128)) + (4.0 * M * P if h_out is not None else 0.0)):
                 _lib.call("bf_crown_linear_concretize_parts" if in_parts else "bf_crown_linear_concretize",
                           _lib.ptr(A_u), _lib.ptr(A_l), stride, B, S, N,
-                          _lib.ptr(chain_parts(layers, layer, M, S, nz, save) if in_parts else transposed(W)), P, _lib.ptr(rad), eps, input_norm_p(pert), _lib.ptr(c_u), _lib.ptr(c_l), _lib.ptr(b_u),
+                          _lib.ptr(chain_parts(layers, k, M, S, nz, save) if in_parts else transposed(W)), P, _lib.ptr(rad), eps, input_norm_p(pert), _lib.ptr(c_u), _lib.ptr(c_l), _lib.ptr(b_u),
                           _lib.ptr(b_l),
                           _lib.ptr(h_scale), _lib.ptr(h_out), _lib.ptr(ws), _lib.ptr(lb), _lib.ptr(ub), stream)
             if save is not None:
@@ -798,7 +810,7 @@ def crown_backward(
         # next region then relaxes the kept product in a pass of its own.
         head_memo = (k == len(layers) - 1 and relax is None and add is None and save is not None
                      and save.get("memo") is not None and torch.is_tensor(linear_spec_C))
-        if not head_memo and layers[k - 1].kind == "linear" and S >= EPILOGUE_MIN_ROWS and M >= EPILOGUE_MIN_M:
+        if not head_memo and relaxes_in_epilogue(layers, k, M, S):
             # the next region's relaxation in this contraction's epilogue
             n_alpha, n_alpha_ld, n_add, n_add_ld, _, _, _ = relax_params(k - 1)
             n_table = relax_table(k - 1)
@@ -831,7 +843,7 @@ def crown_backward(
                          _lib.ptr(nb_u), _lib.ptr(nb_l), _lib.ptr(nc_u), _lib.ptr(nc_l), stream)
                 if packed:
                     _lib.call("bf_crown_linear_relu_fwd_parts", _lib.ptr(A_u), _lib.ptr(A_l), stride, B, S, N,
-                              _lib.ptr(chain_parts(layers, layer, M, S, nz, save)), P, *after)
+                              _lib.ptr(chain_parts(layers, k, M, S, nz, save)), P, *after)
                 else:
                     _lib.call("bf_crown_relu_linear_relu_fwd", _lib.ptr(A_u), _lib.ptr(A_l), stride, B, S, N,
                               _lib.ptr(relax), _lib.ptr(add), add_ld, _lib.ptr(transposed(W)), P, _lib.ptr(bias),
@@ -864,7 +876,7 @@ def crown_backward(
                 with _timed("crown_linear_parts" if packed else "crown_relu_linear_fwd", flops, nbytes):
                     if packed:
                         _lib.call("bf_crown_linear_parts", _lib.ptr(A_u), _lib.ptr(A_l), stride, B, S, N,
-                                  _lib.ptr(chain_parts(layers, layer, M, S, nz, save)), P, *rows)
+                                  _lib.ptr(chain_parts(layers, k, M, S, nz, save)), P, *rows)
                     else:
                         _lib.call("bf_crown_relu_linear_fwd", _lib.ptr(A_u), _lib.ptr(A_l), stride, B, S, N,
                                   _lib.ptr(relax), _lib.ptr(add), add_ld, _lib.ptr(transposed(W)), P, 1, *rows)

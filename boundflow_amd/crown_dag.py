@@ -714,7 +714,7 @@ def lower_grad_pass(module: BFTaskModule, spec: InputSpec, trace: DagTrace, save
     G bias^T; relu through the relaxation (bf_relu_grad, which also reduces dL/dalpha and
     dL/dbeta); add the sum of its operands' gradients (plus G c^T for a constant c);
     concat the concatenation of its operands' gradients; flatten/reshape the same rows."""
-    from .crown import STORE, takes_parts, weight_parts
+    from .crown import reverse_takes_parts, weight_parts
 
     task = _module_task(module)
     params = module.params
@@ -746,9 +746,7 @@ def lower_grad_pass(module: BFTaskModule, spec: InputSpec, trace: DagTrace, save
             n_out, n_in = int(W.shape[0]), int(W.shape[1])
             gt = torch.empty(M, n_out, device=dev)
             rank1 = (_lib.ptr(G if bias is not None else None), _lib.ptr(bias), 0)
-            wsz = int(_lib.load().bf_gemm_rank1_workspace(M, n_out, n_in))
-            # (a contraction the fp32 kernels split over K keeps the split)
-            packed = not wsz and takes_parts(STORE, M, n_out, n_in, S, 1)
+            packed = reverse_takes_parts(M, n_out, n_in, S)
             with _timed("grad_gemm_parts" if packed else "grad_gemm", 2.0 * M * n_in * n_out,
                         4.0 * (M * n_in + M * n_out + n_in * n_out)):
                 if packed:
@@ -756,6 +754,7 @@ def lower_grad_pass(module: BFTaskModule, spec: InputSpec, trace: DagTrace, save
                               _lib.ptr(weight_parts(params[op.inputs[1]], True)), _lib.ptr(gt), n_out, M, n_out, n_in,
                               S, *rank1, stream)
                 else:
+                    wsz = int(_lib.load().bf_gemm_rank1_workspace(M, n_out, n_in))
                     ws = torch.empty(wsz, device=dev) if wsz else None
                     _lib.call("bf_gemm_rank1", _lib.ptr(GA[x]), n_in, _lib.ptr(W), n_in, 1, _lib.ptr(gt), n_out, M,
                               n_out, n_in, S, *rank1, _lib.ptr(ws), wsz, stream)
