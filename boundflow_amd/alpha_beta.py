@@ -217,16 +217,17 @@ def _grad_pass(spec: InputSpec, chain: Chain, trace: ForwardTrace, saved: dict, 
         if layer.kind == "linear":
             rank1 = (_lib.ptr(G if vec is not None else None), _lib.ptr(vec), vec_ld)
             packed = reverse_takes_parts(M, n_out, n_in, S)
+            weight = weight_parts(layer.weight, True) if packed else layer.weight.contiguous()
             with _timed("grad_gemm_parts" if packed else "grad_gemm", 2.0 * M * n_in * n_out,
                         4.0 * (M * n_in + M * n_out + n_in * n_out)):
                 if packed:
-                    _lib.call("bf_gemm_rank1_parts", _lib.ptr(g), n_in, _lib.ptr(weight_parts(layer.weight, True)),
-                              _lib.ptr(gt), n_out, M, n_out, n_in, S, *rank1, stream)
+                    _lib.call("bf_gemm_rank1_parts", _lib.ptr(g), n_in, _lib.ptr(weight), _lib.ptr(gt), n_out, M, n_out,
+                              n_in, S, *rank1, stream)
                 else:
                     wsz = int(_lib.load().bf_gemm_rank1_workspace(M, n_out, n_in))
                     ws = torch.empty(wsz, device=dev) if wsz else None
-                    _lib.call("bf_gemm_rank1", _lib.ptr(g), n_in, _lib.ptr(layer.weight.contiguous()), n_in, 1,
-                              _lib.ptr(gt), n_out, M, n_out, n_in, S, *rank1, _lib.ptr(ws), wsz, stream)
+                    _lib.call("bf_gemm_rank1", _lib.ptr(g), n_in, _lib.ptr(weight), n_in, 1, _lib.ptr(gt), n_out, M,
+                              n_out, n_in, S, *rank1, _lib.ptr(ws), wsz, stream)
         else:
             Ci, Hi, Wi = layer.in_shape
             Co, Ho, Wo = layer.out_shape

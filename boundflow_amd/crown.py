@@ -749,14 +749,14 @@ def crown_backward(
                 save["cvec"] = trace.input_center_proj.get(layer.out_name)
             nz = int(A_u is not None) + int(A_l is not None)
             in_parts = takes_parts(CONCRETIZE, M, P, N, S, nz)
+            weight = chain_parts(layers, k, M, S, nz, save) if in_parts else transposed(W)
             # bytes: the coefficient rows and the weight read, the row partial norms written, the
             # gradient seed [M, P] written when asked
             with _timed("crown_linear_concretize_parts" if in_parts else "crown_linear_concretize", 2.0 * nz * M * N * P,
                         4.0 * nz * (M * N + N * P + M * -(-P // 128)) + (4.0 * M * P if h_out is not None else 0.0)):
                 _lib.call("bf_crown_linear_concretize_parts" if in_parts else "bf_crown_linear_concretize",
-                          _lib.ptr(A_u), _lib.ptr(A_l), stride, B, S, N,
-                          _lib.ptr(chain_parts(layers, k, M, S, nz, save) if in_parts else transposed(W)), P, _lib.ptr(rad), eps, input_norm_p(pert), _lib.ptr(c_u), _lib.ptr(c_l), _lib.ptr(b_u),
-                          _lib.ptr(b_l),
+                          _lib.ptr(A_u), _lib.ptr(A_l), stride, B, S, N, _lib.ptr(weight), P, _lib.ptr(rad), eps,
+                          input_norm_p(pert), _lib.ptr(c_u), _lib.ptr(c_l), _lib.ptr(b_u), _lib.ptr(b_l),
                           _lib.ptr(h_scale), _lib.ptr(h_out), _lib.ptr(ws), _lib.ptr(lb), _lib.ptr(ub), stream)
             if save is not None:
                 save["final_ws"] = ws
@@ -789,10 +789,9 @@ def crown_backward(
             with _timed("crown_relu_linear_concretize", 2.0 * nz * M * N * P,
                         4.0 * nz * (M * N + N * P) + 16.0 * B * N + (4.0 * M * P if h_out is not None else 0.0)):
                 _lib.call("bf_crown_relu_linear_concretize", _lib.ptr(A_u), _lib.ptr(A_l), stride, B, S, N,
-                          _lib.ptr(relax), _lib.ptr(add), add_ld, _lib.ptr(transposed(W)), P, 1, _lib.ptr(bias), _lib.ptr(cvec),
-                          _lib.ptr(rad), eps, input_norm_p(pert), _lib.ptr(b_u),
-                          _lib.ptr(b_l), _lib.ptr(h_scale), _lib.ptr(h_out), _lib.ptr(ws), _lib.ptr(lb),
-                          _lib.ptr(ub), stream)
+                          _lib.ptr(relax), _lib.ptr(add), add_ld, _lib.ptr(transposed(W)), P, 1, _lib.ptr(bias),
+                          _lib.ptr(cvec), _lib.ptr(rad), eps, input_norm_p(pert), _lib.ptr(b_u), _lib.ptr(b_l),
+                          _lib.ptr(h_scale), _lib.ptr(h_out), _lib.ptr(ws), _lib.ptr(lb), _lib.ptr(ub), stream)
             if save is not None:
                 save["final_ws"] = ws
             return IntervalState(lower=lb, upper=ub)
@@ -836,6 +835,7 @@ def crown_backward(
                        + (4.0 * B * P if cvec is not None else 0.0)
                        + 4.0 * nz * M * -(-P // 128) * (2 if cvec is not None else 1))
             packed = plain and takes_parts(RELAX, M, P, N, S, nz)
+            weight = chain_parts(layers, k, M, S, nz, save) if packed else transposed(W)
             with _timed("crown_linear_relu_fwd_parts" if packed else "crown_relu_linear_relu_fwd", flops,
                         nbytes + e_bytes + (4.0 * M * P if pre_l is not None else 0.0)):
                 after = (_lib.ptr(b_u), _lib.ptr(b_l), _lib.ptr(n_table), _lib.ptr(n_add), n_add_ld, _lib.ptr(n_bias),
@@ -843,11 +843,10 @@ def crown_backward(
                          _lib.ptr(nb_u), _lib.ptr(nb_l), _lib.ptr(nc_u), _lib.ptr(nc_l), stream)
                 if packed:
                     _lib.call("bf_crown_linear_relu_fwd_parts", _lib.ptr(A_u), _lib.ptr(A_l), stride, B, S, N,
-                              _lib.ptr(chain_parts(layers, k, M, S, nz, save)), P, *after)
+                              _lib.ptr(weight), P, *after)
                 else:
                     _lib.call("bf_crown_relu_linear_relu_fwd", _lib.ptr(A_u), _lib.ptr(A_l), stride, B, S, N,
-                              _lib.ptr(relax), _lib.ptr(add), add_ld, _lib.ptr(transposed(W)), P, _lib.ptr(bias),
-                              *after)
+                              _lib.ptr(relax), _lib.ptr(add), add_ld, _lib.ptr(weight), P, _lib.ptr(bias), *after)
             if pre_l is not None:
                 save.setdefault("A_in", {})[k - 1] = (pre_l, S * P)
                 save.setdefault("b_in", {})[k - 1] = nb_l
@@ -873,13 +872,14 @@ def crown_backward(
                         _lib.ptr(nA_u), _lib.ptr(nA_l), None if keep_b else _lib.ptr(nb_u),
                         None if keep_b else _lib.ptr(nb_l), stream)
                 packed = plain and takes_parts(STORE, M, P, N, S, nz)
+                weight = chain_parts(layers, k, M, S, nz, save) if packed else transposed(W)
                 with _timed("crown_linear_parts" if packed else "crown_relu_linear_fwd", flops, nbytes):
                     if packed:
                         _lib.call("bf_crown_linear_parts", _lib.ptr(A_u), _lib.ptr(A_l), stride, B, S, N,
-                                  _lib.ptr(chain_parts(layers, k, M, S, nz, save)), P, *rows)
+                                  _lib.ptr(weight), P, *rows)
                     else:
                         _lib.call("bf_crown_relu_linear_fwd", _lib.ptr(A_u), _lib.ptr(A_l), stride, B, S, N,
-                                  _lib.ptr(relax), _lib.ptr(add), add_ld, _lib.ptr(transposed(W)), P, 1, *rows)
+                                  _lib.ptr(relax), _lib.ptr(add), add_ld, _lib.ptr(weight), P, 1, *rows)
                 if head_key is not None:
                     save["memo"][head_key] = (nA_u, nA_l, nb_u, nb_l)
             pre_relaxed = False

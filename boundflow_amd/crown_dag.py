@@ -539,6 +539,8 @@ def crown_backward_dag(
             A_l_in = None if one else st.A_l
             nz = int(st.A_u is not None) + int(A_l_in is not None)
             packed = takes_parts(STORE, M, P, N, S, nz)
+            # (unpacked, the contraction reads W^T [P, N]: 128-bit operand loads along N)
+            weight = weight_parts(params[op.inputs[1]], False) if packed else transposed(W)
             with _timed("crown_linear_parts" if packed else "crown_linear", 2.0 * nz * M * N * P,
                         4.0 * nz * (M * N + N * P + M * P)):
                 out_b = (None, None) if keep_b else (_lib.ptr(nb_u), _lib.ptr(None if one else nb_l))
@@ -547,11 +549,10 @@ def crown_backward_dag(
                         _lib.ptr(None if one else nA_l), *out_b, stream)
                 if packed:
                     _lib.call("bf_crown_linear_parts", _lib.ptr(st.A_u), _lib.ptr(A_l_in), S * N, B, S, N,
-                              _lib.ptr(weight_parts(params[op.inputs[1]], False)), P, *rows)
+                              _lib.ptr(weight), P, *rows)
                 else:
-                    # the contraction reads W^T [P, N]: 128-bit operand loads along N
                     _lib.call("bf_crown_relu_linear_fwd", _lib.ptr(st.A_u), _lib.ptr(A_l_in), S * N, B, S, N, None,
-                              None, 0, _lib.ptr(transposed(W)), P, 1, *rows)
+                              None, 0, _lib.ptr(weight), P, 1, *rows)
             accumulate(x, _Rows(nA_u, nA_l, nb_u, nb_l))
         elif t == "conv2d":
             W = params[op.inputs[1]].contiguous()
@@ -747,16 +748,16 @@ def lower_grad_pass(module: BFTaskModule, spec: InputSpec, trace: DagTrace, save
             gt = torch.empty(M, n_out, device=dev)
             rank1 = (_lib.ptr(G if bias is not None else None), _lib.ptr(bias), 0)
             packed = reverse_takes_parts(M, n_out, n_in, S)
+            weight = weight_parts(params[op.inputs[1]], True) if packed else W
             with _timed("grad_gemm_parts" if packed else "grad_gemm", 2.0 * M * n_in * n_out,
                         4.0 * (M * n_in + M * n_out + n_in * n_out)):
                 if packed:
-                    _lib.call("bf_gemm_rank1_parts", _lib.ptr(GA[x]), n_in,
-                              _lib.ptr(weight_parts(params[op.inputs[1]], True)), _lib.ptr(gt), n_out, M, n_out, n_in,
-                              S, *rank1, stream)
+                    _lib.call("bf_gemm_rank1_parts", _lib.ptr(GA[x]), n_in, _lib.ptr(weight), _lib.ptr(gt), n_out, M,
+                              n_out, n_in, S, *rank1, stream)
                 else:
                     wsz = int(_lib.load().bf_gemm_rank1_workspace(M, n_out, n_in))
                     ws = torch.empty(wsz, device=dev) if wsz else None
-                    _lib.call("bf_gemm_rank1", _lib.ptr(GA[x]), n_in, _lib.ptr(W), n_in, 1, _lib.ptr(gt), n_out, M,
+                    _lib.call("bf_gemm_rank1", _lib.ptr(GA[x]), n_in, _lib.ptr(weight), n_in, 1, _lib.ptr(gt), n_out, M,
                               n_out, n_in, S, *rank1, _lib.ptr(ws), wsz, stream)
             GA[y] = gt
         elif t == "conv2d":

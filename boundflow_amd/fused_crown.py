@@ -285,6 +285,8 @@ class HipFusedCrownExecutor:
             with _timed("executor_relax_table", 0.0, 4.0 * 8 * D * N):
                 _lib.call("bf_relu_relax_table_from_planes", *[_lib.ptr(t) for t in planes], D * N, _lib.ptr(table), st)
             packed = takes_parts(STORE, M, P, N, S, 2)
+            # (unpacked: W^T [P, N], the kernel's faster operand layout, kept across calls)
+            weight = weight_parts(request.weight, False) if packed else transposed(request.weight)
             if packed or (M < EPILOGUE_MIN_M and N >= RELAX_PASS_MIN_K):
                 # the relaxation pass, then the plain contraction: on the packed weight, or, for a
                 # region of few rows, as 64 x 64 tiles that spread the short grid over more CUs (as
@@ -300,16 +302,15 @@ class HipFusedCrownExecutor:
                     rows = (None, None, None, _lib.ptr(pu), _lib.ptr(pl), None, None, st)
                     if packed:
                         _lib.call("bf_crown_linear_parts", _lib.ptr(ru), _lib.ptr(rl), S * N, D, S, N,
-                                  _lib.ptr(weight_parts(request.weight, False)), P, *rows)
+                                  _lib.ptr(weight), P, *rows)
                     else:
-                        # W^T [P, N]: the kernel's faster operand layout, kept across calls
                         _lib.call("bf_crown_relu_linear_fwd", _lib.ptr(ru), _lib.ptr(rl), S * N, D, S, N, None, None,
-                                  0, _lib.ptr(transposed(request.weight)), P, 1, *rows)
+                                  0, _lib.ptr(weight), P, 1, *rows)
                 return FusedReluAffineResult(pu, pl, du, dl)
             with _timed("executor_relu_linear", 4.0 * M * N * P, 4.0 * (2 * M * N + 4 * D * N + N * P + 2 * M * P)):
                 _lib.call("bf_crown_relu_linear_fwd", _lib.ptr(request.A_u), _lib.ptr(request.A_l), S * N, D, S, N,
-                          _lib.ptr(table), None, 0, _lib.ptr(transposed(request.weight)), P, 1, _lib.ptr(bias), None, None,
-                          _lib.ptr(pu), _lib.ptr(pl), _lib.ptr(du), _lib.ptr(dl), st)
+                          _lib.ptr(table), None, 0, _lib.ptr(weight), P, 1, _lib.ptr(bias), None, None, _lib.ptr(pu),
+                          _lib.ptr(pl), _lib.ptr(du), _lib.ptr(dl), st)
             return FusedReluAffineResult(pu, pl, du, dl)
         Co, Ho, Wo = (int(d) for d in request.output_shape)
         Ci, Hi, Wi = (int(d) for d in request.input_shape)
