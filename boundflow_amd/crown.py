@@ -50,6 +50,12 @@ from .spec import BoxPerturbation, InputSpec, IntervalState, LpBallPerturbation,
 
 _DERIVED: "OrderedDict[tuple, tuple]" = OrderedDict()
 _DERIVED_MAX = 192   # a layer keeps up to three: its transpose and its packed parts either way
+# an entry holds its operand and its sources: what they may come to (packed parts are 1.5 times their
+# weight; callers that pass fresh weights leave old ones here)
+_DERIVED_BYTES = 16 << 30
+_HELD: Dict[tuple, tuple] = {}   # key -> (bytes, the keys that share one buffer with it)
+_held_bytes = 0                  # their sum
+_LOCK = threading.RLock()        # of the three
 _SCOPE = threading.local()
 
 
@@ -60,10 +66,12 @@ def derived(tag: str, sources: Tuple[torch.Tensor, ...], make: Callable[[], torc
     queries skip the copy.  Operands that depend on a query's inputs are never kept here.
 
     * The entry keeps its sources alive, so their storage cannot be reused under the same
-      key; at most ``_DERIVED_MAX`` entries are kept.  A change written through ``tensor.data`` does not
+      key; at most ``_DERIVED_MAX`` entries of ``_DERIVED_BYTES`` are kept, the oldest go
+      first.  A change written through ``tensor.data`` does not
       bump the version and is not seen: change parameters through the tensor itself.
     * A hit on another stream than the one that made the entry waits for the producer
-      (an event recorded after ``make()``), so the consumer never reads it half-written.
+      (an event recorded after ``make()``), so the consumer never reads it half-written, and
+      keeps the allocator from reusing an entry dropped meanwhile before it is read.
     * Inside ``derived_scope()`` (graph capture) entries live in the scope's own dict,
       which the captured query keeps: a replay never reads an entry the process-wide
       cache has since evicted, and ``refresh_scope`` remakes (in place, before a replay)
@@ -77,31 +85,57 @@ def derived(tag: str, sources: Tuple[torch.Tensor, ...], make: Callable[[], torc
 
 def _kept(tag: str, sources: Tuple[torch.Tensor, ...]) -> Optional[torch.Tensor]:
     scope = getattr(_SCOPE, "memo", None)
-    table = _DERIVED if scope is None else scope
     key = (tag,) + tuple(id(t) for t in sources)
-    hit = table.get(key)
-    if hit is None or hit[1] != tuple(t._version for t in sources) or not all(a is b for a, b in zip(hit[0], sources)):
-        return None
-    if scope is None:
-        _DERIVED.move_to_end(key)
-        out, stream, event = hit[2]
-        if event is not None and _lib.current_raw_stream(out.device.index) != stream.cuda_stream:
-            torch.cuda.current_stream(out.device).wait_event(event)
-        return out
-    return hit[2][0]
+    with _LOCK:
+        hit = (_DERIVED if scope is None else scope).get(key)
+        if hit is None or hit[1] != tuple(t._version for t in sources) or not all(
+                a is b for a, b in zip(hit[0], sources)):
+            return None
+        if scope is None:
+            _DERIVED.move_to_end(key)
+    out, stream, event = hit[2]
+    if event is not None and _lib.current_raw_stream(out.device.index) != stream.cuda_stream:
+        here = torch.cuda.current_stream(out.device)
+        here.wait_event(event)
+        out.record_stream(here)
+    return out
 
 
 def _keep(tag: str, sources: Tuple[torch.Tensor, ...], out: torch.Tensor, make: Callable[[], torch.Tensor],
-          made=None) -> None:
-    """Enter ``out``; ``made``: the (stream, event) of a launch that made several entries."""
+          made=None, group=None) -> None:
+    """Enter ``out``; ``made``: the (stream, event) of a launch that made several entries; ``group``: a
+    set for the keys of the entries that lie in one buffer, which are given back together."""
+    global _held_bytes
     scope = getattr(_SCOPE, "memo", None)
-    table = _DERIVED if scope is None else scope
-    stream, event = made or (_made_here(out) if scope is None else (None, None))
     key = (tag,) + tuple(id(t) for t in sources)
     versions = tuple(t._version for t in sources)
-    table[key] = (tuple(sources), versions, (out, stream, event), make if scope is not None else None)
-    if scope is None and len(_DERIVED) > _DERIVED_MAX:
-        _DERIVED.popitem(last=False)
+    if scope is not None:
+        scope[key] = (tuple(sources), versions, (out, None, None), make)
+        return
+    entry = (tuple(sources), versions, (out, *(made or _made_here(out))), None)
+    group = {key} if group is None else group
+    with _LOCK:
+        if key in _DERIVED:
+            _drop(key)
+        group.add(key)
+        _DERIVED[key] = entry
+        nbytes = sum(t.numel() * t.element_size() for t in (out, *sources))
+        _HELD[key] = (nbytes, group)
+        _held_bytes += nbytes
+        while len(_DERIVED) > _DERIVED_MAX or _held_bytes > _DERIVED_BYTES:
+            oldest = next(iter(_DERIVED))
+            if oldest in group:   # (this launch's own entries stay, whatever their size)
+                break
+            for other in list(_HELD[oldest][1]):
+                _drop(other)
+
+
+def _drop(key: tuple) -> None:
+    global _held_bytes
+    nbytes, group = _HELD.pop(key)
+    _held_bytes -= nbytes
+    group.discard(key)
+    del _DERIVED[key]
 
 
 def _made_here(out: torch.Tensor):
@@ -176,21 +210,23 @@ def weight_parts(W: torch.Tensor, trans_b: bool, also=()) -> torch.Tensor:
     outs = _pack(todo)
     scope = getattr(_SCOPE, "memo", None)
     made = _made_here(outs[0]) if scope is None else None
+    group: set = set()
     for (w, t), o in zip(todo, outs):
-        _keep(_PARTS[t], (w,), o, lambda w=w, t=t: _pack([(w, t)])[0], made)
+        _keep(_PARTS[t], (w,), o, lambda w=w, t=t: _pack([(w, t)])[0], made, group)
     return outs[0]
 
 
 _PARTS = {False: "parts", True: "parts_t"}
 
 
-def _pack(todo) -> List[torch.Tensor]:
+def _pack(todo) -> Tuple[torch.Tensor, ...]:
     src = [w.contiguous() for w, _t in todo]
     sizes = [(int(w.shape[0]), int(w.shape[1])) for w in src]
     N = [n if t else p for (n, p), (_w, t) in zip(sizes, todo)]
     K = [p if t else n for (n, p), (_w, t) in zip(sizes, todo)]
-    outs = [torch.empty(int(_lib.load().bf_gemm_parts_floats(n, k)), device=w.device, dtype=torch.float32)
-            for n, k, w in zip(N, K, src)]
+    # (one buffer: a new network's first query then asks the device for memory once, not per weight)
+    floats = [int(_lib.load().bf_gemm_parts_floats(n, k)) for n, k in zip(N, K)]
+    outs = torch.empty(sum(floats), device=src[0].device, dtype=torch.float32).split(floats)
     _lib.call("bf_gemm_pack_parts", len(todo), _lib.ptr_array(src), _lib.i64_array([p for _n, p in sizes]),
               _lib.i32_array([int(t) for _w, t in todo]), _lib.i64_array(N), _lib.i64_array(K), _lib.ptr_array(outs),
               _lib.stream_handle())

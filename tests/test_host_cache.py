@@ -44,6 +44,68 @@ def test_cache_is_bounded():
     assert torch.equal(crown.derived("bound_test", (last,), lambda: torch.zeros(1)), last * 2.0)
 
 
+def _entries(tag):
+    return [key for key in crown._DERIVED if key[0] == tag]
+
+
+def test_cache_is_bounded_in_bytes(monkeypatch):
+    """Fresh weights, as a caller of single regions passes them: what the cache holds of them (the operand
+    and the source it pins) stays below the bound, and the oldest go first."""
+    made = [torch.full((256,), float(i)) for i in range(40)]
+    monkeypatch.setattr(crown, "_DERIVED_BYTES", 10 * 2 * 1024)      # ten entries of 1 KB and their sources
+    for t in made:
+        crown.derived("bytes_test", (t,), lambda t=t: t * 2.0)
+    assert crown._held_bytes == sum(n for n, _group in crown._HELD.values()) <= 10 * 2 * 1024
+    assert _entries("bytes_test") == [("bytes_test", id(t)) for t in made[-10:]]
+    assert crown._HELD.keys() == crown._DERIVED.keys()
+    big = torch.ones(1 << 16)
+    assert torch.equal(crown.derived("bytes_test", (big,), lambda: big * 3.0), big * 3.0)   # past the bound by itself
+    assert _entries("bytes_test") == [("bytes_test", id(big))]
+
+
+def test_entries_of_one_buffer_go_together(monkeypatch):
+    """A part of a buffer that stays would hold all of it: the first of its entries to go takes the others."""
+    monkeypatch.setattr(crown, "_DERIVED_MAX", len(crown._DERIVED) + 3)
+    ws = [torch.full((4,), float(i)) for i in range(3)]
+    group = set()
+    for w, part in zip(ws, torch.zeros(12).split(4)):
+        crown._keep("group_test", (w,), part, None, None, group)
+    assert len(_entries("group_test")) == 3
+    assert crown._kept("group_test", (ws[1],)) is not None          # the newest use, which the first does not share
+    ws[2].add_(1.0)                                                  # made again: in no shared buffer any more
+    crown._keep("group_test", (ws[2],), torch.ones(4), None)
+    while ("group_test", id(ws[0])) in crown._DERIVED:
+        t = torch.zeros(1)
+        crown.derived("filler", (t,), lambda: t + 1.0)
+    assert _entries("group_test") == [("group_test", id(ws[2]))]
+    assert crown._HELD.keys() == crown._DERIVED.keys()
+
+
+def test_threads_share_the_cache(monkeypatch):
+    """Hits, entries and evictions from several threads."""
+    import threading
+    monkeypatch.setattr(crown, "_DERIVED_MAX", 4)
+    ws = [torch.full((2,), float(i)) for i in range(8)]
+    failed = []
+
+    def work(seed):
+        try:
+            for i in range(400):
+                w = ws[(i * 7 + seed) % len(ws)]
+                if not torch.equal(crown.derived("thread_test", (w,), lambda: w * 2.0), w * 2.0):
+                    raise AssertionError("another weight's operand")
+        except BaseException as e:   # noqa: BLE001 (reported by the test)
+            failed.append(e)
+
+    threads = [threading.Thread(target=work, args=(s,)) for s in range(6)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not failed, failed[0]
+    assert len(crown._DERIVED) <= 4 and crown._HELD.keys() == crown._DERIVED.keys()
+
+
 def test_scope_keeps_entries_out_of_the_global_cache():
     """Inside derived_scope (graph capture) entries go to the scope's dict: the
     process-wide cache is neither read nor filled, so the captured work makes
