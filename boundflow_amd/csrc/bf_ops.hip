@@ -9,6 +9,7 @@
 
 #include <cstring>
 #include <mutex>
+#include <type_traits>
 
 namespace bf {
 
@@ -576,11 +577,25 @@ ibp_batched_linear_kernel(const float* __restrict__ lo, const float* __restrict_
 // own.  The launches are short of work, not of bandwidth: a residual query of 64 x 10 rows (4 blocks of
 // 512, both bounds) took 449 us with the sums as launches (16 of about 4.3 us) and the affine ops' bias
 // sums as passes (8 of about 5.6 us), 365 us with both inside the relaxation pass; a residual conv
-// net of 16 x 10 rows 431 and 332 us.
+// net of 16 x 10 rows 431 and 332 us.  A pass without one is compiled without it (OneRow): a query of
+// nine rows has three of them in its 67 us, which took 0.5 us more with the tests for it.
 struct RowAddend {
   const float* A[2];   // [M, K] of the upper and the lower bound, or null
   const float* b[2];   // [M]
 };
+struct OneRow {};
+template <class Two>
+__device__ __forceinline__ float with_addend(const Two& two, int side, int64_t i, float v) {
+  if constexpr (std::is_same<Two, RowAddend>::value) return two.A[side] ? v + two.A[side][i] : v;
+  else return v;
+}
+// b_in[m], zero without it, plus the addend's
+template <class Two>
+__device__ __forceinline__ float bias_row(const Two& two, int side, const float* b_in, int64_t m) {
+  const float b = b_in ? b_in[m] : 0.f;
+  if constexpr (std::is_same<Two, RowAddend>::value) return b + (two.b[side] ? two.b[side][m] : 0.f);
+  else return b;
+}
 
 // ---------------------------------------------------------------------------
 // Where a relaxation pass reads the slopes/intercepts {alpha_u, beta_u, alpha_l,
@@ -634,6 +649,7 @@ struct RelaxSrc {
 // one wave64 per coefficient row, float loads strided by 64 lanes, wave
 // reduction of the bias terms.  Writes A' for both bounds and
 //   b_out = (b_in + sum_k A * beta_sel)  [+ sum_k A' * kbias if kbias].
+template <class Two>
 __global__ void __launch_bounds__(256)
 relu_relax_rows_kernel(const float* __restrict__ Au, const float* __restrict__ Al, int64_t a_dstride, int64_t M,
                        int64_t S, int64_t K,
@@ -641,7 +657,7 @@ relu_relax_rows_kernel(const float* __restrict__ Au, const float* __restrict__ A
                        const float* __restrict__ kbias, const float* __restrict__ cvec,
                        const float* __restrict__ bu_in, const float* __restrict__ bl_in, float* __restrict__ Au_out,
                        float* __restrict__ Al_out, float* __restrict__ bu_out, float* __restrict__ bl_out,
-                       float* __restrict__ cu_out, float* __restrict__ cl_out, RowAddend two) {
+                       float* __restrict__ cu_out, float* __restrict__ cl_out, Two two) {
   const int lane = threadIdx.x & 63;
   const int64_t m = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (m >= M) return;
@@ -652,8 +668,7 @@ relu_relax_rows_kernel(const float* __restrict__ Au, const float* __restrict__ A
     // {alpha_u, beta_u, alpha_l, beta_l}; no source = no ReLU (identity)
     const float4 r = relax.at(d, K, k);
     if (Au) {
-      float v = Au[a_row + k];
-      if (two.A[0]) v = v + two.A[0][m * K + k];
+      float v = with_addend(two, 0, m * K + k, Au[a_row + k]);
       bool nn = v >= 0.f;
       float o = v * (nn ? r.x : r.z);
       su += v * (nn ? r.y : r.w);
@@ -662,8 +677,7 @@ relu_relax_rows_kernel(const float* __restrict__ Au, const float* __restrict__ A
       if (Au_out) Au_out[m * K + k] = o;
     }
     if (Al) {
-      float v = Al[a_row + k];
-      if (two.A[1]) v = v + two.A[1][m * K + k];
+      float v = with_addend(two, 1, m * K + k, Al[a_row + k]);
       bool nn = v >= 0.f;
       float o = v * (nn ? r.z : r.x);
       sl += v * (nn ? r.w : r.y);
@@ -682,8 +696,8 @@ relu_relax_rows_kernel(const float* __restrict__ Au, const float* __restrict__ A
     cl += __shfl_xor(cl, off, 64);
   }
   if (lane == 0) {
-    if (bu_out) bu_out[m] = ((bu_in ? bu_in[m] : 0.f) + (two.b[0] ? two.b[0][m] : 0.f) + su) + ku;
-    if (bl_out) bl_out[m] = ((bl_in ? bl_in[m] : 0.f) + (two.b[1] ? two.b[1][m] : 0.f) + sl) + kl;
+    if (bu_out) bu_out[m] = (bias_row(two, 0, bu_in, m) + su) + ku;
+    if (bl_out) bl_out[m] = (bias_row(two, 1, bl_in, m) + sl) + kl;
     if (cu_out) cu_out[m] = cu;
     if (cl_out) cl_out[m] = cl;
   }
@@ -777,11 +791,17 @@ relu_relax_domain_kernel(const float* __restrict__ Au, const float* __restrict__
 // bound and four table entries in flight per thread.  Needs K % 4 == 0 and
 // 16-byte aligned rows.  Row sums: per-thread partials in k order, then a fixed
 // tree (wave shuffles, then the workgroup's waves through LDS when TPR > 64).
-__device__ __forceinline__ float4 add4(float4 a, float4 b) {
-  return make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w);
+template <class Two>
+__device__ __forceinline__ float4 with_addend4(const Two& two, int side, int64_t i, float4 v) {
+  if constexpr (std::is_same<Two, RowAddend>::value)
+    if (two.A[side]) {
+      const float4 a = *reinterpret_cast<const float4*>(two.A[side] + i);
+      return make_float4(v.x + a.x, v.y + a.y, v.z + a.z, v.w + a.w);
+    }
+  return v;
 }
 
-template <int TPR>
+template <int TPR, class Two>
 __global__ void __launch_bounds__(256)
 relu_relax_rows4_kernel(const float* __restrict__ Au, const float* __restrict__ Al, int64_t a_dstride, int64_t M,
                         int64_t S, int64_t K,
@@ -789,7 +809,7 @@ relu_relax_rows4_kernel(const float* __restrict__ Au, const float* __restrict__ 
                         const float* __restrict__ kbias, const float* __restrict__ cvec,
                         const float* __restrict__ bu_in, const float* __restrict__ bl_in, float* __restrict__ Au_out,
                         float* __restrict__ Al_out, float* __restrict__ bu_out, float* __restrict__ bl_out,
-                        float* __restrict__ cu_out, float* __restrict__ cl_out, RowAddend two) {
+                        float* __restrict__ cu_out, float* __restrict__ cl_out, Two two) {
   constexpr int RPB = 256 / TPR;   // rows per workgroup
   constexpr int WPR = TPR / 64;    // waves per row
   __shared__ float red[6][256 / 64];
@@ -811,8 +831,7 @@ relu_relax_rows4_kernel(const float* __restrict__ Au, const float* __restrict__ 
       // one load serves both bounds when they share the coefficient (the first region of a C = I query)
       const float4 vu4 = Au ? *reinterpret_cast<const float4*>(Au + a_row + k) : make_float4(0.f, 0.f, 0.f, 0.f);
       if (Au) {
-        float4 v4 = vu4;
-        if (two.A[0]) v4 = add4(v4, *reinterpret_cast<const float4*>(two.A[0] + m * K + k));
+        const float4 v4 = with_addend4(two, 0, m * K + k, vu4);
         const float v[4] = {v4.x, v4.y, v4.z, v4.w};
         float o[4];
 #pragma unroll
@@ -826,8 +845,8 @@ relu_relax_rows4_kernel(const float* __restrict__ Au, const float* __restrict__ 
         if (Au_out) *reinterpret_cast<float4*>(Au_out + m * K + k) = make_float4(o[0], o[1], o[2], o[3]);
       }
       if (Al) {
-        float4 v4 = Al == Au ? vu4 : *reinterpret_cast<const float4*>(Al + a_row + k);
-        if (two.A[1]) v4 = add4(v4, *reinterpret_cast<const float4*>(two.A[1] + m * K + k));
+        const float4 v4 =
+            with_addend4(two, 1, m * K + k, Al == Au ? vu4 : *reinterpret_cast<const float4*>(Al + a_row + k));
         const float v[4] = {v4.x, v4.y, v4.z, v4.w};
         const float4 ad =
             add_l ? *reinterpret_cast<const float4*>(add_l + d * add_ld + k) : make_float4(0.f, 0.f, 0.f, 0.f);
@@ -866,8 +885,8 @@ relu_relax_rows4_kernel(const float* __restrict__ Au, const float* __restrict__ 
       }
   }
   if (live && t == 0) {
-    if (bu_out) bu_out[m] = ((bu_in ? bu_in[m] : 0.f) + (two.b[0] ? two.b[0][m] : 0.f) + s[0]) + s[2];
-    if (bl_out) bl_out[m] = ((bl_in ? bl_in[m] : 0.f) + (two.b[1] ? two.b[1][m] : 0.f) + s[1]) + s[3];
+    if (bu_out) bu_out[m] = (bias_row(two, 0, bu_in, m) + s[0]) + s[2];
+    if (bl_out) bl_out[m] = (bias_row(two, 1, bl_in, m) + s[1]) + s[3];
     if (cu_out) cu_out[m] = s[4];
     if (cl_out) cl_out[m] = s[5];
   }
@@ -2018,16 +2037,18 @@ static int relax_pass(const float* A_u, const float* A_l, int64_t a_dstride, int
                          K, chunks, rpw, src, add_l, add_ld, kbias, cvec, b_u_in, b_l_in, A_u_out, A_l_out, b_u_out,
                          b_l_out, c_u_out, c_l_out);
     BF_LAUNCH_CHECK("relu_relax_shared_kernel");
-  } else if (vec && K >= 1024) {
-    hipLaunchKernelGGL(relu_relax_rows4_kernel<256>, dim3((unsigned)M), dim3(256), 0, stream, A_u, A_l, a_dstride, M, S,
-                       K, src, add_l, add_ld, kbias, cvec, b_u_in, b_l_in, A_u_out, A_l_out, b_u_out, b_l_out, c_u_out,
-                       c_l_out, two);
-    BF_LAUNCH_CHECK("relu_relax_rows4_kernel<256>");
   } else if (vec) {
-    hipLaunchKernelGGL(relu_relax_rows4_kernel<64>, dim3((unsigned)ceil_div(M, 4)), dim3(256), 0, stream, A_u, A_l,
-                       a_dstride, M, S, K, src, add_l, add_ld, kbias, cvec, b_u_in, b_l_in, A_u_out, A_l_out, b_u_out,
-                       b_l_out, c_u_out, c_l_out, two);
-    BF_LAUNCH_CHECK("relu_relax_rows4_kernel<64>");
+    const bool wide = K >= 1024;   // a workgroup per row, else a wave
+    auto launch = [&](auto kernel, auto addend) {
+      hipLaunchKernelGGL(kernel, dim3((unsigned)(wide ? M : ceil_div(M, 4))), dim3(256), 0, stream, A_u, A_l, a_dstride,
+                         M, S, K, src, add_l, add_ld, kbias, cvec, b_u_in, b_l_in, A_u_out, A_l_out, b_u_out, b_l_out,
+                         c_u_out, c_l_out, addend);
+    };
+    if (one && wide) launch(relu_relax_rows4_kernel<256, OneRow>, OneRow{});
+    else if (one) launch(relu_relax_rows4_kernel<64, OneRow>, OneRow{});
+    else if (wide) launch(relu_relax_rows4_kernel<256, RowAddend>, two);
+    else launch(relu_relax_rows4_kernel<64, RowAddend>, two);
+    BF_LAUNCH_CHECK("relu_relax_rows4_kernel");
   } else if (one && !vec && K <= 512 && S >= 16 && M >= 1024) {
     // (fewer rows: 16 rows of 77 in 100 domains 9.2 / 9.0 us, row / domain kernel)
     const int rpw = 16;
@@ -2044,9 +2065,13 @@ static int relax_pass(const float* A_u, const float* A_l, int64_t a_dstride, int
     else launch(relu_relax_domain_kernel<8>);
     BF_LAUNCH_CHECK("relu_relax_domain_kernel");
   } else {
-    hipLaunchKernelGGL(relu_relax_rows_kernel, dim3((unsigned)ceil_div(M, 4)), dim3(256), 0, stream, A_u, A_l,
-                       a_dstride, M, S, K, src, add_l, add_ld, kbias, cvec, b_u_in, b_l_in, A_u_out, A_l_out, b_u_out,
-                       b_l_out, c_u_out, c_l_out, two);
+    auto launch = [&](auto kernel, auto addend) {
+      hipLaunchKernelGGL(kernel, dim3((unsigned)ceil_div(M, 4)), dim3(256), 0, stream, A_u, A_l, a_dstride, M, S, K, src,
+                         add_l, add_ld, kbias, cvec, b_u_in, b_l_in, A_u_out, A_l_out, b_u_out, b_l_out, c_u_out,
+                         c_l_out, addend);
+    };
+    if (one) launch(relu_relax_rows_kernel<OneRow>, OneRow{});
+    else launch(relu_relax_rows_kernel<RowAddend>, two);
     BF_LAUNCH_CHECK("relu_relax_rows_kernel");
   }
   return BF_OK;
