@@ -45,6 +45,7 @@ CASES = [
     (3, 3, 32, 16, 4, 2, 1, 1, 0, False),   # Linf ball input
     (6, 5, 8, 24, 3, 1, 1, 0, 1, True),     # 24 channels: the second half's block is partly padding
     (2, 4, 6, 48, 3, 1, 0, 0, 1, False),    # three blocks, one pixel tile: the odd half has no task
+    (1601, 12, 14, 24, 3, 1, 1, 0, 1, True),   # several rows a workgroup, a map of two batches: the next row's ahead
     (2, 16, 20, 16, 3, 1, 1, 0, 1, True),   # two maps above the kernel's LDS: products, then finalize
 ]
 
