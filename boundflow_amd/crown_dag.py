@@ -112,6 +112,37 @@ def _conv_bias_map(bias: torch.Tensor, out_shape) -> torch.Tensor:
     return bias.reshape(Co, 1).expand(Co, Ho * Wo).reshape(Co * Ho * Wo).contiguous()
 
 
+def _relu_biases(x: str, maker, readers, dynamic, output_value):
+    """((index, op), (index, op), add): the affine ops whose bias the pass of the ReLU reading ``x`` can
+    sum, because the relaxed coefficient reaches them as it is -- through flattens, reshapes and sums of
+    values that nothing else reads.  The first is the one that the bias rows go with (x's maker, or down
+    the first operands of sums); the second is the second operand of the sum that makes x, whose output
+    is named third: its branch begins with bias rows of its own, so that every row is summed in the order
+    it has without this.  (None, None) where there is none."""
+    def source(v):
+        while readers.get(v) == 1 and v != output_value and v in maker:
+            if maker[v][1].op_type not in ("flatten", "reshape"):
+                return maker[v]
+            v = maker[v][1].inputs[0]
+        return None, None
+
+    def affine(v):
+        i, op = source(v)
+        return (i, op) if op is not None and op.op_type in ("linear", "conv2d") and len(op.inputs) == 3 else (None, None)
+
+    def is_sum(op):   # (a constant operand joins the bias rows between the two)
+        return op is not None and op.op_type == "add" and all(v in dynamic for v in op.inputs)
+
+    second, add_out = (None, None), None
+    op = source(x)[1]
+    if is_sum(op) and len(op.inputs) == 2:
+        second, add_out = affine(op.inputs[1]), op.outputs[0]
+    while is_sum(op):
+        x = op.inputs[0]
+        op = source(x)[1]
+    return affine(x), second, add_out
+
+
 def _module_task(module: BFTaskModule):
     module.validate()
     task = module.get_entry_task()
@@ -402,28 +433,32 @@ def crown_backward_dag(
         return (zero_b if st.b_u is not None else None), (zero_b if st.b_l is not None else None)
 
     def rows_pass(st: _Rows, n: int, *, pre=None, alpha=None, alpha_ld=0, add=None, add_ld=0, kbias=None,
-                  cvec=None, name="crown_relu_relax", two: Optional[_Rows] = None):
+                  cvec=None, name="crown_relu_relax", two: Optional[_Rows] = None, kbias2=None):
         """bf_crown_relu_relax_lu over the bounds st carries (``two``: over the sum of st and two):
-        (A', b + sums, center sums).  Without a relaxation, rows shared by both bounds are passed once."""
+        (A', b + sums, center sums, or with ``kbias2`` its sums).  Without a relaxation, rows shared
+        by both bounds are passed once."""
         one = pre is None and add is None and shared(st)
         rA_u, rA_l = like(st, n, one)
         nb_u, nb_l = like(_Rows(st.b_u, st.b_l, None, None), 1, one)
         nb_u = None if nb_u is None else nb_u.reshape(M)
         nb_l = None if nb_l is None else nb_l.reshape(M)
-        c_u = torch.empty(M, device=dev) if (cvec is not None and st.A_u is not None) else None
-        c_l = (c_u if one else torch.empty(M, device=dev)) if (cvec is not None and st.A_l is not None) else None
+        apart = cvec is not None or kbias2 is not None
+        c_u = torch.empty(M, device=dev) if (apart and st.A_u is not None) else None
+        c_l = (c_u if one else torch.empty(M, device=dev)) if (apart and st.A_l is not None) else None
         A_l_in = None if one else st.A_l
         nz = int(st.A_u is not None) + int(A_l_in is not None)
         reads = 1 if (nz == 2 and ptr_of(st.A_u) == ptr_of(st.A_l)) else nz
-        if two is not None:
-            with _timed(name, 0.0, 4.0 * (reads + 2 * nz) * M * n):
-                _lib.call("bf_crown_relu_relax_sum_lu", _lib.ptr(st.A_u), _lib.ptr(st.A_l), _lib.ptr(two.A_u),
+        if two is not None or kbias2 is not None:
+            with_two = two is not None
+            two = two if with_two else _Rows(None, None, None, None)
+            with _timed(name, 0.0, 4.0 * (reads + (2 if with_two else 1) * nz) * M * n):
+                _lib.call("bf_crown_relu_relax_biases_lu", _lib.ptr(st.A_u), _lib.ptr(st.A_l), _lib.ptr(two.A_u),
                           _lib.ptr(two.A_l), B, S, n, _lib.ptr(pre.lower.reshape(B, n)),
                           _lib.ptr(pre.upper.reshape(B, n)), _lib.ptr(alpha), alpha_ld,
-                          _lib.ptr(add if st.A_l is not None else None), add_ld, _lib.ptr(kbias), _lib.ptr(st.b_u),
-                          _lib.ptr(st.b_l), _lib.ptr(two.b_u), _lib.ptr(two.b_l), _lib.ptr(rA_u), _lib.ptr(rA_l),
-                          _lib.ptr(nb_u), _lib.ptr(nb_l), stream)
-            return _Rows(rA_u, rA_l, nb_u, nb_l), (None, None)
+                          _lib.ptr(add if st.A_l is not None else None), add_ld, _lib.ptr(kbias), _lib.ptr(kbias2),
+                          _lib.ptr(st.b_u), _lib.ptr(st.b_l), _lib.ptr(two.b_u), _lib.ptr(two.b_l), _lib.ptr(rA_u),
+                          _lib.ptr(rA_l), _lib.ptr(nb_u), _lib.ptr(nb_l), _lib.ptr(c_u), _lib.ptr(c_l), stream)
+            return _Rows(rA_u, rA_l, nb_u, nb_l), (c_u, c_l)
         with _timed(name, 0.0, 4.0 * (reads + nz) * M * n):
             _lib.call("bf_crown_relu_relax_lu", _lib.ptr(st.A_u), _lib.ptr(A_l_in), S * n, B, S, n,
                       _lib.ptr(None if pre is None else pre.lower.reshape(B, n)),
@@ -478,39 +513,17 @@ def crown_backward_dag(
             readers[name] = readers.get(name, 0) + 1
     maker = {op.outputs[0]: (i, op) for i, op in enumerate(task.ops)}
     folded = set()   # the affine ops whose bias a ReLU's pass has summed
+    branch_b: Dict[str, tuple] = {}   # an add's output -> the bias rows of its second operand, summed there
 
-    def bias_of(x: str):
-        """The biases of the affine ops whose coefficient is the relaxed one of the ReLU reading x:
-        x's own maker's or, through adds and reshapes, those of the values x is the sum of, where
-        nothing else reads them."""
-        if readers.get(x) != 1 or x == output_value or x not in maker:
-            return
-        i, op = maker[x]
-        if op.op_type in ("linear", "conv2d"):
-            if len(op.inputs) == 3:
-                yield i, op
-        elif op.op_type in ("add", "flatten", "reshape"):
-            for v in op.inputs:
-                if v in dynamic and _numel(trace.shapes[v]) == _numel(trace.shapes[x]):
-                    yield from bias_of(v)
-
-    def relu_bias(x: str) -> Optional[torch.Tensor]:
-        """Their sum as one value per element of x (kept across queries)."""
-        ops = list(bias_of(x))
-        folded.update(i for i, _op in ops)
-        if not ops:
-            return None
-        maps = [(params[op.inputs[2]], trace.shapes[op.outputs[0]] if op.op_type == "conv2d" else None)
-                for _i, op in ops]
-
-        def make():
-            flat = [b.detach().contiguous() if shape is None else _conv_bias_map(b.detach(), shape)
-                    for b, shape in maps]
-            return flat[0] if len(flat) == 1 else torch.stack(flat).sum(dim=0)
-
-        if len(maps) == 1 and maps[0][1] is None:
-            return make()
-        return derived("dag_bias:" + ":".join(str(shape) for _b, shape in maps), tuple(b for b, _s in maps), make)
+    def bias_map(op) -> torch.Tensor:
+        """An affine op's bias as one value per output element (a conv's kept across queries)."""
+        bias = params[op.inputs[2]]
+        if op.op_type == "linear":
+            return bias.contiguous()
+        shape = trace.shapes[op.outputs[0]]
+        # (bound to this op's shape: a captured query remakes the map long after the backward has moved on)
+        return derived(f"conv_bias_map:{shape[1]}x{shape[2]}", (bias,),
+                       lambda b=bias, shape=shape: _conv_bias_map(b.detach(), shape))
 
     for op_index in range(len(task.ops) - 1, -1, -1):
         op = task.ops[op_index]
@@ -562,11 +575,7 @@ def crown_backward_dag(
             Ci, Hi, Wi = in_shape
             n_out = Co * Ho * Wo
             if len(op.inputs) == 3 and op_index not in folded:
-                bias = params[op.inputs[2]]
-                # (bound here: a captured query remakes the map long after this loop has moved on)
-                kbias = derived(f"conv_bias_map:{Ho}x{Wo}", (bias,),
-                                lambda b=bias, shape=out_shape: _conv_bias_map(b.detach(), shape))
-                st, _ = rows_pass(st, n_out, kbias=kbias, name="conv_bias_rows")
+                st, _ = rows_pass(st, n_out, kbias=bias_map(op), name="conv_bias_rows")
             one = shared(st)
             y_u, y_l = like(st, Ci * Hi * Wi, one)
             A_l_in = None if one else st.A_l
@@ -595,8 +604,13 @@ def crown_backward_dag(
                 relu_influence[x] = infl
             if save is not None:
                 save["relu_A"][op_index] = st.A_l      # the coefficient before the relaxation
-            new, _ = rows_pass(st, n, pre=pre, alpha=alpha, alpha_ld=alpha_ld, add=add, add_ld=add_ld,
-                               kbias=relu_bias(x), two=two)
+            first, second, add_out = _relu_biases(x, maker, readers, dynamic, output_value)
+            folded.update(i for i, _op in (first, second) if _op is not None)
+            new, rows2 = rows_pass(st, n, pre=pre, alpha=alpha, alpha_ld=alpha_ld, add=add, add_ld=add_ld,
+                                   kbias=None if first[1] is None else bias_map(first[1]), two=two,
+                                   kbias2=None if second[1] is None else bias_map(second[1]))
+            if second[1] is not None:
+                branch_b[add_out] = rows2
             accumulate(x, new)
         elif t in ("flatten", "reshape"):
             accumulate(x, st)          # the rows are already laid out in the input's element order
@@ -633,7 +647,7 @@ def crown_backward_dag(
                 if idx == 0:
                     bu, bl = cb_u, cb_l
                 else:
-                    bu, bl = zeros_like_b(st)
+                    bu, bl = branch_b.get(out) or zeros_like_b(st)
                 accumulate(name, _Rows(st.A_u, st.A_l, bu, bl))
         elif t == "concat":
             out_shape = trace.shapes[out]

@@ -577,7 +577,8 @@ ibp_batched_linear_kernel(const float* __restrict__ lo, const float* __restrict_
 // own.  The launches are short of work, not of bandwidth: a residual query of 64 x 10 rows (4 blocks of
 // 512, both bounds) took 449 us with the sums as launches (16 of about 4.3 us) and the affine ops' bias
 // sums as passes (8 of about 5.6 us), 365 us with both inside the relaxation pass; a residual conv
-// net of 16 x 10 rows 431 and 332 us.  A pass without one is compiled without it (OneRow): a query of
+// net of 16 x 10 rows 431 and 332 us.  In a pass with an addend cvec is no center but the bias of a second
+// affine op, one vector for every domain, whose sums the caller keeps apart.  A pass without one is compiled without it (OneRow): a query of
 // nine rows has three of them in its 67 us, which took 0.5 us more with the tests for it.
 struct RowAddend {
   const float* A[2];   // [M, K] of the upper and the lower bound, or null
@@ -588,6 +589,10 @@ template <class Two>
 __device__ __forceinline__ float with_addend(const Two& two, int side, int64_t i, float v) {
   if constexpr (std::is_same<Two, RowAddend>::value) return two.A[side] ? v + two.A[side][i] : v;
   else return v;
+}
+template <class Two>
+__device__ __forceinline__ int64_t cvec_index(int64_t d, int64_t K, int64_t k) {
+  return std::is_same<Two, RowAddend>::value ? k : d * K + k;
 }
 // b_in[m], zero without it, plus the addend's
 template <class Two>
@@ -673,7 +678,7 @@ relu_relax_rows_kernel(const float* __restrict__ Au, const float* __restrict__ A
       float o = v * (nn ? r.x : r.z);
       su += v * (nn ? r.y : r.w);
       if (kbias) ku += o * kbias[k];
-      if (cvec) cu += o * cvec[d * K + k];
+      if (cvec) cu += o * cvec[cvec_index<Two>(d, K, k)];
       if (Au_out) Au_out[m * K + k] = o;
     }
     if (Al) {
@@ -683,7 +688,7 @@ relu_relax_rows_kernel(const float* __restrict__ Au, const float* __restrict__ A
       sl += v * (nn ? r.w : r.y);
       if (add_l) o = o + add_l[d * add_ld + k];
       if (kbias) kl += o * kbias[k];
-      if (cvec) cl += o * cvec[d * K + k];
+      if (cvec) cl += o * cvec[cvec_index<Two>(d, K, k)];
       if (Al_out) Al_out[m * K + k] = o;
     }
   }
@@ -825,7 +830,8 @@ relu_relax_rows4_kernel(const float* __restrict__ Au, const float* __restrict__ 
       float4 r[4];
       relax.quad(d, K, k, r);
       const float4 kb = kbias ? *reinterpret_cast<const float4*>(kbias + k) : make_float4(0.f, 0.f, 0.f, 0.f);
-      const float4 cv = cvec ? *reinterpret_cast<const float4*>(cvec + d * K + k) : make_float4(0.f, 0.f, 0.f, 0.f);
+      const float4 cv = cvec ? *reinterpret_cast<const float4*>(cvec + cvec_index<Two>(d, K, k))
+                             : make_float4(0.f, 0.f, 0.f, 0.f);
       const float kbv[4] = {kb.x, kb.y, kb.z, kb.w};
       const float cvv[4] = {cv.x, cv.y, cv.z, cv.w};
       // one load serves both bounds when they share the coefficient (the first region of a C = I query)
@@ -1586,7 +1592,7 @@ static int relax_pass(const float* A_u, const float* A_l, int64_t a_dstride, int
                       const RelaxSrc& src, const float* add_l, int64_t add_ld, const float* kbias, const float* cvec,
                       const float* b_u_in, const float* b_l_in, float* A_u_out, float* A_l_out, float* b_u_out,
                       float* b_l_out, float* c_u_out, float* c_l_out, hipStream_t stream, bool sums_only,
-                      const RowAddend& two = RowAddend{});
+                      const RowAddend* two = nullptr);
 
 int bf_crown_relu_linear_fwd(const float* A_u, const float* A_l, int64_t a_dstride, int64_t D, int64_t S, int64_t N,
                              const float* relax, const float* add_l, int64_t add_ld, const float* W, int64_t P,
@@ -2002,7 +2008,7 @@ static int relax_pass(const float* A_u, const float* A_l, int64_t a_dstride, int
                       const RelaxSrc& src, const float* add_l, int64_t add_ld, const float* kbias, const float* cvec,
                       const float* b_u_in, const float* b_l_in, float* A_u_out, float* A_l_out, float* b_u_out,
                       float* b_l_out, float* c_u_out, float* c_l_out, hipStream_t stream, bool sums_only,
-                      const RowAddend& two) {
+                      const RowAddend* two) {
   BF_REQUIRE(D >= 0 && S >= 0 && K > 0, "bf_crown_relu_relax: bad sizes");
   const int64_t M = D * S;
   if (M == 0) return BF_OK;
@@ -2015,8 +2021,8 @@ static int relax_pass(const float* A_u, const float* A_l, int64_t a_dstride, int
   const bool vec = (K % 4 == 0) && (a_dstride % 4 == 0) && al16(A_u) && al16(A_l) && al16(A_u_out) &&
                    al16(A_l_out) && al16(kbias) &&
                    al16(cvec) && al16(add_l) && (add_l == nullptr || add_ld % 4 == 0) && al16(src.lo) &&
-                   al16(src.hi) && al16(src.alpha) && (src.alpha_ld % 4 == 0) && al16(two.A[0]) && al16(two.A[1]);
-  const bool one = !two.A[0] && !two.A[1];   // (the kernels that keep a domain's operands take no second coefficient)
+                   al16(src.hi) && al16(src.alpha) && (src.alpha_ld % 4 == 0) && (!two || (al16(two->A[0]) && al16(two->A[1])));
+  const bool one = two == nullptr;   // (the kernels that keep a domain's operands take no second coefficient)
   if (one && vec && K <= 512 && (a_dstride == 0 ? S >= 16 : (S >= 8 && M >= 8192))) {
     // a shared coefficient: 16 rows of one domain per workgroup (4 per wave), the
     // domain's operands held in registers across them (C2's 500 x 500 shape: 8, 16 and
@@ -2046,8 +2052,8 @@ static int relax_pass(const float* A_u, const float* A_l, int64_t a_dstride, int
     };
     if (one && wide) launch(relu_relax_rows4_kernel<256, OneRow>, OneRow{});
     else if (one) launch(relu_relax_rows4_kernel<64, OneRow>, OneRow{});
-    else if (wide) launch(relu_relax_rows4_kernel<256, RowAddend>, two);
-    else launch(relu_relax_rows4_kernel<64, RowAddend>, two);
+    else if (wide) launch(relu_relax_rows4_kernel<256, RowAddend>, *two);
+    else launch(relu_relax_rows4_kernel<64, RowAddend>, *two);
     BF_LAUNCH_CHECK("relu_relax_rows4_kernel");
   } else if (one && !vec && K <= 512 && S >= 16 && M >= 1024) {
     // (fewer rows: 16 rows of 77 in 100 domains 9.2 / 9.0 us, row / domain kernel)
@@ -2071,7 +2077,7 @@ static int relax_pass(const float* A_u, const float* A_l, int64_t a_dstride, int
                          c_l_out, addend);
     };
     if (one) launch(relu_relax_rows_kernel<OneRow>, OneRow{});
-    else launch(relu_relax_rows_kernel<RowAddend>, two);
+    else launch(relu_relax_rows_kernel<RowAddend>, *two);
     BF_LAUNCH_CHECK("relu_relax_rows_kernel");
   }
   return BF_OK;
@@ -2098,18 +2104,31 @@ int bf_crown_relu_relax_lu(const float* A_u, const float* A_l, int64_t a_dstride
                     b_u_out, b_l_out, c_u_out, c_l_out, stream, false);
 }
 
+int bf_crown_relu_relax_biases_lu(const float* A_u, const float* A_l, const float* A2_u, const float* A2_l, int64_t D,
+                                  int64_t S, int64_t K, const float* pre_lo, const float* pre_hi, const float* alpha,
+                                  int64_t alpha_ld, const float* add_l, int64_t add_ld, const float* kbias,
+                                  const float* kbias2, const float* b_u_in, const float* b_l_in, const float* b2_u,
+                                  const float* b2_l, float* A_u_out, float* A_l_out, float* b_u_out, float* b_l_out,
+                                  float* k2_u, float* k2_l, hipStream_t stream) {
+  BF_REQUIRE(alpha == nullptr || alpha_ld == 0 || alpha_ld >= K, "bf_crown_relu_relax_biases_lu: bad alpha_ld");
+  BF_REQUIRE((kbias2 != nullptr) == (k2_u != nullptr || k2_l != nullptr),
+             "bf_crown_relu_relax_biases_lu: a second bias goes with its sums");
+  const RelaxSrc src{nullptr, pre_lo, pre_hi, alpha, alpha_ld};
+  const RowAddend two{{A2_u, A2_l}, {b2_u, b2_l}};
+  return relax_pass(A_u, A_l, S * K, D, S, K, src, add_l, add_ld, kbias, kbias2, b_u_in, b_l_in, A_u_out, A_l_out,
+                    b_u_out, b_l_out, k2_u, k2_l, stream, false, &two);
+}
+
 int bf_crown_relu_relax_sum_lu(const float* A_u, const float* A_l, const float* A2_u, const float* A2_l, int64_t D,
                                int64_t S, int64_t K, const float* pre_lo, const float* pre_hi, const float* alpha,
                                int64_t alpha_ld, const float* add_l, int64_t add_ld, const float* kbias,
                                const float* b_u_in, const float* b_l_in, const float* b2_u, const float* b2_l,
                                float* A_u_out, float* A_l_out, float* b_u_out, float* b_l_out, hipStream_t stream) {
-  BF_REQUIRE(alpha == nullptr || alpha_ld == 0 || alpha_ld >= K, "bf_crown_relu_relax_sum_lu: bad alpha_ld");
   BF_REQUIRE((A_u == nullptr) == (A2_u == nullptr) && (A_l == nullptr) == (A2_l == nullptr),
              "bf_crown_relu_relax_sum_lu: a bound's two coefficients go together");
-  const RelaxSrc src{nullptr, pre_lo, pre_hi, alpha, alpha_ld};
-  const RowAddend two{{A2_u, A2_l}, {b2_u, b2_l}};
-  return relax_pass(A_u, A_l, S * K, D, S, K, src, add_l, add_ld, kbias, nullptr, b_u_in, b_l_in, A_u_out, A_l_out,
-                    b_u_out, b_l_out, nullptr, nullptr, stream, false, two);
+  return bf_crown_relu_relax_biases_lu(A_u, A_l, A2_u, A2_l, D, S, K, pre_lo, pre_hi, alpha, alpha_ld, add_l, add_ld,
+                                       kbias, nullptr, b_u_in, b_l_in, b2_u, b2_l, A_u_out, A_l_out, b_u_out, b_l_out,
+                                       nullptr, nullptr, stream);
 }
 
 int bf_concretize_dense(const float* A, int64_t D, int64_t S, int64_t I, const float* center, const float* rad,

@@ -438,6 +438,14 @@ int bf_crown_relu_relax_sum_lu(const float* A_u, const float* A_l, const float* 
                                int64_t alpha_ld, const float* add_l, int64_t add_ld, const float* kbias,
                                const float* b_u_in, const float* b_l_in, const float* b2_u, const float* b2_l,
                                float* A_u_out, float* A_l_out, float* b_u_out, float* b_l_out, hipStream_t stream);
+/* The same, the second coefficient optional, with the sums k2[m] = sum_k A'[m, k] kbias2[k] of another
+ * affine op's bias (both NULL without one): the branch of a sum beside the one the bias rows follow. */
+int bf_crown_relu_relax_biases_lu(const float* A_u, const float* A_l, const float* A2_u, const float* A2_l, int64_t D,
+                                  int64_t S, int64_t K, const float* pre_lo, const float* pre_hi, const float* alpha,
+                                  int64_t alpha_ld, const float* add_l, int64_t add_ld, const float* kbias,
+                                  const float* kbias2, const float* b_u_in, const float* b_l_in, const float* b2_u,
+                                  const float* b2_l, float* A_u_out, float* A_l_out, float* b_u_out, float* b_l_out,
+                                  float* k2_u, float* k2_l, hipStream_t stream);
 
 /* Dense coefficient rows A [M, I] against the input set:
  * out = A . center[d] -/+ eps * sum |A| (Linf, rad NULL) or -/+ sum |A| * rad[d] (box), + b;

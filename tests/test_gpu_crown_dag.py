@@ -350,3 +350,67 @@ def test_relu_influence_matches_oracle(net):
     for k in ref_infl:
         scale = float(ref_infl[k].abs().max())
         assert_bounds_close(infl[k], ref_infl[k], f"{net} influence[{k}]", rtol=1e-5, atol=1e-6 * scale)
+
+
+def _residual(kind, gen, constant=False):
+    """A residual block net whose ReLUs read a maker with a bias, a sum of a skip and a biased branch (either
+    way round), a sum of two biased branches, and with ``constant`` a sum that a constant joins."""
+    from boundflow_amd.ir import BFTaskModule, BoundTask, TaskKind, TaskOp
+    from boundflow_amd.spec import InputSpec
+    params, ops, c = {}, [], 6
+    conv = kind == "cnn"
+
+    def affine(name, x, n_in, n_out):
+        shape = (n_out, n_in, 3, 3) if conv else (n_out, n_in)
+        params["W" + name] = torch.randn(shape, generator=gen) / (n_in * (9 if conv else 1)) ** 0.5
+        params["b" + name] = torch.randn(n_out, generator=gen) * 0.3
+        ops.append(TaskOp("conv2d" if conv else "linear", name, [x, "W" + name, "b" + name], ["h" + name],
+                          {"stride": 1, "padding": 1} if conv else {}))
+        return "h" + name
+
+    def relu(x):
+        ops.append(TaskOp("relu", "r" + x, [x], ["a" + x]))
+        return "a" + x
+
+    def add(name, *xs):
+        ops.append(TaskOp("add", name, list(xs), ["s" + name]))
+        return "s" + name
+
+    B = 5
+    x = relu(affine("1", "input", 2 if conv else 9, c))
+    x = relu(add("p", x, affine("2", x, c, c)))
+    x = relu(add("q", affine("3", x, c, c), x))
+    x = relu(add("r", add("t", affine("4", x, c, c), x), affine("5", x, c, c)))
+    if constant:
+        params["k"] = torch.randn((B, c, 7, 7) if conv else (B, c), generator=gen)
+        x = relu(add("u", affine("6", x, c, c), "k"))
+    if conv:
+        ops.append(TaskOp("flatten", "f", [x], ["flat"], {"start_dim": 1, "end_dim": -1}))
+        x = "flat"
+    params["Wh"] = torch.randn(4, c * 49 if conv else c, generator=gen)
+    ops.append(TaskOp("linear", "head", [x, "Wh"], ["out"]))
+    task = BoundTask(task_id="t0", kind=TaskKind.INTERVAL_IBP, ops=ops, input_values=["input"], output_values=["out"])
+    spec = InputSpec.linf(value_name="input", eps=0.05,
+                          center=torch.rand((B, 2, 7, 7) if conv else (B, 9), generator=gen))
+    return wl.Workload(kind, BFTaskModule(tasks=[task], entry_task_id="t0", bindings={"params": params}), spec,
+                       torch.randn(B, 3, 4, generator=gen), torch.zeros(B))
+
+
+@pytest.mark.parametrize("constant", [False, True])
+@pytest.mark.parametrize("kind", ["cnn", "mlp"])
+def test_biases_in_the_relaxation_pass(kind, constant, monkeypatch):
+    """The affine ops' biases summed inside the ReLUs' passes leave every bias row's order of additions: a conv
+    net's bounds keep their bits (a linear op sums its own in its contraction), and all match the oracle."""
+    dev = device()
+    announce(f"DAG biases in the relaxation pass {kind} constant={constant}")
+    w = _residual(kind, torch.Generator().manual_seed(11), constant)
+    got = _check(w, dev, f"{kind} constant={constant}")
+    monkeypatch.setattr(crown_dag, "_relu_biases", lambda *a: ((None, None), (None, None), None))
+    wd = wl.to_device(w, dev)
+    apart = hc.run_crown_ibp_mlp(wd.module, wd.spec, linear_spec_C=wd.C)
+    torch.cuda.synchronize()
+    if kind == "cnn":
+        assert torch.equal(got.lower, apart.lower) and torch.equal(got.upper, apart.upper)
+    else:
+        assert_bounds_close(got.lower, apart.lower, "lower")
+        assert_bounds_close(got.upper, apart.upper, "upper")
