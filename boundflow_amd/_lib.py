@@ -65,8 +65,8 @@ SIGNATURES = {
                                      P]),
     "bf_crown_relu_relax_sum_lu": (I32, [P, P, P, P, I64, I64, I64, P, P, P, I64, P, I64, P, P, P, P, P, P, P, P, P,
                                          P]),
-    "bf_crown_relu_relax_biases_lu": (I32, [P, P, P, P, I64, I64, I64, P, P, P, I64, P, I64, P, P, P, P, P, P, P, P, P, P,
-                                            P, P, P]),
+    "bf_crown_relu_relax_biases_lu": (I32, [P, P, P, P, I64, I64, I64, P, P, P, I64, P, I64, P, P, P, P, P, P, P, P, P,
+                                            P, P, P, P]),
     "bf_concretize_dense": (I32, [P, I64, I64, I64, P, P, F32, I32, P, I32, P, P]),
     "bf_concretize_dense_grad": (I32, [P, I64, I64, I64, P, P, F32, I32, P, P, P]),
     "bf_rows_abs_max": (I32, [P, P, I64, I64, I64, P, P]),

@@ -246,7 +246,8 @@ def chain_parts(layers: List[AffineLayer], k: int, M: int, S: int, nz: int, save
                 yield other.weight, False
         if save is not None and save.get("grad_rows") is not None:
             for other in layers[:-1]:
-                if other.kind == "linear" and reverse_takes_parts(M, _numel(other.out_shape), _numel(other.in_shape), S):
+                if other.kind == "linear" and reverse_takes_parts(M, _numel(other.out_shape),
+                                                                  _numel(other.in_shape), S):
                     yield other.weight, True
     return weight_parts(layers[k].weight, False, also())
 
@@ -788,7 +789,8 @@ def crown_backward(
             weight = chain_parts(layers, k, M, S, nz, save) if in_parts else transposed(W)
             # bytes: the coefficient rows and the weight read, the row partial norms written, the
             # gradient seed [M, P] written when asked
-            with _timed("crown_linear_concretize_parts" if in_parts else "crown_linear_concretize", 2.0 * nz * M * N * P,
+            with _timed("crown_linear_concretize_parts" if in_parts else "crown_linear_concretize",
+                        2.0 * nz * M * N * P,
                         4.0 * nz * (M * N + N * P + M * -(-P // 128)) + (4.0 * M * P if h_out is not None else 0.0)):
                 _lib.call("bf_crown_linear_concretize_parts" if in_parts else "bf_crown_linear_concretize",
                           _lib.ptr(A_u), _lib.ptr(A_l), stride, B, S, N, _lib.ptr(weight), P, _lib.ptr(rad), eps,

@@ -128,7 +128,8 @@ def _relu_biases(x: str, maker, readers, dynamic, output_value):
 
     def affine(v):
         i, op = source(v)
-        return (i, op) if op is not None and op.op_type in ("linear", "conv2d") and len(op.inputs) == 3 else (None, None)
+        biased = op is not None and op.op_type in ("linear", "conv2d") and len(op.inputs) == 3
+        return (i, op) if biased else (None, None)
 
     def is_sum(op):   # (a constant operand joins the bias rows between the two)
         return op is not None and op.op_type == "add" and all(v in dynamic for v in op.inputs)

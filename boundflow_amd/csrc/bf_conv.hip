@@ -320,12 +320,12 @@ __device__ __forceinline__ void stage_conv_weights(const GatherArgs& g, float* W
 // Elements of a row's map a thread of the interval conv stages at a time: the first batch of a row
 // is loaded ahead of the weights (the first row) or of the products of the row before, so its way from
 // memory runs beside them.  What is loaded ahead is held in registers across the products, and a thread
-// past the map loads for nothing, so a batch is short.  us of 4 / 6 / 8 / 12 at a time (inputs x map, all
-// loads in place in brackets): 2048 x 16 x 18 x 18 -> 32 channels 104 / 103 / 112 / 98 (138), 2048 x 3 x 34 x 34 -> 16
-// 57 / 66 / 58 / 67 (73), -> 32 84 / 93 / 87 / 96 (101), 2048 x 16 x 16 x 16 -> 32 89 / 98 / 88 / 97 (105), 2048 x 30 x 30 -> 16
-// 34 / 37 / 44 / 52 (55), 512 x 16 x 10 x 10 -> 32 16 / 18 / 21 / 25 (21); one input of them 10.1 / 10.3 / 11.2 / 10.6
-// (11.8), 7.1 / 7.8 / 7.1 / 8.6 (7.8), 8.7 / 9.9 / 9.0 / 10.2 (9.4), 9.4 / 10.3 / 9.6 / 10.7 (10.1), 5.4 / 6.0 / 6.4 / 7.5 (6.6),
-// 6.7 / 7.3 / 7.9 / 9.0 (8.2).
+// past the map loads for nothing, so a batch is short.  us of 4 / 6 / 8 / 12 at a time (all loads in place):
+//   2048 inputs of 16 x 18 x 18 -> 32 channels 104 / 103 / 112 / 98 (138), 3 x 34 x 34 -> 16 57 / 66 / 58 / 67 (73),
+//   3 x 34 x 34 -> 32 84 / 93 / 87 / 96 (101), 16 x 16 x 16 -> 32 89 / 98 / 88 / 97 (105),
+//   30 x 30 -> 16 34 / 37 / 44 / 52 (55);
+//   one input of them 10.1 / 10.3 / 11.2 / 10.6 (11.8), 7.1 / 7.8 / 7.1 / 8.6 (7.8), 8.7 / 9.9 / 9.0 / 10.2 (9.4),
+//   9.4 / 10.3 / 9.6 / 10.7 (10.1), 5.4 / 6.0 / 6.4 / 7.5 (6.6).
 // conv_mfma_kernel loads a map in place, 8 at a time: its maps are small and its launches short, and what a
 // load ahead holds in registers (109 against 57) costs more than it hides.  Slope optimisation on a CNN of 8
 // channels, 8 steps: 4 inputs 766 us ahead, 735 in place; 32 inputs 970, 925; of 16 channels, 32 inputs

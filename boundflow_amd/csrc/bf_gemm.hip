@@ -154,11 +154,11 @@ int gemm_parts_choice(int64_t M, int64_t N, int64_t K, int64_t S, int nz, int ep
 
 // Where the three-part kernel is the faster one.  us on one MI355X:
 // stores, fp32 / 64 x 64 / 128 x 128 tiles (in brackets the 64 x 64 tiles):
-//   576 x 256 (36):       K = 64 7.4 / 6.6 / 9.1, 128 8.8 / 8.5 / 12.0, 256 11.6 / 12.3 / 17.9, 512 17.5 / 20.0 / 29.1
-//   2304 x 512 (288):     K = 64 8.8 / 8.1 / 9.7, 256 16.6 / 15.8 / 18.5, 512 26.3 / 26.3 / 29.9, 1024 45.6 / 46.0 / 51.9
-//   4608 x 784 (936):     K = 256 28.3 / 20.4 / 22.1, 1024 83.4 / 60.3 / 60.3
-//   9216 x 784 (1872):    K = 256 42.5 / 38.0 / 31.5
-//   36864 x 256 (2304):   K = 16 13.3 / 12.1 / 15.0, 64 21.6 / 18.4 / 22.1, 256 53.6 / 41.7 / 45.0
+//   576 x 256 (36):     K = 64 7.4 / 6.6 / 9.1, 128 8.8 / 8.5 / 12.0, 256 11.6 / 12.3 / 17.9, 512 17.5 / 20.0 / 29.1
+//   2304 x 512 (288):   K = 64 8.8 / 8.1 / 9.7, 256 16.6 / 15.8 / 18.5, 512 26.3 / 26.3 / 29.9, 1024 45.6 / 46.0 / 51.9
+//   4608 x 784 (936):   K = 256 28.3 / 20.4 / 22.1, 1024 83.4 / 60.3 / 60.3
+//   9216 x 784 (1872):  K = 256 42.5 / 38.0 / 31.5
+//   36864 x 256 (2304): K = 16 13.3 / 12.1 / 15.0, 64 21.6 / 18.4 / 22.1, 256 53.6 / 41.7 / 45.0
 // stores where K is no multiple of 32 (the fp32 tiles then check their loads) or of four (float by float):
 //   576 x 256:   K = 50 8.4 / 8.3 / 10.3, 100 10.1 / 7.9 / 11.1, 250 16.2 / 16.2 / 21.6, 500 23.0 / 20.1 / 29.4
 //   36864 x 256: K = 50 32.2 / 22.4 / 23.6, 250 93.0 / 47.6 / 50.7, 500 94.5 / 76.6 / 78.3

@@ -7,7 +7,8 @@
 // parts before it leave: x = x0 + x1 + x2 exactly (8 + 8 + 8 significant bits against 24).
 // The exponent range of bf16 is fp32's, so the lower parts of a small value would be subnormal,
 // which the matrix cores read as zero: values are split times 2^24, which leaves the least part
-// of the least subnormal at 2^-125, and the sums are multiplied by 2^-48 at the end.  A product is the sum of eight part products,
+// of the least subnormal at 2^-125, and the sums are multiplied by 2^-48 at the end.  A product
+// is the sum of eight part products,
 //   x0 y0 + (x0 y1 + x1 y0) + (x1 y1 + x0 y2 + x2 y0) + (x1 y2 + x2 y1),
 // each exact; x2 y2, the ninth, is below 2^-32 of it.  They are summed in fp32 by
 // v_mfma_f32_32x32x16_bf16: eight of these take 256 cycles for the 16 k steps that eight

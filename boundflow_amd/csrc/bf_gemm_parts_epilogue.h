@@ -227,7 +227,8 @@ __device__ __forceinline__ void parts_epilogue(const GemmArgs& p, floatx16 (&acc
       constexpr bool LDS = decltype(from_lds)::value, X = decltype(extra)::value, CV = decltype(center)::value;
 #pragma unroll
       for (int i = 0; i < FM; ++i) {
-        const EpilogueRows<T> rows(C, p.ldc, m0, n0, wm, wn, i, lane), pre(X ? Cpre : C, p.ldc, m0, n0, wm, wn, i, lane);
+        const EpilogueRows<T> rows(C, p.ldc, m0, n0, wm, wn, i, lane);
+        const EpilogueRows<T> pre(X ? Cpre : C, p.ldc, m0, n0, wm, wn, i, lane);
 #pragma unroll
         for (int g = 0; g < 16; g += EPI_GROUP) {
           int dom[EPI_GROUP];   // the row's domain: its block of LDS entries, or its rows of the global operands

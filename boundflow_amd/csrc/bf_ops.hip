@@ -577,9 +577,10 @@ ibp_batched_linear_kernel(const float* __restrict__ lo, const float* __restrict_
 // own.  The launches are short of work, not of bandwidth: a residual query of 64 x 10 rows (4 blocks of
 // 512, both bounds) took 449 us with the sums as launches (16 of about 4.3 us) and the affine ops' bias
 // sums as passes (8 of about 5.6 us), 365 us with both inside the relaxation pass; a residual conv
-// net of 16 x 10 rows 431 and 332 us.  In a pass with an addend cvec is no center but the bias of a second
-// affine op, one vector for every domain, whose sums the caller keeps apart.  A pass without one is compiled without it (OneRow): a query of
-// nine rows has three of them in its 67 us, which took 0.5 us more with the tests for it.
+// net of 16 x 10 rows 431 and 332 us.  In a pass with an addend cvec is no center but the bias of a
+// second affine op, one vector for every domain, whose sums the caller keeps apart.  A pass without an
+// addend is compiled without it (OneRow): a query of nine rows has two of them in its 67 us, which took
+// 0.5 us more with the tests for it.
 struct RowAddend {
   const float* A[2];   // [M, K] of the upper and the lower bound, or null
   const float* b[2];   // [M]
@@ -1749,14 +1750,14 @@ int bf_crown_relu_linear_concretize_noalloc(const float* A_u, const float* A_l, 
                                          cvec, rad, eps, norm_p, b_u_in, b_l_in, h_scale, h_out, ws, lb, ub, stream);
 }
 
-static int relu_linear_relu_fwd(int b_parts, const float* A_u, const float* A_l, int64_t a_dstride, int64_t D, int64_t S,
-                                  int64_t N, const float* relax, const float* add_l, int64_t add_ld,
-                                  const float* W_t, int64_t P, const float* bias, const float* b_u_in,
-                                  const float* b_l_in, const float* relax_next, const float* add_next,
-                                  int64_t add_next_ld, const float* bias_next, const float* cvec_next,
-                                  int64_t cvec_next_ld, float* workspace, float* A_next_u, float* A_next_l,
-                                  float* A_pre_u, float* A_pre_l, float* b_u_out, float* b_l_out, float* c_u_out,
-                                  float* c_l_out, hipStream_t stream) {
+static int relu_linear_relu_fwd(int b_parts, const float* A_u, const float* A_l, int64_t a_dstride, int64_t D,
+                                int64_t S, int64_t N, const float* relax, const float* add_l, int64_t add_ld,
+                                const float* W_t, int64_t P, const float* bias, const float* b_u_in,
+                                const float* b_l_in, const float* relax_next, const float* add_next,
+                                int64_t add_next_ld, const float* bias_next, const float* cvec_next,
+                                int64_t cvec_next_ld, float* workspace, float* A_next_u, float* A_next_l,
+                                float* A_pre_u, float* A_pre_l, float* b_u_out, float* b_l_out, float* c_u_out,
+                                float* c_l_out, hipStream_t stream) {
   BF_REQUIRE(D >= 0 && S > 0 && N > 0 && P > 0, "bf_crown_relu_linear_relu_fwd: bad sizes");
   const int64_t M = D * S;
   if (M == 0) return BF_OK;
@@ -1867,7 +1868,9 @@ int bf_crown_relu_linear_relu_fwd(const float* A_u, const float* A_l, int64_t a_
                                   int64_t cvec_next_ld, float* workspace, float* A_next_u, float* A_next_l,
                                   float* A_pre_u, float* A_pre_l, float* b_u_out, float* b_l_out, float* c_u_out,
                                   float* c_l_out, hipStream_t stream) {
-  return relu_linear_relu_fwd(0, A_u, A_l, a_dstride, D, S, N, relax, add_l, add_ld, W_t, P, bias, b_u_in, b_l_in, relax_next, add_next, add_next_ld, bias_next, cvec_next, cvec_next_ld, workspace, A_next_u, A_next_l, A_pre_u, A_pre_l, b_u_out, b_l_out, c_u_out, c_l_out, stream);
+  return relu_linear_relu_fwd(0, A_u, A_l, a_dstride, D, S, N, relax, add_l, add_ld, W_t, P, bias, b_u_in, b_l_in,
+                              relax_next, add_next, add_next_ld, bias_next, cvec_next, cvec_next_ld, workspace,
+                              A_next_u, A_next_l, A_pre_u, A_pre_l, b_u_out, b_l_out, c_u_out, c_l_out, stream);
 }
 
 // The two-region step of an already relaxed coefficient against a packed weight.
@@ -1928,10 +1931,10 @@ int64_t bf_crown_relu_linear_relu_fwd_workspace(int64_t D, int64_t S, int64_t P)
 }
 
 static int linear_concretize(int b_parts, const float* A_u, const float* A_l, int64_t a_dstride, int64_t D, int64_t S,
-                               int64_t N, const float* W_t, int64_t I, const float* rad, float eps, int norm_p,
-                               const float* cen_u, const float* cen_l, const float* b_u, const float* b_l,
-                               const float* h_scale, float* h_out, float* workspace, float* lb, float* ub,
-                               hipStream_t stream) {
+                             int64_t N, const float* W_t, int64_t I, const float* rad, float eps, int norm_p,
+                             const float* cen_u, const float* cen_l, const float* b_u, const float* b_l,
+                             const float* h_scale, float* h_out, float* workspace, float* lb, float* ub,
+                             hipStream_t stream) {
   BF_REQUIRE(D >= 0 && S > 0 && N > 0 && I > 0, "bf_crown_linear_concretize: bad sizes");
   BF_REQUIRE(norm_p >= 0 && norm_p <= 2 && (norm_p == 0 || rad == nullptr),
              "bf_crown_linear_concretize: norm_p %d (0 Linf/box, 1 L1, 2 L2; the box radius goes with 0 only)",
@@ -1986,8 +1989,8 @@ int bf_crown_linear_concretize(const float* A_u, const float* A_l, int64_t a_dst
                                const float* cen_u, const float* cen_l, const float* b_u, const float* b_l,
                                const float* h_scale, float* h_out, float* workspace, float* lb, float* ub,
                                hipStream_t stream) {
-  return linear_concretize(0, A_u, A_l, a_dstride, D, S, N, W_t, I, rad, eps, norm_p, cen_u, cen_l, b_u, b_l, h_scale, h_out,
-                           workspace, lb, ub, stream);
+  return linear_concretize(0, A_u, A_l, a_dstride, D, S, N, W_t, I, rad, eps, norm_p, cen_u, cen_l, b_u, b_l, h_scale,
+                           h_out, workspace, lb, ub, stream);
 }
 
 int bf_crown_linear_concretize_parts(const float* A_u, const float* A_l, int64_t a_dstride, int64_t D, int64_t S,
@@ -1995,8 +1998,8 @@ int bf_crown_linear_concretize_parts(const float* A_u, const float* A_l, int64_t
                                const float* cen_u, const float* cen_l, const float* b_u, const float* b_l,
                                const float* h_scale, float* h_out, float* workspace, float* lb, float* ub,
                                hipStream_t stream) {
-  return linear_concretize(1, A_u, A_l, a_dstride, D, S, N, parts, I, rad, eps, norm_p, cen_u, cen_l, b_u, b_l, h_scale, h_out,
-                           workspace, lb, ub, stream);
+  return linear_concretize(1, A_u, A_l, a_dstride, D, S, N, parts, I, rad, eps, norm_p, cen_u, cen_l, b_u, b_l,
+                           h_scale, h_out, workspace, lb, ub, stream);
 }
 
 int64_t bf_crown_linear_concretize_workspace(int64_t D, int64_t S, int64_t I) {
@@ -2021,7 +2024,8 @@ static int relax_pass(const float* A_u, const float* A_l, int64_t a_dstride, int
   const bool vec = (K % 4 == 0) && (a_dstride % 4 == 0) && al16(A_u) && al16(A_l) && al16(A_u_out) &&
                    al16(A_l_out) && al16(kbias) &&
                    al16(cvec) && al16(add_l) && (add_l == nullptr || add_ld % 4 == 0) && al16(src.lo) &&
-                   al16(src.hi) && al16(src.alpha) && (src.alpha_ld % 4 == 0) && (!two || (al16(two->A[0]) && al16(two->A[1])));
+                   al16(src.hi) && al16(src.alpha) && (src.alpha_ld % 4 == 0) &&
+                   (!two || (al16(two->A[0]) && al16(two->A[1])));
   const bool one = two == nullptr;   // (the kernels that keep a domain's operands take no second coefficient)
   if (one && vec && K <= 512 && (a_dstride == 0 ? S >= 16 : (S >= 8 && M >= 8192))) {
     // a shared coefficient: 16 rows of one domain per workgroup (4 per wave), the

@@ -93,3 +93,39 @@ def test_sum_of_two_coefficients_matches_the_summed_one(D, S, K, sides, one):
         # |beta| <= |A'| |lower|-like terms: both sides sum the same addends, in another order at most
         size = b[q].abs() + b2[q].abs() + (added[q].abs() * (kbias.abs() + 3 * (1 + lo.abs().repeat_interleave(S, 0)))).sum(1)
         assert bool(((bo[q] - bw[q]).abs() <= 2 * (K + 8) * 2.0 ** -24 * size).all())
+
+
+@pytest.mark.parametrize("D,S,K,sides", [(3, 5, 20, "ul"), (2, 7, 255, "l"), (4, 9, 256, "u"), (2, 3, 1028, "ul")])
+@pytest.mark.parametrize("pair", [True, False])
+def test_a_second_bias_is_summed_apart(D, S, K, sides, pair):
+    """The sums of another bias beside the pass's own, with and without a second coefficient: the other
+    outputs keep the bits of the pass without it, its sums those of float64 to their rounding."""
+    dev = device()
+    M = D * S
+    announce(f"relaxation with a second bias D={D} S={S} K={K} sides={sides} pair={pair}")
+    g = torch.Generator().manual_seed(D + 3 * S + 7 * K + pair)
+    r = lambda *shape: torch.randn(*shape, generator=g).to(dev)   # noqa: E731
+    A, b = {q: r(M, K) for q in sides}, {q: r(M) for q in sides}
+    A2, b2 = ({q: r(M, K) for q in sides}, {q: r(M) for q in sides}) if pair else ({}, {})
+    lo, kbias, kbias2 = r(D, K), r(K), r(K)
+    hi = lo + torch.rand(D, K, generator=g).to(dev) * 2
+    out, want = ({q: torch.empty(M, K, device=dev) for q in sides} for _ in range(2))
+    bo, bw, k2 = ({q: torch.empty(M, device=dev) for q in sides} for _ in range(3))
+    p = lambda m, q: _lib.ptr(m.get(q))   # noqa: E731
+    box = (_lib.ptr(lo), _lib.ptr(hi), None, 0, None, 0, _lib.ptr(kbias))
+    _lib.call("bf_crown_relu_relax_biases_lu", p(A, "u"), p(A, "l"), p(A2, "u"), p(A2, "l"), D, S, K, *box,
+              _lib.ptr(kbias2), p(b, "u"), p(b, "l"), p(b2, "u"), p(b2, "l"), p(out, "u"), p(out, "l"), p(bo, "u"),
+              p(bo, "l"), p(k2, "u"), p(k2, "l"), _lib.stream_handle())
+    rows = (p(want, "u"), p(want, "l"), p(bw, "u"), p(bw, "l"))
+    if pair:
+        _lib.call("bf_crown_relu_relax_sum_lu", p(A, "u"), p(A, "l"), p(A2, "u"), p(A2, "l"), D, S, K, *box, p(b, "u"),
+                  p(b, "l"), p(b2, "u"), p(b2, "l"), *rows, _lib.stream_handle())
+    else:
+        _lib.call("bf_crown_relu_relax_lu", p(A, "u"), p(A, "l"), S * K, D, S, K, *box, None, p(b, "u"), p(b, "l"),
+                  *rows, None, None, _lib.stream_handle())
+    torch.cuda.synchronize()
+    for q in sides:
+        assert torch.equal(out[q], want[q]) and torch.equal(bo[q], bw[q])
+        ref = out[q].double() @ kbias2.double()
+        size = out[q].double().abs() @ kbias2.double().abs()
+        assert bool(((k2[q].double() - ref).abs() <= (K + 8) * 2.0 ** -24 * size).all())

@@ -14,8 +14,8 @@ pytestmark = [
 
 def _layers(*dims):
     g = torch.Generator().manual_seed(len(dims))
-    return [crown.AffineLayer(kind="linear", op_index=i, in_name=f"a{i}", out_name=f"h{i}", in_shape=(a,), out_shape=(b,), bias=None,
-                              weight=torch.randn(b, a, generator=g)) for i, (a, b) in enumerate(zip(dims, dims[1:]))]
+    return [crown.AffineLayer(kind="linear", op_index=i, in_name=f"a{i}", out_name=f"h{i}", in_shape=(a,),
+                              out_shape=(b,), bias=None, weight=torch.randn(b, a, generator=g)) for i, (a, b) in enumerate(zip(dims, dims[1:]))]
 
 
 # rows, rows per domain, widths.  36864 rows: every contraction on packed parts, the relaxation in the
