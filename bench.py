@@ -39,8 +39,8 @@ import sys
 import time
 
 PEAK_FP32_MFMA_TFLOPS = 157.3   # MI355X dense fp32 matrix peak
-# an fp32 contraction as six products of bf16 parts (the *_parts launches): a sixth of the dense bf16 peak
-PEAK_PARTS_MFMA_TFLOPS = round(2500.0 / 6.0, 1)
+# an fp32 contraction as eight products of bf16 parts (the *_parts launches): an eighth of the dense bf16 peak
+PEAK_PARTS_MFMA_TFLOPS = round(2500.0 / 8.0, 1)
 PEAK_HBM_GBPS = 8000.0          # MI355X HBM3E
 
 # HBM bytes per launch of a dominant kernel, measured with rocprofv3 --pmc

@@ -165,10 +165,15 @@ int gemm_parts_choice(int64_t M, int64_t N, int64_t K, int64_t S, int nz, int ep
 // norms, both bounds, fp32 / three-part:
 //   288 x 784 (130 64 x 64 tiles): K = 128 15.9 / 15.1, 256 19.7 / 20.2, 512 24.9 / 27.6
 //   36864 x 5 (576 128 x 128 tiles): K = 50 24.6 / 22.8, 256 33.5 / 41.6
-// relaxation, fp32 / three-part (in brackets the 128 x 128 tiles, 512 of which are resident at once):
-//   9216 x 256 (144):   K = 64 19.8 / 19.0, 256 32.6 / 27.5
-//   36864 x 256 (576):  K = 64 30.0 / 37.0, 128 40.9 / 44.0, 256 62.2 / 59.8
+// relaxation, fp32 / three-part (in brackets the 128 x 128 tiles, 512 of which are resident at once; after
+// the comma with a split term and the unrelaxed product stored, as a gradient's pass has them):
+//   9216 x 256 (144):   K = 64 19.8 / 19.0, 256 32.6 / 27.7, 37.7 / 32.6
+//   64800 x 64 (507):   K = 64 23.7 / 19.7, 28.3 / 25.6
+//   36864 x 256 (576):  K = 64 30.0 / 37.0, 128 40.9 / 44.0, 256 62.4 / 59.3, 67.1 / 69.4
+//   18432 x 500 (576):  K = 500 105.9 / 91.8, 110.0 / 102.3
+//   64800 x 256 (1014): K = 256 91.6 / 74.3, 115.8 / 85.4
 //   36864 x 256, both bounds (1152): K = 64 51.7 / 58.0, 128 71.3 / 68.9, 256 111.5 / 95.1
+//   18432 and 36864 x 50 (144, 288): K = 50 18.0 / 17.0, 19.6 / 20.0 and 27.8 / 18.7, 30.3 / 22.3
 bool gemm_parts_pays(int64_t M, int64_t N, int64_t K, int64_t S, int nz, int epi) {
   const int tile = gemm_parts_choice(M, N, K, S, nz, epi);
   if (!tile) return false;
@@ -184,10 +189,9 @@ bool gemm_parts_pays(int64_t M, int64_t N, int64_t K, int64_t S, int nz, int epi
     if (tile == 'S') return K <= 128 || K % 4 || (t64 >= 256 && N > 32);
     return N > 64 || K % 4;   // (columns past N cost a 128 x 128 tile what those inside do)
   }
-  // a second round of 128 x 128 workgroups, mostly empty, outweighs what a short K gains
-  const bool fills = t128 <= 512 || t128 > 768;
   if (K % 4) return t128 >= 256 || K >= 100;
-  return (K >= 100 && fills) || (K >= 256 && N > 64);
+  // a second round of 128 x 128 workgroups, mostly empty, outweighs what a short K gains
+  return t128 <= 512 ? K >= 64 : t128 <= 768 ? K > 256 : K >= 100;
 }
 
 int gemm_dispatch(const GemmArgs& a, int pro, int epi, int nz, hipStream_t stream) {

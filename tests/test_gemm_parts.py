@@ -48,8 +48,9 @@ def test_shapes_taken():
     # norms: the 64-column tile, the 128-column one over a few columns
     (True, 288, 784, 128, 2, 1), (False, 288, 784, 256, 2, 1), (True, 100000, 5, 50, 2, 1), (False, 100000, 5, 256, 2, 1),
     # relaxation: a second round of workgroups that fills, one that does not
-    (False, 9216, 256, 64, 1, 2), (True, 9216, 256, 128, 1, 2), (False, 36864, 256, 128, 1, 2), (True, 36864, 256, 256, 1, 2),
-    (True, 36864, 256, 128, 2, 2), (True, 50000, 50, 50, 2, 2), (False, 8192, 256, 50, 1, 2),
+    (False, 9216, 256, 60, 1, 2), (True, 9216, 256, 64, 1, 2), (False, 36864, 256, 256, 1, 2),
+    (True, 18432, 500, 500, 1, 2), (False, 36864, 256, 64, 2, 2), (True, 36864, 256, 128, 2, 2),
+    (True, 50000, 50, 50, 2, 2), (False, 8192, 256, 50, 1, 2),
     (False, 255, 256, 64, 1, 0), (False, 36864, 256, 256, 3, 0)])
 def test_shapes_that_gain(gains, M, N, K, nz, form):
     if not _lib.LIB_PATH.exists():

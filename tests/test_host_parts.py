@@ -18,11 +18,11 @@ def _layers(*dims):
                               out_shape=(b,), bias=None, weight=torch.randn(b, a, generator=g)) for i, (a, b) in enumerate(zip(dims, dims[1:]))]
 
 
-# rows, rows per domain, widths.  36864 rows: every contraction on packed parts, the relaxation in the
+# rows, rows per domain, widths.  64800 rows: every contraction on packed parts, the relaxation in the
 # epilogue.  2304 of 500 values: the backward's stores are packed, the reverse pass's are split over K.
 # 73728 of 128: the relaxation epilogue stays on the fp32 tiles, the reverse pass's store does not.
 @pytest.mark.parametrize("M,S,dims,below,reverse", [
-    (36864, 9, (784, 256, 256, 256, 10), {0, 1}, {0, 1, 2}), (2304, 9, (784, 500, 500, 500, 10), {1}, set()),
+    (64800, 9, (784, 256, 256, 256, 10), {0, 1}, {0, 1, 2}), (2304, 9, (784, 500, 500, 500, 10), {1}, set()),
     (73728, 9, (784, 128, 128, 128, 10), {0}, {0, 1, 2})])
 @pytest.mark.parametrize("gradient", [False, True])
 def test_a_query_packs_what_it_reads(monkeypatch, M, S, dims, below, reverse, gradient):
