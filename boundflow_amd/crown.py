@@ -257,8 +257,8 @@ def relaxes_in_epilogue(layers: List[AffineLayer], k: int, M: int, S: int) -> bo
     return layers[k - 1].kind == "linear" and S >= EPILOGUE_MIN_ROWS and M >= EPILOGUE_MIN_M
 
 
-# forms of a contraction on packed parts (bf_gemm_parts_config)
-STORE, CONCRETIZE, RELAX = 0, 1, 2
+# forms of a contraction on packed parts (bf_gemm_parts_pays)
+STORE, CONCRETIZE, RELAX, RANK1 = 0, 1, 2, 3
 
 
 def takes_parts(form: int, M: int, N: int, K: int, S: int, nz: int) -> bool:
@@ -272,7 +272,7 @@ def takes_parts(form: int, M: int, N: int, K: int, S: int, nz: int) -> bool:
 def reverse_takes_parts(M: int, N: int, K: int, S: int) -> bool:
     """Whether the reverse pass's contraction of M rows of K values into N (bf_gemm_rank1) runs on packed
     weight parts: one that the fp32 kernels split over K keeps the split."""
-    return takes_parts(STORE, M, N, K, S, 1) and not _lib.load().bf_gemm_rank1_workspace(M, N, K)
+    return takes_parts(RANK1, M, N, K, S, 1) and not _lib.load().bf_gemm_rank1_workspace(M, N, K)
 
 
 @functools.lru_cache(maxsize=4096)

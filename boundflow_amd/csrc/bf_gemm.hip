@@ -159,12 +159,16 @@ int gemm_parts_choice(int64_t M, int64_t N, int64_t K, int64_t S, int nz, int ep
 //   4608 x 784 (936):   K = 256 28.3 / 20.4 / 22.1, 1024 83.4 / 60.3 / 60.3
 //   9216 x 784 (1872):  K = 256 42.5 / 38.0 / 31.5
 //   36864 x 256 (2304): K = 16 13.3 / 12.1 / 15.0, 64 21.6 / 18.4 / 22.1, 256 53.6 / 41.7 / 45.0
+// (with a rank-1 term both kinds read more and the difference shrinks: 2457 rows between launches of other
+// kernels, K = N = 64 level, 103 0.4 us, 128 0.4 us and 160 0.7 us to the fp32 tiles, 100 2.5 us to 64 x 64)
 // stores where K is no multiple of 32 (the fp32 tiles then check their loads) or of four (float by float):
 //   576 x 256:   K = 50 8.4 / 8.3 / 10.3, 100 10.1 / 7.9 / 11.1, 250 16.2 / 16.2 / 21.6, 500 23.0 / 20.1 / 29.4
 //   36864 x 256: K = 50 32.2 / 22.4 / 23.6, 250 93.0 / 47.6 / 50.7, 500 94.5 / 76.6 / 78.3
-// norms, both bounds, fp32 / three-part:
-//   288 x 784 (130 64 x 64 tiles): K = 128 15.9 / 15.1, 256 19.7 / 20.2, 512 24.9 / 27.6
-//   36864 x 5 (576 128 x 128 tiles): K = 50 24.6 / 22.8, 256 33.5 / 41.6
+// norms, fp32 less three-part between launches of other kernels:
+//   576 x 784 (117 64 x 64 tiles): K = 50 0.8, 64 0.8, 100 3.7, 128 0.6, 250 1.4, 256 -1.5, 500 6.4; with the gradient
+//   seeds stored -0.9, -1.0, 2.2, -0.9, 0.4, -2.2 and 4.9
+//   4608 x 784: K = 64 4.5, 256 7.4;  36864 x 784: K = 64 28.8, with the seeds 20.3, 256 60.9 and 55.9
+//   36864 x 5, both bounds (576 128 x 128 tiles): K = 50 -4.7, 128 -8.4
 // relaxation, fp32 / three-part (in brackets the 128 x 128 tiles, 512 of which are resident at once; after
 // the comma with a split term and the unrelaxed product stored, as a gradient's pass has them):
 //   9216 x 256 (144):   K = 64 19.8 / 19.0, 256 32.6 / 27.7, 37.7 / 32.6
@@ -174,7 +178,7 @@ int gemm_parts_choice(int64_t M, int64_t N, int64_t K, int64_t S, int nz, int ep
 //   64800 x 256 (1014): K = 256 91.6 / 74.3, 115.8 / 85.4
 //   36864 x 256, both bounds (1152): K = 64 51.7 / 58.0, 128 71.3 / 68.9, 256 111.5 / 95.1
 //   18432 and 36864 x 50 (144, 288): K = 50 18.0 / 17.0, 19.6 / 20.0 and 27.8 / 18.7, 30.3 / 22.3
-bool gemm_parts_pays(int64_t M, int64_t N, int64_t K, int64_t S, int nz, int epi) {
+bool gemm_parts_pays(int64_t M, int64_t N, int64_t K, int64_t S, int nz, int epi, bool rank1) {
   const int tile = gemm_parts_choice(M, N, K, S, nz, epi);
   if (!tile) return false;
   const int64_t t64 = ceil_div(M, (int64_t)64) * ceil_div(N, (int64_t)64) * nz;
@@ -182,15 +186,15 @@ bool gemm_parts_pays(int64_t M, int64_t N, int64_t K, int64_t S, int nz, int epi
   if (epi == EPI_STORE) {
     if (tile == 'P') return K > 64 || K % 4 || t64 < 2048 || t64 >= 3072;
     // fewer tiles than CUs: a tile's own K loop is the time, and fp32's is the shorter one past K = 128
-    if (t64 < 256) return K <= 128 || (K % 32 && K % 4 == 0);
+    if (t64 < 256) return (K <= 128 && !rank1) || (K % 32 && K % 4 == 0);
     return t64 >= 512 || K <= 256 || K % 32;
   }
   if (epi == EPI_ABSSUM) {
-    if (tile == 'S') return K <= 128 || K % 4 || (t64 >= 256 && N > 32);
-    return N > 64 || K % 4;   // (columns past N cost a 128 x 128 tile what those inside do)
+    if (tile == 'S') return K <= 64 || K % 32 || (t64 >= 256 && N > 32);
+    return N > 64;   // (columns past N cost a 128 x 128 tile what those inside do)
   }
-  if (K % 4) return t128 >= 256 || K >= 100;
   // a second round of 128 x 128 workgroups, mostly empty, outweighs what a short K gains
+  if (K % 4) return K >= 100 || (t128 >= 256 && (t128 <= 512 || t128 > 768));
   return t128 <= 512 ? K >= 64 : t128 <= 768 ? K > 256 : K >= 100;
 }
 

@@ -32,6 +32,35 @@ struct EpilogueRows {
   }
 };
 
+// The values of rows g .. g + EPI_GROUP - 1's vectors (ld floats a domain; one for all with ld 0, read with
+// the first group) at a lane's columns col0 + 32 j.  Groups alternate between the two halves of v, so that
+// one is read while the group before it is stored: the compiler moves no load over those stores.
+// (bf_gemm_rank1_parts on 36864 x 256 x 256, between launches of other kernels: 13 us less than with the
+// values read where they are used; 2457 x 64 x 64 1.3 us.)
+template <class T>
+__device__ __forceinline__ void row_vectors(const GemmArgs& p, const EpilogueRows<T>& rows, const float* vec, int64_t ld,
+                                            int64_t col0, int g, bool fits32, float (&v)[2][EPI_GROUP][T::FN]) {
+  float (&to)[EPI_GROUP][T::FN] = v[g / EPI_GROUP & 1];
+#pragma unroll
+  for (int e = 0; e < EPI_GROUP; ++e) {
+    const int64_t row = rows.row(g + e) < p.M ? rows.row(g + e) : p.M - 1;
+    const float* at = ld ? vec + div_rows(row, p.S, fits32) * ld : vec;
+#pragma unroll
+    for (int j = 0; j < T::FN; ++j) {
+      const int64_t col = col0 + 32 * j;
+      to[e][j] = g > 0 && !ld ? v[0][0][j] : at[col < p.N ? col : p.N - 1];
+    }
+  }
+}
+
+// A value of each of a lane's 16 rows.
+template <class T>
+__device__ __forceinline__ void row_scalars(const GemmArgs& p, const EpilogueRows<T>& rows, const float* of,
+                                            float (&s)[16]) {
+#pragma unroll
+  for (int r = 0; r < 16; ++r) s[r] = of[rows.row(r) < p.M ? rows.row(r) : p.M - 1];
+}
+
 // The store, norm or relaxation epilogue of one workgroup tile: gemm_kernel's arithmetic in its
 // order, taken column block by column block so that a lane's store is one instruction.  A whole
 // row block takes neither bounds nor 64-bit addresses per element: the relaxation epilogue's launch
@@ -54,30 +83,28 @@ __device__ __forceinline__ void parts_epilogue(const GemmArgs& p, floatx16 (&acc
     const bool r1 = p.r1_row != nullptr;
     const bool fits32 = M < (1LL << 31);
     auto store = [&](auto rank1) {
+      constexpr bool R1 = decltype(rank1)::value;
 #pragma unroll
       for (int i = 0; i < FM; ++i) {
         const EpilogueRows<T> rows(C, ldc, m0, n0, wm, wn, i, lane);
+        const int64_t col0 = n0 + wn * T::WTN + lrow;
+        float rf[16], v[2][EPI_GROUP][FN];   // each row's rank-1 factor and vector
+        if constexpr (R1) {
+          row_scalars(p, rows, p.r1_row, rf);
+          row_vectors(p, rows, p.r1_col, p.r1_ld, col0, 0, fits32, v);
+        }
 #pragma unroll
         for (int g = 0; g < 16; g += EPI_GROUP) {
-          float rf[EPI_GROUP];
-          const float* vrow[EPI_GROUP];
-          if constexpr (decltype(rank1)::value) {
-            // each row's rank-1 factor and vector (no division when the vector is shared)
-#pragma unroll
-            for (int e = 0; e < EPI_GROUP; ++e) {
-              const int64_t row = rows.row(g + e) < M ? rows.row(g + e) : M - 1;
-              rf[e] = p.r1_row[row];
-              vrow[e] = p.r1_ld ? p.r1_col + div_rows(row, p.S, fits32) * p.r1_ld : p.r1_col;
-            }
-          }
+          if constexpr (R1)
+            if (g + EPI_GROUP < 16) row_vectors(p, rows, p.r1_col, p.r1_ld, col0, g + EPI_GROUP, fits32, v);
 #pragma unroll
           for (int j = 0; j < FN; ++j) {
-            const int64_t col = n0 + wn * T::WTN + j * 32 + lrow;
-            if (col >= N) continue;
+            if (col0 + 32 * j >= N) continue;
 #pragma unroll
             for (int e = 0; e < EPI_GROUP; ++e)
               if (rows.whole(M) || rows.row(g + e) < M) {
-                if constexpr (decltype(rank1)::value) rows.put(g + e, j, acc[i][j][g + e] + rf[e] * vrow[e][col]);
+                if constexpr (R1)
+                  rows.put(g + e, j, acc[i][j][g + e] + rf[g + e] * v[g / EPI_GROUP & 1][e][j]);
                 else rows.put(g + e, j, acc[i][j][g + e]);
               }
           }
@@ -100,21 +127,19 @@ __device__ __forceinline__ void parts_epilogue(const GemmArgs& p, floatx16 (&acc
 #pragma unroll
       for (int i = 0; i < FM; ++i) {
         const EpilogueRows<T> rows(p.h_out, N, m0, n0, wm, wn, i, lane);
+        const int64_t col0 = n0 + wn * T::WTN + lrow;
+        float hs[16], w[2][EPI_GROUP][FN];   // each row's seed scale and column weights
+        if constexpr (H && NK == 0) row_scalars(p, rows, p.h_scale, hs);
+        if constexpr (W) row_vectors(p, rows, p.wvec, p.w_ld, col0, 0, fits32, w);
 #pragma unroll
         for (int g = 0; g < 16; g += EPI_GROUP) {
-          float hs[EPI_GROUP];
-          const float* wrow[EPI_GROUP];
+          if constexpr (W)
+            if (g + EPI_GROUP < 16) row_vectors(p, rows, p.wvec, p.w_ld, col0, g + EPI_GROUP, fits32, w);
 #pragma unroll
-          for (int e = 0; e < EPI_GROUP; ++e) {
-            const int64_t row = rows.row(g + e) < M ? rows.row(g + e) : M - 1;
-            if constexpr (H && NK == 0) hs[e] = p.h_scale[row];
-            if constexpr (W) wrow[e] = p.wvec + div_rows(row, p.S, fits32) * p.w_ld;
-            rs[i][g + e] = 0.f;
-          }
+          for (int e = 0; e < EPI_GROUP; ++e) rs[i][g + e] = 0.f;
 #pragma unroll
           for (int j = 0; j < FN; ++j) {
-            const int64_t col = n0 + wn * T::WTN + j * 32 + lrow;
-            if (col >= N) continue;   // columns past N hold products no one keeps
+            if (col0 + 32 * j >= N) continue;   // columns past N hold products no one keeps
 #pragma unroll
             for (int e = 0; e < EPI_GROUP; ++e) {
               const int r = g + e;
@@ -122,7 +147,7 @@ __device__ __forceinline__ void parts_epilogue(const GemmArgs& p, floatx16 (&acc
               float v = NK == 2 ? a * a : fabsf(a);
               float wgt = 1.f;
               if constexpr (W) {
-                wgt = wrow[e][col];
+                wgt = w[g / EPI_GROUP & 1][e][j];
                 v = v * wgt;
               }
               rs[i][r] = join(rs[i][r], v);
@@ -132,7 +157,7 @@ __device__ __forceinline__ void parts_epilogue(const GemmArgs& p, floatx16 (&acc
                   rows.put(r, j, a);   // the L1/L2 seeds need the whole row's norm: made from C afterwards
                 } else {
                   const float sg = (a > 0.f) ? 1.f : ((a < 0.f) ? -1.f : 0.f);
-                  rows.put(r, j, W ? hs[e] * sg * wgt : hs[e] * sg);
+                  rows.put(r, j, W ? hs[r] * sg * wgt : hs[r] * sg);
                 }
               }
             }

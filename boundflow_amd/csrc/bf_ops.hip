@@ -36,7 +36,7 @@ int concretize_finalize(const float* pu, const float* pl, int nparts, int64_t M,
 int gemm_partial_count(int64_t N);
 int gemm_norm_partial_count(int64_t M, int64_t N, int pro);
 int gemm_parts_choice(int64_t M, int64_t N, int64_t K, int64_t S, int nz, int epi);
-bool gemm_parts_pays(int64_t M, int64_t N, int64_t K, int64_t S, int nz, int epi);
+bool gemm_parts_pays(int64_t M, int64_t N, int64_t K, int64_t S, int nz, int epi, bool rank1);
 int64_t parts_floats(int64_t N, int64_t K);
 int pack_parts(int count, const float* const* B, const int64_t* ldb, const int* trans_b, const int64_t* N,
                const int64_t* K, float* const* out, hipStream_t stream);
@@ -1500,7 +1500,8 @@ int bf_gemm_parts_config(int64_t M, int64_t N, int64_t K, int64_t S, int nz, int
 }
 
 int bf_gemm_parts_pays(int64_t M, int64_t N, int64_t K, int64_t S, int nz, int form) {
-  return nz >= 1 && nz <= 2 && form >= 0 && form <= 2 && gemm_parts_pays(M, N, K, S, nz, form) ? 1 : 0;
+  if (nz < 1 || nz > 2 || form < 0 || form > 3) return 0;
+  return gemm_parts_pays(M, N, K, S, nz, form == 3 ? 0 : form, form == 3) ? 1 : 0;
 }
 
 int64_t bf_gemm_parts_floats(int64_t N, int64_t K) { return N <= 0 || K <= 0 ? 0 : parts_floats(N, K); }

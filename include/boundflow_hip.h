@@ -60,7 +60,8 @@ int bf_gemm_tile_config(int64_t M, int64_t N, int nz, int ksplit, int relax_prol
  * over K with nz bounds, 'P' (128 x 128) or 'S' (64 x 64), else 0 (K below 16, a short
  * grid, or rows past 32-bit offsets): the caller then takes the namesake.
  * bf_gemm_parts_pays: whether that is also faster than the namesake.  form: 0 the stores (bf_gemm_rank1_parts,
- * bf_crown_linear_parts), 1 bf_crown_linear_concretize_parts, 2 bf_crown_linear_relu_fwd_parts.
+ * bf_crown_linear_parts), 1 bf_crown_linear_concretize_parts, 2 bf_crown_linear_relu_fwd_parts; for pays also 3,
+ * bf_gemm_rank1_parts with a rank-1 term.
  * Coefficient rows must be dense.
  * bf_gemm_pack_parts: count weights in one launch, B[j] as [N, K] (trans_b) or [K, N]
  * row-major with row stride ldb -> parts[j], bf_gemm_parts_floats(N, K) floats, 16-byte
