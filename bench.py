@@ -48,9 +48,9 @@ PEAK_HBM_GBPS = 8000.0          # MI355X HBM3E
 # reads for a 1 GiB device copy: x2.0 and x1.0), averaged over the launch mix
 # of that query.  Keyed by (config, kernel family); other pairs report null.
 MEASURED_TRAFFIC = {
-    ("C2", "crown_linear_relu_fwd_parts"): (1.4112e9, "profiles/hbm_traffic_dominant_kernels.md"),
-    ("C5", "crown_linear_relu_fwd_parts"): (1.3330e8, "profiles/hbm_traffic_dominant_kernels.md"),
-    ("C5", "grad_gemm_parts"): (1.0440e8, "profiles/hbm_traffic_dominant_kernels.md"),
+    ("C2", "crown_linear_relu_fwd_parts"): (1.4538e9, "profiles/hbm_traffic_dominant_kernels.md"),
+    ("C5", "crown_relu_linear_relu_fwd"): (1.3250e8, "profiles/hbm_traffic_dominant_kernels.md"),
+    ("C5", "grad_gemm_parts"): (1.0820e8, "profiles/hbm_traffic_dominant_kernels.md"),
 }
 
 
